@@ -130,12 +130,6 @@ __device__ __forceinline__ bool stopped(const Status* st, unsigned int* s_stop) 
   return *s_stop != 0;
 }
 
-__device__ __forceinline__ uint32_t wave_sum_u32(uint32_t v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
-
 __device__ __forceinline__ uint64_t block_sum_u64(uint64_t v, uint64_t* s_w) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
@@ -191,7 +185,6 @@ __global__ __launch_bounds__(256) void k_seg_count(const int4* __restrict__ rayi
   }
   __syncthreads();
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  uint32_t nseg = 0;
   RayGeom g;
   if (i < ctl->n_rays && ray_geom(rayinfo, scans, i, g)) {
     SegEnum en;
@@ -206,7 +199,6 @@ __global__ __launch_bounds__(256) void k_seg_count(const int4* __restrict__ rayi
         const uint32_t gs = brick_slot(bv, key, true, &st->overflow);
         if (gs != kNone) atomicAdd(&bv.cnt[gs], 1u);
       }
-      ++nseg;
     }
   }
   __syncthreads();
@@ -223,8 +215,6 @@ __global__ __launch_bounds__(256) void k_seg_count(const int4* __restrict__ rayi
     if (gs != kNone) atomicAdd(&bv.cnt[gs], lcnt[e]);
     wsc[tb + e] = ((uint64_t)gs << 32) | lcnt[e];
   }
-  nseg = wave_sum_u32(nseg);
-  if (bw_lane() == 0 && nseg) atomicAdd(&st->segs, nseg);
 }
 
 // Per 256 slots: (work items << 32) | segments.
@@ -238,10 +228,13 @@ __global__ __launch_bounds__(256) void k_brick_sums(BrickView bv, uint64_t* __re
   if (threadIdx.x == 0) bsum[blockIdx.x] = t;
 }
 
-// Exclusive scan of nb packed sums (one workgroup of 1024); totals to st.
+// Exclusive scan of nb packed sums (one workgroup); totals to st: the sum's
+// bits from total_shift up, and its low half where `low` is given (the
+// segments: one atomic per wave of the count on st->segs took 40 of its 103 us
+// for 262,144 rays).
 __global__ __launch_bounds__(256) void k_scan_u64(const uint64_t* __restrict__ bsum,
                                                   uint64_t* __restrict__ boff, uint32_t nb,
-                                                  unsigned int* total, int total_shift) {
+                                                  unsigned int* total, int total_shift, unsigned int* low) {
   __shared__ uint64_t wsum[4];
   uint64_t carry = 0;
   for (uint32_t base = 0; base < nb; base += 256) {
@@ -265,7 +258,10 @@ __global__ __launch_bounds__(256) void k_scan_u64(const uint64_t* __restrict__ b
     carry += tot;
     __syncthreads();
   }
-  if (threadIdx.x == 0) *total = (unsigned int)(carry >> total_shift);
+  if (threadIdx.x == 0) {
+    *total = (unsigned int)(carry >> total_shift);
+    if (low) *low = (unsigned int)carry;
+  }
 }
 
 __global__ __launch_bounds__(256) void k_brick_offsets(BrickView bv, const uint64_t* __restrict__ boff,
@@ -778,7 +774,7 @@ hipError_t launch_brick_offsets(hipStream_t s, BrickView bv, uint64_t* bsum, uin
   hipLaunchKernelGGL(k_brick_sums, dim3(nb), dim3(256), 0, s, bv, bsum, st);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_scan_u64, dim3(1), dim3(256), 0, s, bsum, boff, nb, &st->items, 32);
+  hipLaunchKernelGGL(k_scan_u64, dim3(1), dim3(256), 0, s, bsum, boff, nb, &st->items, 32, &st->segs);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(k_brick_offsets, dim3(nb), dim3(256), 0, s, bv, boff, items, seg_cap, item_cap,
@@ -810,7 +806,8 @@ hipError_t launch_rec_list(hipStream_t s, const unsigned long long* leaf_mask, u
   hipLaunchKernelGGL(k_mask_sums, dim3(nb_cap), dim3(256), 0, s, leaf_mask, bsum, st);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_scan_u64, dim3(1), dim3(256), 0, s, bsum, boff, nb_cap, &st->records, 0);
+  hipLaunchKernelGGL(k_scan_u64, dim3(1), dim3(256), 0, s, bsum, boff, nb_cap, &st->records, 0,
+                     (unsigned int*)nullptr);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(k_mask_list, dim3(nb_cap), dim3(256), 0, s, leaf_mask, boff, list, st);

@@ -31,6 +31,9 @@ constexpr uint32_t kScanMask = 0x7Fu;
 constexpr int kMaxBatchScans = 128;
 constexpr int kBatchCoordLimit = 1 << 21;   // batched keys: 19-bit leaf coords + 7-bit scan
 constexpr int kPrepBlock = 256;
+// sums of a prep workgroup: visits in the low bits (256 * (1 + 3 * 8192) < 2^23), valid rays (<= 256) above
+constexpr int kPrepValidShift = 23;
+constexpr uint32_t kPrepVisitMask = (1u << kPrepValidShift) - 1;
 constexpr int kMaxQuerySteps = 1 << 24;  // per-axis voxel extent bound of a raytrace query
 
 // Status bits written by kernels.

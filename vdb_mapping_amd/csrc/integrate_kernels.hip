@@ -102,6 +102,14 @@ struct Run {
   }
 };
 
+// Workgroup of the kernels that append a record per lane to a list: every
+// append of a workgroup is one atomic on the list's counter, and those of a
+// grid run one after another (about 10 ns each), so large lists take 1,024
+// records per append. Below 65,536 records (64 workgroups of 1,024) the
+// smaller workgroups reach more CUs instead.
+constexpr int kListBlockMax = 1024;
+inline int list_block(uint32_t count) { return count < 65536 ? 256 : kListBlockMax; }
+
 // ---------------------------------------------------------------- kernels --
 
 // Row n of the crossing table: next_0 = 0.5 * fl(1/n), next_j = fl(next_{j-1} + fl(1/n)),
@@ -201,11 +209,11 @@ __global__ __launch_bounds__(kPrepBlock) void k_prep(const float* __restrict__ p
       scans[b].s[2] = sz;
     }
   }
-  // valid-ray count, one atomic per wave
-  const uint64_t vm = __ballot(valid);
-  if (lane_id() == 0 && vm) atomicAdd(&st->rays, (unsigned long long)__popcll(vm));
-  // block-inclusive prefix of the visit counts
-  uint32_t v = cnt;
+  // block-inclusive prefix of the visit counts, the valid rays counted above
+  // them (kPrepValidShift): the scan of the block sums totals both. One atomic
+  // per wave on st->rays took most of the kernel: 54 us of 262,144 rays, 8
+  // us with the count in the block sums.
+  uint32_t v = cnt + (valid ? 1u << kPrepValidShift : 0u);
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
     const uint32_t t = __shfl_up(v, o, 64);
@@ -217,7 +225,7 @@ __global__ __launch_bounds__(kPrepBlock) void k_prep(const float* __restrict__ p
   uint32_t add = 0;
   for (int w = 0; w < wv; ++w) add += wsum[w];
   v += add;
-  if (i < n) pre[i] = v;
+  if (i < n) pre[i] = v & kPrepVisitMask;
   if (threadIdx.x == kPrepBlock - 1) bsum[blockIdx.x] = v;
 }
 
@@ -227,10 +235,12 @@ __global__ __launch_bounds__(256) void k_scan_blocks(const uint32_t* __restrict_
                                                      Status* st) {
   __shared__ unsigned long long wsum[4];
   const uint32_t nb = ctl->nb;
-  unsigned long long carry = 0;
+  unsigned long long carry = 0, rays = 0;
   for (uint32_t base = 0; base < nb; base += 256) {
     const uint32_t i = base + threadIdx.x;
-    const unsigned long long x = i < nb ? bsum[i] : 0ull;
+    const uint32_t b = i < nb ? bsum[i] : 0u;
+    rays += b >> kPrepValidShift;
+    const unsigned long long x = b & kPrepVisitMask;
     unsigned long long v = x;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
@@ -249,7 +259,14 @@ __global__ __launch_bounds__(256) void k_scan_blocks(const uint32_t* __restrict_
     carry += tot;
     __syncthreads();
   }
-  if (threadIdx.x == 0) st->total = carry;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) rays += __shfl_xor(rays, o, 64);
+  if (lane_id() == 0) wsum[threadIdx.x >> 6] = rays;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    st->total = carry;
+    st->rays = wsum[0] + wsum[1] + wsum[2] + wsum[3];
+  }
 }
 
 // Global visit offset of each ray and, for every chunk of `chunk` visits,
@@ -490,27 +507,35 @@ __global__ __launch_bounds__(256) void k_compact(UpdView u, uint32_t cap,
                                                  const Status* st) {
   __shared__ uint32_t s_wave[4], s_base;
   if (st->error != 0 || st->overflow != 0) return;  // same for every thread
-  const uint32_t G = gridDim.x * blockDim.x;
-  const uint32_t rounds = (cap + G - 1) / G;
-  for (uint32_t rd = 0; rd < rounds; ++rd) {
-    const uint32_t slot = rd * G + blockIdx.x * blockDim.x + threadIdx.x;
-    const bool valid = slot < cap && u.keys[slot] != kEmpty;
-    const uint32_t pos = block_append(valid, counter, s_wave, &s_base);
-    if (valid) list[pos] = slot;
+  // eight slots per thread and append: at one slot a table of 4 M slots made
+  // 16 k appends to one counter, which was all of its 190 us
+  constexpr int kSlots = 8;
+  const uint32_t tile = blockDim.x * kSlots;
+  for (uint32_t base = blockIdx.x * tile; base < cap; base += gridDim.x * tile) {
+    bool valid[kSlots];
+    uint32_t pos[kSlots];
+#pragma unroll
+    for (int r = 0; r < kSlots; ++r) {
+      const uint32_t slot = base + r * blockDim.x + threadIdx.x;
+      valid[r] = slot < cap && u.keys[slot] != kEmpty;
+    }
+    block_append_n(valid, pos, counter, s_wave, &s_base);
+#pragma unroll
+    for (int r = 0; r < kSlots; ++r)
+      if (valid[r]) list[pos[r]] = base + r * blockDim.x + threadIdx.x;
   }
 }
 
 // One lane per update leaf: find its map leaf, or create it when the update
 // changes a background voxel (OpenVDB creates a child node only when the
 // modify op changes the tile's value or active state).
-__global__ __launch_bounds__(256) void k_map_insert(UpdView u, const uint32_t* __restrict__ list,
-                                                    uint32_t count, MapView mp,
-                                                    uint32_t* __restrict__ eidx,
-                                                    uint32_t create_hit, uint32_t create_miss,
-                                                    unsigned long long* noop_set,
-                                                    uint32_t noop_mask, Status* st, Status* stc) {
-  __shared__ uint32_t s_wave[4], s_base;
-  uint32_t listed = 0;
+__global__ __launch_bounds__(kListBlockMax) void k_map_insert(UpdView u, const uint32_t* __restrict__ list,
+                                                              uint32_t count, MapView mp,
+                                                              uint32_t* __restrict__ eidx,
+                                                              uint32_t create_hit, uint32_t create_miss,
+                                                              unsigned long long* noop_set,
+                                                              uint32_t noop_mask, Status* st) {
+  __shared__ uint32_t s_wave[kListBlockMax / 64], s_base;
   const uint32_t G = gridDim.x * blockDim.x;
   const uint32_t e0 = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t rounds = (count + G - 1) / G;
@@ -519,8 +544,7 @@ __global__ __launch_bounds__(256) void k_map_insert(UpdView u, const uint32_t* _
     bool created = false;
     uint32_t h = kNone, idx = kNone;
     uint64_t key = 0;
-    if (e < count && (list || u.keys[e] != kEmpty)) {
-      ++listed;
+    if (e < count) {
       const uint32_t slot = list ? list[e] : e;
       key = u.keys[slot];
       // every listed leaf has a visited voxel: with both ops creating, it needs
@@ -576,16 +600,6 @@ __global__ __launch_bounds__(256) void k_map_insert(UpdView u, const uint32_t* _
       eidx[e] = idx;
       if (idx != kNone) mp.dirty[idx] = 1;
     }
-  }
-  // update leaves of this call: one atomic per workgroup
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) listed += __shfl_xor(listed, o, 64);
-  if (lane_id() == 0) s_wave[threadIdx.x >> 6] = listed;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    uint32_t t = 0;
-    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) t += s_wave[w];
-    if (t) atomicAdd(&stc->entries, t);
   }
 }
 
@@ -719,13 +733,16 @@ __global__ __launch_bounds__(256) void k_apply(UpdView u, const uint32_t* __rest
 // record of a map leaf opens its group (the group's record positions cleared,
 // its own entered); a later one enters its position in the group that an
 // earlier scan's record opened (a map leaf has one record per scan).
-__global__ __launch_bounds__(256) void k_group_add(const uint32_t* __restrict__ eidx,
-                                                   const uint32_t* __restrict__ list, uint32_t count, uint32_t t,
-                                                   uint32_t* gslot, uint32_t* rgrp, uint32_t rgrp_stride,
-                                                   uint32_t* glist, uint32_t* grec, unsigned int* ngroups) {
-  __shared__ uint32_t s_wave[4];
+// Its cost is the append counter (see list_block): 66 -> 52 us a scan on the
+// outdoor stream with 1,024 records per append instead of 256.
+__global__ __launch_bounds__(kListBlockMax) void k_group_add(const uint32_t* __restrict__ eidx,
+                                                             const uint32_t* __restrict__ list, uint32_t count,
+                                                             uint32_t t, uint32_t* gslot, uint32_t* rgrp,
+                                                             uint32_t rgrp_stride, uint32_t* glist, uint32_t* grec,
+                                                             unsigned int* ngroups) {
+  __shared__ uint32_t s_wave[kListBlockMax / 64];
   __shared__ uint32_t s_base;
-  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t e = i < count ? eidx[i] : kNone;
   uint32_t code = kNone;
   if (e != kNone) code = atomicCAS(&gslot[e], kNone, (t << kGroupScanShift) | i);
@@ -1040,18 +1057,21 @@ hipError_t launch_fast_cast(hipStream_t s, int grid, const int4* rayinfo, const 
   return hipGetLastError();
 }
 
-hipError_t launch_compact(hipStream_t s, int grid, UpdView u, uint32_t cap, uint32_t* list,
+hipError_t launch_compact(hipStream_t s, UpdView u, uint32_t cap, uint32_t* list,
                           unsigned int* counter, const Status* st) {
+  const int grid = (int)std::min<uint32_t>(4096, (cap + 2047) / 2048);
   hipLaunchKernelGGL(k_compact, dim3(grid), dim3(256), 0, s, u, cap, list, counter, st);
   return hipGetLastError();
 }
 
-hipError_t launch_map_insert(hipStream_t s, int grid, UpdView u, const uint32_t* list,
-                             uint32_t count, MapView mp, uint32_t* eidx, bool create_hit,
-                             bool create_miss, unsigned long long* noop_set, uint32_t noop_mask,
-                             Status* st, Status* stc) {
-  hipLaunchKernelGGL(k_map_insert, dim3(grid), dim3(256), 0, s, u, list, count, mp, eidx,
-                     (uint32_t)create_hit, (uint32_t)create_miss, noop_set, noop_mask, st, stc);
+hipError_t launch_map_insert(hipStream_t s, UpdView u, const uint32_t* list, uint32_t count, MapView mp,
+                             uint32_t* eidx, bool create_hit, bool create_miss,
+                             unsigned long long* noop_set, uint32_t noop_mask, Status* st) {
+  if (!count) return hipSuccess;
+  const int block = list_block(count);
+  const int grid = (int)std::min<uint32_t>((1u << 20) / block, (count + block - 1) / block);
+  hipLaunchKernelGGL(k_map_insert, dim3(grid), dim3(block), 0, s, u, list, count, mp, eidx,
+                     (uint32_t)create_hit, (uint32_t)create_miss, noop_set, noop_mask, st);
   return hipGetLastError();
 }
 
@@ -1067,7 +1087,8 @@ hipError_t launch_group_add(hipStream_t s, const uint32_t* eidx, const uint32_t*
                             uint32_t* gslot, uint32_t* rgrp, uint32_t rgrp_stride, uint32_t* glist, uint32_t* grec,
                             unsigned int* ngroups) {
   if (!count) return hipSuccess;
-  hipLaunchKernelGGL(k_group_add, dim3((count + 255) / 256), dim3(256), 0, s, eidx, list, count, t, gslot, rgrp,
+  const int block = list_block(count);
+  hipLaunchKernelGGL(k_group_add, dim3((count + block - 1) / block), dim3(block), 0, s, eidx, list, count, t, gslot, rgrp,
                      rgrp_stride, glist, grec, ngroups);
   return hipGetLastError();
 }

@@ -24,7 +24,7 @@ hipError_t launch_traverse(hipStream_t s, int grid, int block, const int4* rayin
 hipError_t launch_fast_cast(hipStream_t s, int grid, const int4* rayinfo, const ScanInfo* scans,
                             const BatchCtl* ctl, RtView rt, MapView mp, UpdView u, bool cast,
                             Status* st);
-hipError_t launch_compact(hipStream_t s, int grid, UpdView u, uint32_t cap, uint32_t* list,
+hipError_t launch_compact(hipStream_t s, UpdView u, uint32_t cap, uint32_t* list,
                           unsigned int* counter, const Status* st);
 hipError_t launch_group_build(hipStream_t s, int grid, UpdView u, const uint32_t* list, GroupView gv,
                               bool create_hit, bool create_miss, const Status* st);
@@ -39,10 +39,9 @@ hipError_t launch_fold(hipStream_t s, int grid, UpdView u, GroupView gv, const u
 hipError_t launch_clear_keys(hipStream_t s, int grid, UpdView u, const uint32_t* list,
                              const Status* st);
 hipError_t launch_zero_words(hipStream_t s, unsigned long long* p, uint32_t n);
-hipError_t launch_map_insert(hipStream_t s, int grid, UpdView u, const uint32_t* list,
-                             uint32_t count, MapView mp, uint32_t* eidx, bool create_hit,
-                             bool create_miss, unsigned long long* noop_set, uint32_t noop_mask,
-                             Status* st, Status* stc);
+hipError_t launch_map_insert(hipStream_t s, UpdView u, const uint32_t* list, uint32_t count, MapView mp,
+                             uint32_t* eidx, bool create_hit, bool create_miss,
+                             unsigned long long* noop_set, uint32_t noop_mask, Status* st);
 hipError_t launch_rec_gather(hipStream_t s, int grid, const uint32_t* list, UpdView sparse, const RecDest* dest,
                              const Status* st);
 hipError_t launch_put_dest(hipStream_t s, RecDest* dst, RecDest v);

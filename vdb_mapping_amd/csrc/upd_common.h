@@ -90,4 +90,37 @@ __device__ __forceinline__ uint32_t block_append(bool valid, unsigned int* count
   return pos;
 }
 
+// The same for N elements per thread: pos[r] of the valid ones, one atomic per
+// N * blockDim.x elements. Atomics of a whole grid on one address run one
+// after another (about 10 ns each here), so a list of a million elements
+// wants few of them.
+template <int N>
+__device__ __forceinline__ void block_append_n(const bool (&valid)[N], uint32_t (&pos)[N], unsigned int* counter,
+                                               uint32_t* s_wave, uint32_t* s_base) {
+  const uint64_t below = (1ull << lane_id()) - 1;
+  const int w = threadIdx.x >> 6;
+  uint32_t sum = 0;
+#pragma unroll
+  for (int r = 0; r < N; ++r) {
+    const uint64_t m = __ballot(valid[r]);
+    pos[r] = sum + (uint32_t)__popcll(m & below);
+    sum += (uint32_t)__popcll(m);
+  }
+  if (lane_id() == 0) s_wave[w] = sum;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    uint32_t tot = 0;
+    for (int i = 0; i < (int)(blockDim.x >> 6); ++i) {
+      const uint32_t c = s_wave[i];
+      s_wave[i] = tot;
+      tot += c;
+    }
+    *s_base = tot ? atomicAdd(counter, tot) : 0u;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < N; ++r) pos[r] += *s_base + s_wave[w];
+  __syncthreads();
+}
+
 }  // namespace vdbgpu

@@ -785,8 +785,7 @@ int launch_fold_stage(vdbgpu_map* m, Source& src, bool from_groups) {
   Status* st = &m->d_st[0];
   if (from_groups) {
     CK(launch_group_build(m->stream, fold_grid(m), upd_view(src), src.list, group_view(m), ch, cm, st));
-    CK(launch_compact(m->stream, std::min<int>(4096, (int)((m->gcap + 255) / 256)),
-                      UpdView{m->gkeys, nullptr, m->gcap - 1}, m->gcap, m->glist, &st->groups, st));
+    CK(launch_compact(m->stream, UpdView{m->gkeys, nullptr, m->gcap - 1}, m->gcap, m->glist, &st->groups, st));
   }
   CK(launch_map_check(m->stream, st, &m->d_st[1], m->lcap, m->mcap));
   CK(launch_group_insert(m->stream, fold_grid(m), group_view(m), m->glist, map_view(m), m->gidx,
@@ -909,7 +908,7 @@ int run_pipeline(vdbgpu_map* m, Source& src, const float* xyz, int64_t stride, b
       }
       {
         Timer t(m, kCompact);
-        CK(launch_compact(m->stream, std::min<int>(4096, (int)((src.cap + 255) / 256)), upd_view(src),
+        CK(launch_compact(m->stream, upd_view(src),
                           src.cap, src.list, &m->d_st[0].entries, &m->d_st[0]));
       }
     }
@@ -961,7 +960,7 @@ int run_pipeline(vdbgpu_map* m, Source& src, const float* xyz, int64_t stride, b
     if (batched && (r = ensure_groups(m, src.cap))) return r;
     if (!batched) {
       CK(hipMemsetAsync(&m->d_st[0], 0, sizeof(Status), m->stream));
-      CK(launch_compact(m->stream, std::min<int>(4096, (int)((src.cap + 255) / 256)), upd_view(src),
+      CK(launch_compact(m->stream, upd_view(src),
                         src.cap, src.list, &m->d_st[0].entries, &m->d_st[0]));
       if ((r = read_status(m))) return r;
       src.pending = m->h_st[0].entries;
@@ -1003,7 +1002,7 @@ int run_fast(vdbgpu_map* m, Source& src, const float* xyz, int64_t n, int64_t st
     }
     {
       Timer t(m, kCompact);
-      CK(launch_compact(m->stream, std::min<int>(4096, (int)((src.cap + 255) / 256)), upd_view(src),
+      CK(launch_compact(m->stream, upd_view(src),
                         src.cap, src.list, &m->d_st[0].entries, &m->d_st[0]));
     }
     if ((r = read_status(m))) return r;
@@ -1502,13 +1501,13 @@ int commit_staged(vdbgpu_map* m) {
   bool ch, cm;
   create_flags(m, &ch, &cm);
   const UpdView rec{m->dkeys[X], m->dmasks[X], 0};
-  const int g1 = std::min<int>(4096, (int)((recs + 255) / 256));
   {
     Timer t(m, kCompact);
-    CK(launch_map_insert(m->stream, g1, rec, m->ident, recs, map_view(m), m->reidx[X], ch, cm, m->noop4096,
-                         vdbgpu_map::kNoopCap - 1, &m->d_st[1], &m->d_st[3]));
+    CK(launch_map_insert(m->stream, rec, m->ident, recs, map_view(m), m->reidx[X], ch, cm, m->noop4096,
+                         vdbgpu_map::kNoopCap - 1, &m->d_st[1]));
   }
   m->leaf_count_ub += recs;
+  m->stats.update_leaves += recs;
   ledger_add(m, recs);
   CK(launch_snap_count(m->stream, &m->d_st[1], &m->d_lc[X]));
   CK(hipEventRecord(m->ins_done[X], m->stream));
@@ -1653,12 +1652,11 @@ int do_integrate(vdbgpu_map* m) {
       m->eidx_cap = (uint32_t)next_pow2(s.pending);
       CK(dalloc(m, &m->eidx, m->eidx_cap));
     }
-    const int g1 = std::min<int>(4096, (int)((s.pending + 255) / 256));
     const int g2 = std::min<int>(m->num_cu * 16, (int)((s.pending + 1) / 2));  // 128 lanes per leaf
     {
       Timer t(m, kCompact);
-      CK(launch_map_insert(m->stream, g1, upd_view(s), s.list, s.pending, map_view(m), m->eidx, ch, cm,
-                           m->noop4096, vdbgpu_map::kNoopCap - 1, &m->d_st[1], &m->d_st[3]));
+      CK(launch_map_insert(m->stream, upd_view(s), s.list, s.pending, map_view(m), m->eidx, ch, cm,
+                           m->noop4096, vdbgpu_map::kNoopCap - 1, &m->d_st[1]));
     }
     {
       Timer t(m, kApply);
@@ -1666,6 +1664,7 @@ int do_integrate(vdbgpu_map* m) {
                       &m->d_st[3], true));
     }
     m->leaf_count_ub += s.pending;
+    m->stats.update_leaves += s.pending;
     ledger_add(m, s.pending);
     m->touched = true;
     m->snap_dirty = true;
@@ -1717,7 +1716,7 @@ int mark_set(vdbgpu_map* m, Source& s, uint32_t cap0, Mark&& mark, uint32_t* cou
   for (int attempt = 0;; ++attempt) {
     CK(hipMemsetAsync(&m->d_st[2], 0, sizeof(Status), m->stream));
     if ((r = mark())) return r;
-    CK(launch_compact(m->stream, std::min<int>(4096, (int)((s.cap + 255) / 256)), upd_view(s), s.cap, s.list,
+    CK(launch_compact(m->stream, upd_view(s), s.cap, s.list,
                       &m->d_st[2].entries, &m->d_st[2]));
     if ((r = read_status(m))) return r;
     const Status st = m->h_st[2];
@@ -1742,9 +1741,8 @@ int mark_set(vdbgpu_map* m, Source& s, uint32_t cap0, Mark&& mark, uint32_t* cou
 int apply_edit(vdbgpu_map* m, Source& s, uint32_t count, uint32_t* eidx, int op, float val, bool need,
                bool clear) {
   if (count == 0) return VDBGPU_OK;
-  const int g1 = std::min<int>(4096, (int)((count + 255) / 256));
-  CK(launch_map_insert(m->stream, g1, upd_view(s), s.list, count, map_view(m), eidx, need, need, m->noop4096,
-                       vdbgpu_map::kNoopCap - 1, &m->d_st[1], &m->d_st[2]));
+  CK(launch_map_insert(m->stream, upd_view(s), s.list, count, map_view(m), eidx, need, need, m->noop4096,
+                       vdbgpu_map::kNoopCap - 1, &m->d_st[1]));
   CK(launch_set_voxels(m->stream, upd_view(s), s.list, eidx, count, map_view(m), op, val, m->lo[3], clear));
   m->touched = true;
   m->snap_dirty = true;
@@ -2752,8 +2750,6 @@ int32_t vdbgpu_get_stats(vdbgpu_map* m, vdbgpu_stats* out) {
   m->stats.device_bytes = m->device_bytes;
   m->stats.scratch_bytes = walk_scratch(m, false);
   *out = m->stats;
-  // batch folds count on the host, every k_map_insert on the device
-  out->update_leaves = m->stats.update_leaves + m->h_st[3].entries;
   return VDBGPU_OK;
 }
 

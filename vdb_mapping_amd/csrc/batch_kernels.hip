@@ -104,7 +104,7 @@ __global__ __launch_bounds__(256) void k_group_insert(GroupView gv, const uint32
       const uint32_t gs = glist[g];
       key = batched_to_leaf_key(gv.keys[gs] << 7);  // group keys drop the 7 scan bits
       const bool need = gv.need[gs] != 0;
-      uint32_t p = (uint32_t)fmix64(key) & mp.cap_mask;
+      uint32_t p = map_hash(key) & mp.cap_mask;
       for (uint32_t probe = 0; probe <= mp.cap_mask; ++probe) {
         const unsigned long long k = mp.keys[p];
         if (k == key) {

@@ -195,6 +195,15 @@ __host__ __device__ inline uint64_t fmix64(uint64_t k) {
   return k;
 }
 
+// Slot of a leaf key in the map's leaf hash before probing: the key without the
+// low two bits of its z coordinate is hashed to a group of four slots, so the
+// four leaves of a z column of a brick (neighbouring records) share one 32-byte
+// sector of keys and one 16-byte run of indices instead of eight scattered lines
+// (the map insert of an outdoor scan: 86 -> 44 us).
+__host__ __device__ inline uint32_t map_hash(uint64_t key) {
+  return ((uint32_t)fmix64(key >> 2) << 2) | (uint32_t)(key & 3);
+}
+
 __device__ inline bool coord_ok(int c) { return c >= -kCoordLimit && c < kCoordLimit; }
 
 // Update-set key of the leaf holding (x,y,z): the 63-bit leaf key, or in a

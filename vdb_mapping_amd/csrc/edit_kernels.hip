@@ -285,7 +285,7 @@ __global__ __launch_bounds__(256) void k_upsert_leaves(const unsigned long long*
     if (e < n) {
       key = keys[e];
       const bool nd = need[e] != 0;
-      uint32_t p = (uint32_t)fmix64(key) & mp.cap_mask;
+      uint32_t p = map_hash(key) & mp.cap_mask;
       for (uint32_t probe = 0; probe <= mp.cap_mask; ++probe) {
         const unsigned long long k = mp.keys[p];
         if (k == key) {
@@ -378,7 +378,7 @@ __global__ __launch_bounds__(256) void k_section_tiles(const unsigned long long*
       if (set_has(s128, s128_mask, node_key(x, y, z, 7))) continue;
     }
     const uint64_t key = leaf_key(x, y, z);
-    uint32_t p = (uint32_t)fmix64(key) & mp.cap_mask;
+    uint32_t p = map_hash(key) & mp.cap_mask;
     for (uint32_t probe = 0; probe <= mp.cap_mask; ++probe) {
       const unsigned long long k = mp.keys[p];
       if (k == key) {

@@ -529,6 +529,9 @@ __global__ __launch_bounds__(256) void k_compact(UpdView u, uint32_t cap,
 // One lane per update leaf: find its map leaf, or create it when the update
 // changes a background voxel (OpenVDB creates a child node only when the
 // modify op changes the tile's value or active state).
+// Random accesses bound it: with the leaf hash in groups of four (map_hash) an
+// outdoor scan's 1.7 M records take 44 us instead of 86. One record per lane:
+// two or four per lane left fewer waves to hide the probes (47 and 59 us).
 __global__ __launch_bounds__(kListBlockMax) void k_map_insert(UpdView u, const uint32_t* __restrict__ list,
                                                               uint32_t count, MapView mp,
                                                               uint32_t* __restrict__ eidx,
@@ -560,7 +563,7 @@ __global__ __launch_bounds__(kListBlockMax) void k_map_insert(UpdView u, const u
         }
         need = (anyhit && create_hit) || (anymiss && create_miss);
       }
-      uint32_t p = (uint32_t)fmix64(key) & mp.cap_mask;
+      uint32_t p = map_hash(key) & mp.cap_mask;
       for (uint32_t probe = 0; probe <= mp.cap_mask; ++probe) {
         const unsigned long long k = mp.keys[p];
         if (k == key) {
@@ -929,7 +932,7 @@ __global__ __launch_bounds__(256) void k_rehash_map(MapView mp, uint32_t leaf_co
   const uint32_t G = gridDim.x * blockDim.x;
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < leaf_count; i += G) {
     const uint64_t key = mp.leaf_keys[i];
-    uint32_t p = (uint32_t)fmix64(key) & mp.cap_mask;
+    uint32_t p = map_hash(key) & mp.cap_mask;
     for (uint32_t probe = 0; probe <= mp.cap_mask; ++probe) {
       if (atomicCAS(&mp.keys[p], kEmpty, (unsigned long long)key) == kEmpty) {
         mp.idx[p] = i;

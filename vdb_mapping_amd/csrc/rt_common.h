@@ -73,7 +73,7 @@ struct ActiveProbe {
     if (k != key) {
       key = k;
       idx = kNone;
-      uint32_t h = (uint32_t)fmix64(k) & mp.cap_mask;
+      uint32_t h = map_hash(k) & mp.cap_mask;
       for (uint32_t p = 0; p <= mp.cap_mask; ++p) {
         const unsigned long long kk = mp.keys[h];
         if (kk == k) {

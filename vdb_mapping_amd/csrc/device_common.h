@@ -160,15 +160,35 @@ __host__ __device__ inline bool tile_active(const TileView& t, uint32_t i) {
   return (t.on[i >> 5] >> (i & 31)) & 1u;
 }
 
-// Topology snapshot used by raytrace: hash sets of leaf, 128^3-node and
-// 4096^3-node keys, plus the padded bbox of leaves with an active voxel.
+// Topology snapshot used by raytrace and the fast-mode raycast: a hash of the
+// 128^3 nodes (key -> node index), one bit per leaf of every node, a hash set
+// of the 4096^3 node keys, and the padded bbox of leaves with an active voxel.
+// A node's 4,096 leaf bits are 64 words of 4 x 4 x 4 leaves, so a ray reads a
+// word once for the two or three leaves it crosses in it; beside each word the
+// one of the leaves that held an active voxel when the snapshot was taken.
 struct RtView {
-  unsigned long long* leaf;
   unsigned long long* n128;
+  uint32_t* nidx;             // node index of each slot of n128
+  unsigned long long* bits;   // per node 64 x (leaves, leaves with an active voxel)
   unsigned long long* n4096;
-  uint32_t leaf_mask, n128_mask, n4096_mask;
+  uint32_t n128_mask, n4096_mask;
+  uint32_t live;              // 1: the map changed since, active states are read from it alone
   int bmin[3], bmax[3];
 };
+constexpr uint32_t kRtNodeWords = 128;  // words of RtView::bits per node
+// What a snapshot build hands back: bbox (min, max) of leaves with an active
+// voxel, nodes in the hash, leaves covered.
+struct RtInfo {
+  int bbox[6];
+  unsigned int nodes, leaves;
+};
+// Word and bit of the leaf at (x, y, z) in its 128^3 node.
+__host__ __device__ inline int rt_word(int x, int y, int z) {
+  return (((x >> 5) & 3) << 4) | (((y >> 5) & 3) << 2) | ((z >> 5) & 3);
+}
+__host__ __device__ inline int rt_bit(int x, int y, int z) {
+  return (((x >> 3) & 3) << 4) | (((y >> 3) & 3) << 2) | ((z >> 3) & 3);
+}
 
 __host__ __device__ inline uint64_t leaf_key(int x, int y, int z) {
   const uint64_t m = (1ull << 21) - 1;
@@ -251,6 +271,19 @@ __device__ __forceinline__ bool set_insert(unsigned long long* keys, uint32_t ma
     h = (h + 1) & mask;
   }
   return false;
+}
+
+// set_insert for keys that are mostly present: a read first, since atomics on
+// one address (every leaf of a node, every node of a root child) run one
+// after another.
+__device__ __forceinline__ void set_add(unsigned long long* keys, uint32_t mask, uint64_t key) {
+  uint32_t h = (uint32_t)fmix64(key) & mask;
+  for (uint32_t p = 0; p <= mask; ++p) {
+    unsigned long long k = __hip_atomic_load(&keys[h], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (k == kEmpty) k = atomicCAS(&keys[h], kEmpty, (unsigned long long)key);
+    if (k == kEmpty || k == key) return;
+    h = (h + 1) & mask;
+  }
 }
 
 __device__ __forceinline__ bool set_has(const unsigned long long* __restrict__ keys, uint32_t mask,

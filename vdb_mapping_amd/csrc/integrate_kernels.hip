@@ -425,15 +425,16 @@ __global__ __launch_bounds__(256) void k_traverse(const int4* __restrict__ rayin
 // probes its origin voxel. Endpoints inside max range are hits as in the
 // normal path (VDBMapping.hpp:533-536). cast == 0 (the map is empty,
 // VDBMapping.hpp:495, :522): endpoints only.
-__global__ __launch_bounds__(256) void k_fast_cast(const int4* __restrict__ rayinfo,
+__global__ __launch_bounds__(256, 4) void k_fast_cast(const int4* __restrict__ rayinfo,
                                                    const ScanInfo* __restrict__ scans,
                                                    const BatchCtl* __restrict__ ctl, RtView rt,
                                                    MapView mp, UpdView u, uint32_t cast,
-                                                   Status* st) {
+                                                   Status* st, int spread) {
   const uint32_t n = ctl->n_rays;
   unsigned int* ovf = &st->overflow;
-  const uint32_t G = gridDim.x * blockDim.x;
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += G) {
+  const uint32_t G = (gridDim.x * blockDim.x) >> spread;
+  if (threadIdx.x & ((1u << spread) - 1)) return;
+  for (uint32_t i = (blockIdx.x * blockDim.x + threadIdx.x) >> spread; i < n; i += G) {
     const int4 r = rayinfo[i];
     const uint32_t wbits = (uint32_t)r.w;
     if (!(wbits & kValidBit)) continue;
@@ -442,61 +443,30 @@ __global__ __launch_bounds__(256) void k_fast_cast(const int4* __restrict__ rayi
     const uint32_t sc = (wbits >> kScanShift) & kScanMask;
     const int s[3] = {scans[sc].s[0], scans[sc].s[1], scans[sc].s[2]};
     const int e[3] = {r.x, r.y, r.z};
-    double eye[3], dir[3], idir[3];
+    RtRay ray;
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-      eye[a] = (double)s[a] + 0.5;
-      dir[a] = (double)e[a] - (double)s[a];
-      idir[a] = 1.0 / dir[a];
+      ray.eye[a] = (double)s[a] + 0.5;
+      ray.dir[a] = (double)e[a] - (double)s[a];
+      ray.idir[a] = 1.0 / ray.dir[a];
     }
     // every DDA level takes at most |dir|_1 / dim + 3 steps over t in [0, 1]
-    int budget = 4 * ((int)(fabs(dir[0]) + fabs(dir[1]) + fabs(dir[2])) + 8);
+    int budget = 4 * ((int)(fabs(ray.dir[0]) + fabs(ray.dir[1]) + fabs(ray.dir[2])) + 8);
     double rt0 = 0.0, rt1 = 1.0;
-    rt_clip(rt, eye, idir, rt0, rt1);
+    rt_clip(rt, ray, rt0, rt1);
+    LeafBits lb;
     ActiveProbe probe;
-    auto walk_span = [&](double t0, double t1) {
-      RtDda fd;
-      fd.init(eye, dir, idir, t0, t1, 0);
+    SpanFinder<false> f;
+    f.init(ray, rt0, rt1);
+    double t0, t1;
+    while (f.next(rt, ray, lb, budget, t0, t1)) {
+      RtDda<1> fd;
+      fd.init(ray, t0, t1);
       do {
-        if (probe.on(mp, fd.vox[0], fd.vox[1], fd.vox[2])) mark_voxel(u, ovf, fd.vox[0], fd.vox[1], fd.vox[2], false);
-      } while (fd.step() && --budget > 0);
-    };
-    double s0 = -1, s1 = -1;  // the open TimeSpan
-    RtDda d12;
-    d12.init(eye, dir, idir, rt0, rt1, 12);
-    do {
-      if (set_has(rt.n4096, rt.n4096_mask, node_key(d12.vox[0], d12.vox[1], d12.vox[2], 12))) {
-        RtDda d7;
-        d7.init(eye, dir, idir, d12.t0, d12.next(), 7);
-        do {
-          if (set_has(rt.n128, rt.n128_mask, node_key(d7.vox[0], d7.vox[1], d7.vox[2], 7))) {
-            RtDda d3;
-            d3.init(eye, dir, idir, d7.t0, d7.next(), 3);
-            do {
-              if (set_has(rt.leaf, rt.leaf_mask, leaf_key(d3.vox[0], d3.vox[1], d3.vox[2]))) {
-                if (s0 < 0) s0 = d3.t0;
-              } else if (s0 >= 0) {
-                s1 = d3.t0;
-                if (span_valid(s0, s1)) walk_span(s0, s1);
-                s0 = s1 = -1;
-              }
-            } while (d3.step() && --budget > 0);
-            if (s0 >= 0) s1 = d3.t1;
-          } else if (s0 >= 0) {
-            s1 = d7.t0;
-            if (span_valid(s0, s1)) walk_span(s0, s1);
-            s0 = s1 = -1;
-          }
-        } while (d7.step() && --budget > 0);
-        if (s0 >= 0) s1 = d7.t1;
-      } else if (s0 >= 0) {
-        s1 = d12.t0;
-        if (span_valid(s0, s1)) walk_span(s0, s1);
-        s0 = s1 = -1;
-      }
-    } while (d12.step() && --budget > 0);
-    if (s0 >= 0) s1 = d12.t1;
-    if (span_valid(s0, s1)) walk_span(s0, s1);
+        if (probe.leaf(mp, rt, lb, fd.vox) && probe.on(mp, fd.vox))
+          mark_voxel(u, ovf, fd.vox[0], fd.vox[1], fd.vox[2], false);
+      } while (fd.step(ray) && --budget > 0);
+    }
     if (budget <= 0) atomicOr(&st->error, kErrWalk);
   }
 }
@@ -1052,11 +1022,13 @@ hipError_t launch_traverse(hipStream_t s, int grid, int block, const int4* rayin
   return hipGetLastError();
 }
 
-hipError_t launch_fast_cast(hipStream_t s, int grid, const int4* rayinfo, const ScanInfo* scans,
+hipError_t launch_fast_cast(hipStream_t s, int num_cu, uint32_t n, const int4* rayinfo, const ScanInfo* scans,
                             const BatchCtl* ctl, RtView rt, MapView mp, UpdView u, bool cast,
                             Status* st) {
+  const int spread = cast ? ray_spread(n, num_cu) : 0;
+  const int grid = (int)std::min<uint64_t>((uint64_t)num_cu * 8, (((uint64_t)n << spread) + 255) / 256);
   hipLaunchKernelGGL(k_fast_cast, dim3(grid), dim3(256), 0, s, rayinfo, scans, ctl, rt, mp, u,
-                     (uint32_t)cast, st);
+                     (uint32_t)cast, st, spread);
   return hipGetLastError();
 }
 

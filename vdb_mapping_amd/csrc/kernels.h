@@ -21,7 +21,7 @@ hipError_t launch_traverse(hipStream_t s, int grid, int block, const int4* rayin
                            const uint64_t* roff, const uint32_t* first_ray, const ScanInfo* scans,
                            const BatchCtl* ctl, const double* tbl, UpdView u, Status* st,
                            uint32_t chunk);
-hipError_t launch_fast_cast(hipStream_t s, int grid, const int4* rayinfo, const ScanInfo* scans,
+hipError_t launch_fast_cast(hipStream_t s, int num_cu, uint32_t n, const int4* rayinfo, const ScanInfo* scans,
                             const BatchCtl* ctl, RtView rt, MapView mp, UpdView u, bool cast,
                             Status* st);
 hipError_t launch_compact(hipStream_t s, UpdView u, uint32_t cap, uint32_t* list,
@@ -102,10 +102,12 @@ hipError_t launch_split_emit(hipStream_t s, int grid, const uint32_t* split_slot
                              unsigned long long* shared_bits, BrickView bv, UpdView rec,
                              unsigned long long* leaf_mask, uint32_t rec_cap, Status* st);
 
-hipError_t launch_snapshot(hipStream_t s, MapView mp, uint32_t leaf_count, RtView rt, int* bbox, TileView tv);
-hipError_t launch_copy_set(hipStream_t s, const unsigned long long* src, uint32_t src_cap,
-                           unsigned long long* dst, uint32_t dst_mask);
-hipError_t launch_raytrace(hipStream_t s, int grid, RtView rt, MapView mp, double inv, double res,
+hipError_t launch_snapshot_nodes(hipStream_t s, MapView mp, uint32_t first, uint64_t leaf_bound, RtView rt,
+                                 RtInfo* info, const unsigned long long* noop, uint32_t noop_cap,
+                                 uint32_t old_nodes, const Status* stmap, bool full);
+hipError_t launch_snapshot_bits(hipStream_t s, MapView mp, uint32_t first, uint32_t leaf_count, RtView rt,
+                                const RtInfo* info, TileView tv);
+hipError_t launch_raytrace(hipStream_t s, int num_cu, RtView rt, MapView mp, double inv, double res,
                            int64_t n, const double* origins, const double* dirs,
                            const double* lens, uint8_t* success, double* ends, unsigned int* err);
 

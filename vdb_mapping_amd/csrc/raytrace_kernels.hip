@@ -5,9 +5,13 @@
 // copy of the map at that moment, walked by a hierarchical DDA over node sizes
 // 4096 -> 128 -> 8 (math::VolumeHDDA), then a voxel DDA that stops at the first
 // active voxel of the live map. Here the topology copy is a snapshot of three
-// device hash sets (leaves, 128^3 nodes, 4096^3 nodes) plus the padded
-// bounding box of the leaves holding an active voxel; one lane walks one ray
-// with exactly the double-precision operations of math::Ray / math::DDA.
+// device sets (a bit per leaf under a hash of 128^3 nodes, a hash of 4096^3
+// nodes) plus the padded bounding box of the leaves holding an active voxel;
+// one lane walks one ray with exactly the double-precision operations of
+// math::Ray / math::DDA. The steps themselves cannot be skipped (their times
+// are accumulated sums), so the lookups beside them are what there is to save:
+// a leaf step reads a bit of a word it mostly holds already, a voxel step
+// tests the OR of its leaf's mask words first.
 //
 // Build with -ffp-contract=off (every double operation rounds on its own).
 #include <float.h>
@@ -20,24 +24,43 @@ namespace vdbgpu {
 
 __device__ __forceinline__ int rt_lane() { return (int)__lane_id(); }
 
-// Snapshot of the map topology: every leaf, its 128^3 and 4096^3 parents, and
-// the leaf-granular bounding box of active voxels (evalActiveBoundingBox with
-// visitVoxels = false). One block-level min/max reduction per workgroup.
-__global__ __launch_bounds__(256) void k_snapshot(MapView mp, uint32_t leaf_count,
-                                                  RtView rt, int* __restrict__ bbox, TileView tv) {
+// Start of a snapshot build: empty bbox, the leaf count at this point of the
+// stream, and on a full build no nodes.
+__global__ void k_snapshot_begin(RtInfo* info, const Status* stmap, uint32_t full) {
+  if (threadIdx.x == 0) {
+    for (int a = 0; a < 3; ++a) {
+      info->bbox[a] = INT_MAX;
+      info->bbox[3 + a] = INT_MIN;
+    }
+    info->leaves = stmap->leaf_count;
+    if (full) info->nodes = 0;
+  }
+}
+
+// Nodes of the snapshot: the 128^3 and 4096^3 parents of the leaves from
+// `first` on (leaves are only ever appended to the pool, so the earlier ones
+// are in), the root children of updates that created no leaf (value and state
+// unchanged, e.g. probability 0.5), and the leaf-granular bounding box of
+// active voxels (evalActiveBoundingBox with visitVoxels = false) of all
+// leaves. Every atomic is preceded by a read: the parents and the box are the
+// same few addresses for the whole grid (116 us of a fast-mode scan with an
+// atomic per leaf).
+__global__ __launch_bounds__(256) void k_snapshot_nodes(MapView mp, uint32_t first, RtView rt, RtInfo* info,
+                                                        const unsigned long long* __restrict__ noop,
+                                                        uint32_t noop_cap, uint32_t old_nodes) {
   __shared__ int smin[3][4], smax[3][4];
   int lo[3] = {INT_MAX, INT_MAX, INT_MAX}, hi[3] = {INT_MIN, INT_MIN, INT_MIN};
-  const uint32_t G = gridDim.x * blockDim.x;
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < leaf_count; i += G) {
-    const uint64_t key = mp.leaf_keys[i];
+  const uint32_t leaf_count = info->leaves;
+  const uint32_t G = gridDim.x * blockDim.x, t = blockIdx.x * blockDim.x + threadIdx.x;
+  for (uint32_t i = t; i < noop_cap; i += G)
+    if (noop[i] != kEmpty) set_add(rt.n4096, rt.n4096_mask, noop[i]);
+  // active leaves are listed anew by the next launch
+  for (uint64_t i = t; i < (uint64_t)old_nodes * 64; i += G) rt.bits[2 * i + 1] = 0;
+  for (uint32_t i = t; i < leaf_count; i += G) {
     int o[3];
-    key_origin(key, o);
-    // an inactive tile is neither a leaf nor an active value for the HDDA; an active
-    // tile is a hit at the leaf level, as a leaf is
-    if (!tile_at(tv, i) || tile_active(tv, i)) set_insert(rt.leaf, rt.leaf_mask, key);
-    set_insert(rt.n128, rt.n128_mask, node_key(o[0], o[1], o[2], 7));
-    set_insert(rt.n4096, rt.n4096_mask, node_key(o[0], o[1], o[2], 12));
+    key_origin(mp.leaf_keys[i], o);
     uint64_t any = 0;
+#pragma unroll
     for (int j = 0; j < 8; ++j) any |= mp.active[(size_t)i * 8 + j];
     if (any) {
 #pragma unroll
@@ -45,6 +68,22 @@ __global__ __launch_bounds__(256) void k_snapshot(MapView mp, uint32_t leaf_coun
         lo[a] = min(lo[a], o[a]);
         hi[a] = max(hi[a], o[a] + 7);
       }
+    }
+    if (i < first) continue;
+    const uint64_t key = node_key(o[0], o[1], o[2], 7);
+    uint32_t h = (uint32_t)fmix64(key) & rt.n128_mask;
+    for (uint32_t p = 0; p <= rt.n128_mask; ++p) {
+      unsigned long long k = __hip_atomic_load(&rt.n128[h], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (k == kEmpty) {
+        k = atomicCAS(&rt.n128[h], kEmpty, (unsigned long long)key);
+        if (k == kEmpty) {  // a new node: its index is read by the next launch
+          rt.nidx[h] = atomicAdd(&info->nodes, 1u);
+          set_add(rt.n4096, rt.n4096_mask, node_key(o[0], o[1], o[2], 12));
+          break;
+        }
+      }
+      if (k == key) break;
+      h = (h + 1) & rt.n128_mask;
     }
   }
 #pragma unroll
@@ -70,34 +109,59 @@ __global__ __launch_bounds__(256) void k_snapshot(MapView mp, uint32_t leaf_coun
       l = min(l, smin[a][k]);
       h = max(h, smax[a][k]);
     }
-    if (l != INT_MAX) atomicMin(&bbox[a], l);
-    if (h != INT_MIN) atomicMax(&bbox[3 + a], h);
+    if (l < __hip_atomic_load(&info->bbox[a], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      atomicMin(&info->bbox[a], l);
+    if (h > __hip_atomic_load(&info->bbox[3 + a], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      atomicMax(&info->bbox[3 + a], h);
   }
 }
 
-// Root children created by updates that created no leaf (value and state
-// unchanged, e.g. probability 0.5): kept so the snapshot sees them too.
-__global__ __launch_bounds__(256) void k_copy_set(const unsigned long long* __restrict__ src,
-                                                  uint32_t src_cap, unsigned long long* dst,
-                                                  uint32_t dst_mask) {
+// Leaf bits of the leaves from `first` on, active bits of all. An inactive
+// tile is neither a leaf nor an active value for the HDDA; an active tile is a
+// hit at the leaf level, as a leaf is.
+__global__ __launch_bounds__(256) void k_snapshot_bits(MapView mp, uint32_t first, RtView rt, const RtInfo* info,
+                                                       TileView tv) {
+  const uint32_t leaf_count = info->leaves;
   const uint32_t G = gridDim.x * blockDim.x;
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < src_cap; i += G)
-    if (src[i] != kEmpty) set_insert(dst, dst_mask, src[i]);
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < leaf_count; i += G) {
+    uint64_t any = 0;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) any |= mp.active[(size_t)i * 8 + j];
+    const bool leaf = i >= first && !(tile_at(tv, i) && !tile_active(tv, i));
+    if (!leaf && !any) continue;
+    int o[3];
+    key_origin(mp.leaf_keys[i], o);
+    const uint64_t key = node_key(o[0], o[1], o[2], 7);
+    uint32_t h = (uint32_t)fmix64(key) & rt.n128_mask;
+    for (uint32_t p = 0; p <= rt.n128_mask; ++p) {
+      const unsigned long long k = rt.n128[h];
+      if (k == key) {
+        unsigned long long* w = &rt.bits[(size_t)rt.nidx[h] * kRtNodeWords + 2 * rt_word(o[0], o[1], o[2])];
+        const unsigned long long bit = 1ull << rt_bit(o[0], o[1], o[2]);
+        if (leaf) atomicOr(&w[0], bit);
+        if (any) atomicOr(&w[1], bit);
+        break;
+      }
+      if (k == kEmpty) break;
+      h = (h + 1) & rt.n128_mask;
+    }
+  }
 }
 
 // One lane per query ray. Mirrors VDBMapping::raytrace: normalise (multiply by
 // 1/length unless length <= 1e-7), scale by the max length, continuous
 // worldToIndex, clip to the padded bbox (result ignored), VolumeHDDA march,
 // then a voxel DDA over the first leaf run that stops at an active voxel.
-__global__ __launch_bounds__(256) void k_raytrace(RtView rt, MapView mp, double inv, double res,
+__global__ __launch_bounds__(256, 4) void k_raytrace(RtView rt, MapView mp, double inv, double res,
                                                   int64_t n, const double* __restrict__ origins,
                                                   const double* __restrict__ dirs,
                                                   const double* __restrict__ lens,
                                                   uint8_t* __restrict__ success,
                                                   double* __restrict__ ends,
-                                                  unsigned int* __restrict__ err) {
-  const int64_t G = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += G) {
+                                                  unsigned int* __restrict__ err, int spread) {
+  const int64_t G = ((int64_t)gridDim.x * blockDim.x) >> spread;
+  if (threadIdx.x & ((1 << spread) - 1)) return;
+  for (int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> spread; i < n; i += G) {
     double d[3] = {dirs[3 * i], dirs[3 * i + 1], dirs[3 * i + 2]};
     const double len = sqrt(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]);
     if (!(fabs(0.0 - len) <= 1e-7)) {
@@ -107,18 +171,18 @@ __global__ __launch_bounds__(256) void k_raytrace(RtView rt, MapView mp, double 
       d[2] *= r;
     }
     const double L = lens[i];
-    double eye[3], dir[3], idir[3];
+    RtRay r;
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
       d[a] *= L;
-      eye[a] = origins[3 * i + a] * inv;
-      dir[a] = d[a] * inv;
-      idir[a] = 1.0 / dir[a];
+      r.eye[a] = origins[3 * i + a] * inv;
+      r.dir[a] = d[a] * inv;
+      r.idir[a] = 1.0 / r.dir[a];
     }
     // A query whose DDA cannot end (non-finite numbers) or would take more
     // than kMaxQuerySteps voxel steps is rejected instead of marched.
-    const double span = fabs(dir[0]) + fabs(dir[1]) + fabs(dir[2]);
-    if (!(isfinite(eye[0]) && isfinite(eye[1]) && isfinite(eye[2]) && isfinite(span) &&
+    const double span = fabs(r.dir[0]) + fabs(r.dir[1]) + fabs(r.dir[2]);
+    if (!(isfinite(r.eye[0]) && isfinite(r.eye[1]) && isfinite(r.eye[2]) && isfinite(span) &&
           span < (double)kMaxQuerySteps)) {
       atomicOr(err, 1u);
       success[i] = 0;
@@ -128,83 +192,31 @@ __global__ __launch_bounds__(256) void k_raytrace(RtView rt, MapView mp, double 
     // every DDA level takes at most span/dim + 3 steps over t in [0, 1]
     int budget = 4 * ((int)span + 8);
     double rt0 = 0.0, rt1 = 1.0;
-    {  // Ray::clip to the padded active bbox
-      double c0 = rt0, c1 = rt1;
-      bool hit = true;
-#pragma unroll
-      for (int a = 0; a < 3; ++a) {
-        if (!hit) break;
-        double ta = ((double)rt.bmin[a] - eye[a]) * idir[a];
-        double tb = ((double)rt.bmax[a] - eye[a]) * idir[a];
-        if (ta > tb) {
-          const double t = ta;
-          ta = tb;
-          tb = t;
-        }
-        if (ta > c0) c0 = ta;
-        if (tb < c1) c1 = tb;
-        if (c0 > c1) hit = false;
-      }
-      if (hit) {
-        rt0 = c0;
-        rt1 = c1;
-      }
-    }
-    double s0 = -1, s1 = -1;  // TimeSpan of the first leaf run
+    rt_clip(rt, r, rt0, rt1);  // Ray::clip to the padded active bbox
+    double s0 = -1, s1 = -1;   // TimeSpan of the first leaf run
+    LeafBits lb;
+    bool run = false;
     if ((rt1 - rt0) > (double)1e-5f) {  // Ray::valid
-      bool done = false;
-      RtDda d12;
-      d12.init(eye, dir, idir, rt0, rt1, 12);
-      do {
-        if (set_has(rt.n4096, rt.n4096_mask, node_key(d12.vox[0], d12.vox[1], d12.vox[2], 12))) {
-          RtDda d7;
-          d7.init(eye, dir, idir, d12.t0, d12.next(), 7);
-          do {
-            if (set_has(rt.n128, rt.n128_mask, node_key(d7.vox[0], d7.vox[1], d7.vox[2], 7))) {
-              RtDda d3;
-              d3.init(eye, dir, idir, d7.t0, d7.next(), 3);
-              do {
-                if (set_has(rt.leaf, rt.leaf_mask, leaf_key(d3.vox[0], d3.vox[1], d3.vox[2]))) {
-                  if (s0 < 0) s0 = d3.t0;
-                } else if (s0 >= 0) {
-                  s1 = d3.t0;
-                  if (span_valid(s0, s1)) {
-                    done = true;
-                    break;
-                  }
-                  s0 = s1 = -1;
-                }
-              } while (d3.step() && --budget > 0);
-              if (done) break;
-              if (s0 >= 0) s1 = d3.t1;
-            } else if (s0 >= 0) {
-              s1 = d7.t0;
-              if (span_valid(s0, s1)) {
-                done = true;
-                break;
-              }
-              s0 = s1 = -1;
-            }
-          } while (d7.step() && --budget > 0);
-          if (done) break;
-          if (s0 >= 0) s1 = d7.t1;
-        } else if (s0 >= 0) {
-          s1 = d12.t0;
-          if (span_valid(s0, s1)) {
-            done = true;
-            break;
-          }
-          s0 = s1 = -1;
-        }
-      } while (d12.step() && --budget > 0);
-      if (!done && s0 >= 0) s1 = d12.t1;
+      SpanFinder<true> f;
+      f.init(r, rt0, rt1);
+      run = f.next(rt, r, lb, budget, s0, s1);
     }
     double* out = ends + 3 * i;
-    if (span_valid(s0, s1)) {
-      RtDda fd;
-      fd.init(eye, dir, idir, s0, s1, 0);
+    if (run) {
+      RtDda<1> fd;
+      fd.init(r, s0, s1);
       ActiveProbe probe;
-      while (fd.step() && !probe.on(mp, fd.vox[0], fd.vox[1], fd.vox[2]) && --budget > 0) {
+      // to the first active voxel after the first one; a leaf without any is
+      // left in one go
+      bool can_skip = true;  // refused once: the run ends in that leaf
+      for (;;) {
+        int n = 1;
+        bool moved = can_skip && !probe.leaf(mp, rt, lb, fd.vox);
+        if (moved) moved = can_skip = fd.skip<8>(r, n);
+        if (!moved && !fd.step(r)) break;
+        budget -= n - 1;
+        if (probe.leaf(mp, rt, lb, fd.vox) && probe.on(mp, fd.vox)) break;
+        if (--budget <= 0) break;
       }
       if (budget <= 0) atomicOr(err, 2u);
 #pragma unroll
@@ -212,31 +224,39 @@ __global__ __launch_bounds__(256) void k_raytrace(RtView rt, MapView mp, double 
       success[i] = 1;
     } else {
 #pragma unroll
-      for (int a = 0; a < 3; ++a) out[a] = (eye[a] + dir[a]) * res;
+      for (int a = 0; a < 3; ++a) out[a] = (r.eye[a] + r.dir[a]) * res;
       success[i] = 0;
     }
   }
 }
 
-hipError_t launch_snapshot(hipStream_t s, MapView mp, uint32_t leaf_count, RtView rt, int* bbox, TileView tv) {
-  const int grid = (int)std::min<uint32_t>(4096, (leaf_count + 255) / 256 + 1);
-  hipLaunchKernelGGL(k_snapshot, dim3(grid), dim3(256), 0, s, mp, leaf_count, rt, bbox, tv);
+hipError_t launch_snapshot_nodes(hipStream_t s, MapView mp, uint32_t first, uint64_t leaf_bound, RtView rt,
+                                 RtInfo* info, const unsigned long long* noop, uint32_t noop_cap,
+                                 uint32_t old_nodes, const Status* stmap, bool full) {
+  hipLaunchKernelGGL(k_snapshot_begin, dim3(1), dim3(64), 0, s, info, stmap, full ? 1u : 0u);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  const int grid = (int)std::min<uint64_t>(2048, (std::max<uint64_t>(leaf_bound, noop_cap) + 255) / 256);
+  hipLaunchKernelGGL(k_snapshot_nodes, dim3(grid), dim3(256), 0, s, mp, first, rt, info, noop, noop_cap, old_nodes);
   return hipGetLastError();
 }
 
-hipError_t launch_copy_set(hipStream_t s, const unsigned long long* src, uint32_t src_cap,
-                           unsigned long long* dst, uint32_t dst_mask) {
-  const int grid = (int)std::min<uint32_t>(4096, (src_cap + 255) / 256);
-  hipLaunchKernelGGL(k_copy_set, dim3(grid), dim3(256), 0, s, src, src_cap, dst, dst_mask);
+hipError_t launch_snapshot_bits(hipStream_t s, MapView mp, uint32_t first, uint32_t leaf_count, RtView rt,
+                                const RtInfo* info, TileView tv) {
+  if (leaf_count == 0) return hipSuccess;
+  const int grid = (int)std::min<uint32_t>(2048, (leaf_count + 255) / 256);
+  hipLaunchKernelGGL(k_snapshot_bits, dim3(grid), dim3(256), 0, s, mp, first, rt, info, tv);
   return hipGetLastError();
 }
 
-hipError_t launch_raytrace(hipStream_t s, int grid, RtView rt, MapView mp, double inv, double res,
+hipError_t launch_raytrace(hipStream_t s, int num_cu, RtView rt, MapView mp, double inv, double res,
                            int64_t n, const double* origins, const double* dirs,
                            const double* lens, uint8_t* success, double* ends,
                            unsigned int* err) {
+  const int spread = ray_spread(n, num_cu);
+  const int grid = (int)std::min<int64_t>((int64_t)num_cu * 16, ((n << spread) + 255) / 256);
   hipLaunchKernelGGL(k_raytrace, dim3(grid), dim3(256), 0, s, rt, mp, inv, res, n, origins, dirs,
-                     lens, success, ends, err);
+                     lens, success, ends, err, spread);
   return hipGetLastError();
 }
 

@@ -123,8 +123,13 @@ struct vdbgpu_map {
   // raytrace topology snapshot (updateVolumeRayIntersectors)
   bool has_isect = false;
   RtView rt{};
-  uint32_t rt_leaf_cap = 0, rt_n128_cap = 0, rt_n4096_cap = 0;
-  int* d_bbox = nullptr;
+  uint32_t rt_n128_cap = 0, rt_n4096_cap = 0, rt_node_cap = 0;
+  RtInfo* rt_info = nullptr;    // device
+  RtInfo* h_rt_info = nullptr;  // pinned
+  // pool leaves the snapshot covers; the next build adds the ones after them,
+  // or starts over (rt_full: the grid was emptied, tiles came or went)
+  uint32_t rt_leaves = 0, rt_nodes = 0;
+  bool rt_full = true;
   // raytrace query staging
   // batch: scan table, control block, fold groups
   ScanInfo* d_scans = nullptr;
@@ -420,6 +425,14 @@ UpdView upd_view(const Source& s) { return UpdView{s.keys, s.masks, s.cap - 1}; 
 
 MapView map_view(vdbgpu_map* m) {
   return MapView{m->mkeys, m->midx, m->mcap - 1, m->values, m->active, m->leaf_keys, m->dirty, m->lcap};
+}
+
+// The snapshot as queries see it: its active-leaf bits count only while the
+// map is unchanged since it was taken.
+RtView rt_view(const vdbgpu_map* m) {
+  RtView v = m->rt;
+  v.live = m->snap_dirty ? 1u : 0u;
+  return v;
 }
 
 TileView tile_view(const vdbgpu_map* m) {
@@ -993,11 +1006,10 @@ int run_fast(vdbgpu_map* m, Source& src, const float* xyz, int64_t n, int64_t st
   if (src.cap == 0) {
     if ((r = alloc_update(m, src, (uint32_t)std::max<uint64_t>(kMinUpdateCap, next_pow2(4 * (uint64_t)n))))) return r;
   }
-  const int grid = std::min<int>(m->num_cu * 8, (int)((n + 255) / 256));
   for (int attempt = 0;; ++attempt) {
     {
       Timer t(m, kTraverse);
-      CK(launch_fast_cast(m->stream, grid, m->rayinfo, m->d_scans, m->d_ctl, m->rt, map_view(m),
+      CK(launch_fast_cast(m->stream, m->num_cu, (uint32_t)n, m->rayinfo, m->d_scans, m->d_ctl, rt_view(m), map_view(m),
                           upd_view(src), cast, &m->d_st[0]));
     }
     {
@@ -1581,40 +1593,71 @@ void create_flags(const vdbgpu_map* m, bool* ch, bool* cm) {
 // updateVolumeRayIntersectors (VDBMapping.hpp:1436-1449): in fast mode, a
 // non-empty map gets a fresh topology snapshot after every integrate.
 int build_snapshot(vdbgpu_map* m) {
-  int r = read_status(m);
-  if (r) return r;
-  const uint32_t L = m->h_st[1].leaf_count;
-  const uint32_t cap = (uint32_t)std::max<uint64_t>(1024, next_pow2(2ull * L + 2));
-  const uint32_t cap_root = (uint32_t)std::max<uint64_t>(1024, next_pow2(2ull * L + 2 * vdbgpu_map::kNoopCap));
-  if (cap > m->rt_leaf_cap) {
-    dfree(m, &m->rt.leaf, m->rt_leaf_cap);
+  if (!m->rt_info) {
+    CK(dalloc(m, &m->rt_info, 1));
+    CK(hipHostMalloc((void**)&m->h_rt_info, sizeof(RtInfo), hipHostMallocDefault));
+  }
+  auto tables_fit = [&] {
+    return 2 * m->leaf_count_ub + 2 <= m->rt_n128_cap &&
+           2 * m->leaf_count_ub + 2 * vdbgpu_map::kNoopCap <= m->rt_n4096_cap;
+  };
+  int r;
+  // the tables are sized for every leaf in a node of its own; ones that grow
+  // (for the exact leaf count) start over
+  if (!tables_fit() && (r = read_status(m))) return r;
+  if (!tables_fit()) {
+    const uint64_t ub = m->leaf_count_ub;
+    m->has_isect = false;  // until this build is through
+    m->rt_full = true;
     dfree(m, &m->rt.n128, m->rt_n128_cap);
-    m->rt_leaf_cap = m->rt_n128_cap = cap;
-    CK(dalloc(m, &m->rt.leaf, cap));
-    CK(dalloc(m, &m->rt.n128, cap));
-  }
-  if (cap_root > m->rt_n4096_cap) {
+    dfree(m, &m->rt.nidx, m->rt_n128_cap);
     dfree(m, &m->rt.n4096, m->rt_n4096_cap);
-    m->rt_n4096_cap = cap_root;
-    CK(dalloc(m, &m->rt.n4096, cap_root));
+    m->rt_n128_cap = (uint32_t)std::min<uint64_t>(1u << 31, std::max<uint64_t>(1024, next_pow2(2 * ub + 2)));
+    m->rt_n4096_cap = (uint32_t)std::min<uint64_t>(1u << 31, next_pow2(2 * ub + 2 * vdbgpu_map::kNoopCap));
+    if (dalloc(m, &m->rt.n128, m->rt_n128_cap) != hipSuccess || dalloc(m, &m->rt.nidx, m->rt_n128_cap) != hipSuccess ||
+        dalloc(m, &m->rt.n4096, m->rt_n4096_cap) != hipSuccess) {
+      dfree(m, &m->rt.n128, m->rt_n128_cap);
+      dfree(m, &m->rt.nidx, m->rt_n128_cap);
+      m->rt_n128_cap = m->rt_n4096_cap = 0;
+      return fail(m, VDBGPU_DEVICE_ERROR, "out of device memory for the topology snapshot");
+    }
   }
-  m->rt.leaf_mask = m->rt_leaf_cap - 1;
   m->rt.n128_mask = m->rt_n128_cap - 1;
   m->rt.n4096_mask = m->rt_n4096_cap - 1;
-  CK(launch_fill_u64(m->stream, m->rt.leaf, m->rt_leaf_cap, kEmpty));
-  CK(launch_fill_u64(m->stream, m->rt.n128, m->rt_n128_cap, kEmpty));
-  CK(launch_fill_u64(m->stream, m->rt.n4096, m->rt_n4096_cap, kEmpty));
-  if (!m->d_bbox) CK(dalloc(m, &m->d_bbox, 6));
-  int hb[6] = {INT_MAX, INT_MAX, INT_MAX, INT_MIN, INT_MIN, INT_MIN};
-  CK(hipMemcpyAsync(m->d_bbox, hb, sizeof hb, hipMemcpyHostToDevice, m->stream));
-  if (L) CK(launch_snapshot(m->stream, map_view(m), L, m->rt, m->d_bbox, tile_view(m)));
-  CK(launch_copy_set(m->stream, m->noop4096, vdbgpu_map::kNoopCap, m->rt.n4096, m->rt.n4096_mask));
-  CK(hipMemcpyAsync(hb, m->d_bbox, sizeof hb, hipMemcpyDeviceToHost, m->stream));
-  CK(hipStreamSynchronize(m->stream));
-  for (int a = 0; a < 3; ++a) {
-    m->rt.bmin[a] = hb[a];
-    m->rt.bmax[a] = hb[3 + a] + 1;  // mBBox.max().offset(1)
+  const bool full = m->rt_full || m->ntiles > 0;
+  m->rt_full = true;  // until this build is through
+  const uint32_t first = full ? 0 : m->rt_leaves;
+  if (full) {
+    CK(launch_fill_u64(m->stream, m->rt.n128, m->rt_n128_cap, kEmpty));
+    CK(launch_fill_u64(m->stream, m->rt.n4096, m->rt_n4096_cap, kEmpty));
+    if (m->rt_node_cap) CK(launch_fill_u64(m->stream, m->rt.bits, (uint64_t)m->rt_node_cap * kRtNodeWords, 0));
+    m->rt_nodes = 0;
   }
+  CK(launch_snapshot_nodes(m->stream, map_view(m), first, m->leaf_count_ub, m->rt, m->rt_info, m->noop4096,
+                           vdbgpu_map::kNoopCap, m->rt_nodes, &m->d_st[1], full));
+  CK(hipMemcpyAsync(m->h_rt_info, m->rt_info, sizeof(RtInfo), hipMemcpyDeviceToHost, m->stream));
+  if ((r = read_status(m))) return r;
+  const RtInfo info = *m->h_rt_info;
+  if (info.nodes > m->rt_node_cap) {
+    const uint32_t cap = std::max<uint32_t>(256, (uint32_t)next_pow2(info.nodes));
+    unsigned long long* bits = nullptr;
+    CK(dalloc(m, &bits, (size_t)cap * kRtNodeWords));
+    CK(launch_fill_u64(m->stream, bits, (uint64_t)cap * kRtNodeWords, 0));
+    if (m->rt_nodes)
+      CK(hipMemcpyAsync(bits, m->rt.bits, (size_t)m->rt_nodes * kRtNodeWords * 8, hipMemcpyDeviceToDevice, m->stream));
+    CK(hipStreamSynchronize(m->stream));
+    dfree(m, &m->rt.bits, (size_t)m->rt_node_cap * kRtNodeWords);
+    m->rt.bits = bits;
+    m->rt_node_cap = cap;
+  }
+  CK(launch_snapshot_bits(m->stream, map_view(m), first, info.leaves, m->rt, m->rt_info, tile_view(m)));
+  for (int a = 0; a < 3; ++a) {
+    m->rt.bmin[a] = info.bbox[a];
+    m->rt.bmax[a] = info.bbox[3 + a] + 1;  // mBBox.max().offset(1)
+  }
+  m->rt_leaves = info.leaves;
+  m->rt_nodes = info.nodes;
+  m->rt_full = m->ntiles > 0;
   m->has_isect = true;
   m->snap_dirty = false;
   for (auto& kv : m->sources) kv.second.has_isect = true;  // every source gets a copy (VDBMapping.hpp:1441-1446)
@@ -2085,10 +2128,12 @@ void vdbgpu_destroy(vdbgpu_map* m) {
   dfree(m, &m->roff, m->ray_cap);
   dfree(m, &m->first_ray, m->chunk_cap);
   dfree(m, &m->tbl, (uint64_t)m->tbl_n * (m->tbl_n + 1) / 2);
-  dfree(m, &m->rt.leaf, m->rt_leaf_cap);
   dfree(m, &m->rt.n128, m->rt_n128_cap);
+  dfree(m, &m->rt.nidx, m->rt_n128_cap);
+  dfree(m, &m->rt.bits, (size_t)m->rt_node_cap * kRtNodeWords);
   dfree(m, &m->rt.n4096, m->rt_n4096_cap);
-  dfree(m, &m->d_bbox, 6);
+  dfree(m, &m->rt_info, 1);
+  if (m->h_rt_info) (void)hipHostFree(m->h_rt_info);
   dfree(m, &m->q_in, (size_t)m->q_cap * 7);
   dfree(m, &m->q_succ, (size_t)m->q_cap);
   dfree(m, &m->q_end, (size_t)m->q_cap * 3);
@@ -2572,9 +2617,8 @@ int32_t vdbgpu_raytrace(vdbgpu_map* m, int64_t n, const double* o, const double*
   CK(hipMemcpyAsync(m->q_in, o, (size_t)n * 24, hipMemcpyHostToDevice, m->stream));
   CK(hipMemcpyAsync(m->q_in + 3 * n, d, (size_t)n * 24, hipMemcpyHostToDevice, m->stream));
   CK(hipMemcpyAsync(m->q_in + 6 * n, len, (size_t)n * 8, hipMemcpyHostToDevice, m->stream));
-  const int grid = (int)std::min<int64_t>((int64_t)m->num_cu * 16, (n + 255) / 256);
   CK(hipMemsetAsync(&m->d_st[2].error, 0, sizeof(unsigned int), m->stream));
-  CK(launch_raytrace(m->stream, grid, m->rt, map_view(m), m->inv, m->res, n, m->q_in, m->q_in + 3 * n,
+  CK(launch_raytrace(m->stream, m->num_cu, rt_view(m), map_view(m), m->inv, m->res, n, m->q_in, m->q_in + 3 * n,
                      m->q_in + 6 * n, m->q_succ, m->q_end, &m->d_st[2].error));
   CK(hipMemcpyAsync(succ, m->q_succ, (size_t)n, hipMemcpyDeviceToHost, m->stream));
   CK(hipMemcpyAsync(ends, m->q_end, (size_t)n * 24, hipMemcpyDeviceToHost, m->stream));
@@ -2589,11 +2633,10 @@ int32_t vdbgpu_raytrace_device(vdbgpu_map* m, int64_t n, const double* o, const 
   if (!m->has_isect)
     return fail(m, VDBGPU_NO_INTERSECTOR, "raytrace needs an integrate in fast mode on a non-empty map");
   if (n == 0) return VDBGPU_OK;
-  const int grid = (int)std::min<int64_t>((int64_t)m->num_cu * 16, (n + 255) / 256);
   CK(hipMemsetAsync(&m->d_st[2].error, 0, sizeof(unsigned int), m->stream));
   {
     Timer t(m, kRaytrace);
-    CK(launch_raytrace(m->stream, grid, m->rt, map_view(m), m->inv, m->res, n, o, d, len, succ, ends,
+    CK(launch_raytrace(m->stream, m->num_cu, rt_view(m), map_view(m), m->inv, m->res, n, o, d, len, succ, ends,
                        &m->d_st[2].error));
   }
   return raytrace_status(m);
@@ -2673,8 +2716,7 @@ int32_t vdbgpu_raytrace_noalloc(vdbgpu_map* m, int64_t n, const double* o, const
   CK(hipMemcpyAsync(q_o, o, (size_t)n * 24, hipMemcpyHostToDevice, m->stream));
   CK(hipMemcpyAsync(q_d, d, (size_t)n * 24, hipMemcpyHostToDevice, m->stream));
   CK(hipMemcpyAsync(q_l, len, (size_t)n * 8, hipMemcpyHostToDevice, m->stream));
-  const int grid = (int)std::min<int64_t>((int64_t)m->num_cu * 16, (n + 255) / 256);
-  CK(launch_raytrace(m->stream, grid, m->rt, map_view(m), m->inv, m->res, n, q_o, q_d, q_l, q_s, q_e, err));
+  CK(launch_raytrace(m->stream, m->num_cu, rt_view(m), map_view(m), m->inv, m->res, n, q_o, q_d, q_l, q_s, q_e, err));
   unsigned int h_err = 0;
   CK(hipMemcpyAsync(succ, q_s, (size_t)n, hipMemcpyDeviceToHost, m->stream));
   CK(hipMemcpyAsync(ends, q_e, (size_t)n * 24, hipMemcpyDeviceToHost, m->stream));
@@ -2848,6 +2890,7 @@ int clear_grid(vdbgpu_map* m) {
   m->ledger.clear();
   m->ins_fifo.clear();
   free_tiles(m);
+  m->rt_full = true;
   m->touched = false;
   m->snap_dirty = true;
   m->art_leaves = false;
@@ -3323,6 +3366,7 @@ int32_t vdbgpu_apply_section_update(vdbgpu_map* m, const int32_t bbox[6], int64_
   int* d_box = nullptr;
   if ((r = upload(m, &d_box, bbox, 6))) return r;
   CK(launch_section_clear(m->stream, map_view(m), L, d_box, tile_view(m)));
+  m->snap_dirty = true;  // active states changed
   if (n) {
     const uint32_t N = (uint32_t)n;
     int* d_o = nullptr;

@@ -35,9 +35,10 @@ __device__ __forceinline__ uint32_t set_slot(unsigned long long* keys, uint32_t 
   return kNone;
 }
 
+// Slot of an update-set entry (upd_slot put it there).
 __device__ __forceinline__ uint32_t find_slot(const unsigned long long* __restrict__ keys,
                                               uint32_t mask, uint64_t key) {
-  uint32_t h = (uint32_t)fmix64(key) & mask;
+  uint32_t h = map_hash(key) & mask;
   for (uint32_t p = 0; p <= mask; ++p) {
     const unsigned long long k = keys[h];
     if (k == key) return h;

@@ -883,6 +883,69 @@ __global__ __launch_bounds__(256) void k_apply_groups(GroupScans gs, const uint3
   }
 }
 
+// The update set of a scan, as the brick path lists it (each leaf once), OR-ed
+// into a source's set: lane per record finds or opens its slot (an open slot's
+// masks are zero), then eight lanes per record OR its sixteen words, 16 bytes
+// each. A record's slot has one owner in a launch, so the words need no
+// atomics; words without a bit (most hit words) are neither read nor written.
+// The host has made room (the load stays under tuning.load_factor).
+__global__ __launch_bounds__(256) void k_merge_records(UpdView rec, uint32_t count, UpdView u,
+                                                       uint32_t* __restrict__ list, unsigned int* listed) {
+  __shared__ uint32_t s_wave[4], s_base, s_slot[256];
+  const uint32_t base = blockIdx.x * 256u;
+  const uint32_t e = base + threadIdx.x;
+  bool fresh = false;
+  uint32_t slot = kNone;
+  if (e < count) {
+    const uint64_t key = rec.keys[e];
+    uint32_t h = map_hash(key) & u.cap_mask;
+    for (uint32_t p = 0; p <= u.cap_mask; ++p) {
+      unsigned long long k = __hip_atomic_load(&u.keys[h], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (k == kEmpty) {
+        k = atomicCAS(&u.keys[h], kEmpty, (unsigned long long)key);
+        fresh = k == kEmpty;
+      }
+      if (fresh || k == key) {
+        slot = h;
+        break;
+      }
+      h = (h + 1) & u.cap_mask;
+    }
+  }
+  s_slot[threadIdx.x] = slot;
+  const uint32_t pos = block_append(fresh, listed, s_wave, &s_base);  // (its barriers cover s_slot)
+  if (fresh) list[pos] = slot;
+  const int l = (int)(threadIdx.x & 7), row = (int)(threadIdx.x >> 3);
+  const ulonglong2* __restrict__ src = reinterpret_cast<const ulonglong2*>(rec.masks);
+  ulonglong2* dst = reinterpret_cast<ulonglong2*>(u.masks);
+#pragma unroll
+  for (int r = 0; r < 8; ++r) {
+    const uint32_t i = (uint32_t)(r * 32 + row), to = s_slot[i];
+    if (to == kNone) continue;
+    const ulonglong2 v = src[(size_t)(base + i) * 8 + l];
+    if (!(v.x | v.y)) continue;
+    ulonglong2 w = dst[(size_t)to * 8 + l];
+    w.x |= v.x;
+    w.y |= v.y;
+    dst[(size_t)to * 8 + l] = w;
+  }
+}
+
+// The listed slots of an update set emptied: keys, and masks 16 bytes per lane.
+__global__ __launch_bounds__(256) void k_clear_listed(UpdView u, const uint32_t* __restrict__ list, uint32_t count) {
+  const uint64_t G = (uint64_t)gridDim.x * blockDim.x;
+  ulonglong2* m = reinterpret_cast<ulonglong2*>(u.masks);
+  for (uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; t < (uint64_t)count * 8; t += G) {
+    const uint32_t slot = list[t >> 3];
+    m[(size_t)slot * 8 + (t & 7)] = ulonglong2{0, 0};
+    if ((t & 7) == 0) u.keys[slot] = kEmpty;
+  }
+}
+
+__global__ void k_set_u32(unsigned int* p, uint32_t v) {
+  if (threadIdx.x == 0) *p = v;
+}
+
 // Move every entry of an update set into a larger one.
 __global__ __launch_bounds__(256) void k_rehash_update(UpdView from, uint32_t from_cap, UpdView to,
                                                        Status* st) {
@@ -1073,6 +1136,25 @@ hipError_t launch_apply_groups(hipStream_t s, int grid, const GroupScans& gs, co
                                const float lo[6], Status* st) {
   hipLaunchKernelGGL(k_apply_groups, dim3(grid), dim3(256), 0, s, gs, glist, grec, ngroups, gslot, mp, lo[0],
                      lo[1], lo[2], lo[3], lo[4], lo[5], st);
+  return hipGetLastError();
+}
+
+hipError_t launch_merge_records(hipStream_t s, UpdView rec, uint32_t count, UpdView u, uint32_t* list,
+                                unsigned int* listed) {
+  if (!count) return hipSuccess;
+  hipLaunchKernelGGL(k_merge_records, dim3((count + 255) / 256), dim3(256), 0, s, rec, count, u, list, listed);
+  return hipGetLastError();
+}
+
+hipError_t launch_clear_listed(hipStream_t s, UpdView u, const uint32_t* list, uint32_t count) {
+  if (!count) return hipSuccess;
+  const int grid = (int)std::min<uint64_t>(8192, ((uint64_t)count * 8 + 255) / 256);
+  hipLaunchKernelGGL(k_clear_listed, dim3(grid), dim3(256), 0, s, u, list, count);
+  return hipGetLastError();
+}
+
+hipError_t launch_set_u32(hipStream_t s, unsigned int* p, uint32_t v) {
+  hipLaunchKernelGGL(k_set_u32, dim3(1), dim3(64), 0, s, p, v);
   return hipGetLastError();
 }
 

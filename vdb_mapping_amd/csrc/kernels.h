@@ -42,6 +42,11 @@ hipError_t launch_zero_words(hipStream_t s, unsigned long long* p, uint32_t n);
 hipError_t launch_map_insert(hipStream_t s, UpdView u, const uint32_t* list, uint32_t count, MapView mp,
                              uint32_t* eidx, bool create_hit, bool create_miss,
                              unsigned long long* noop_set, uint32_t noop_mask, Status* st);
+// Records (one per leaf) OR-ed into an update set with room for them; the slots they open are appended to list.
+hipError_t launch_merge_records(hipStream_t s, UpdView rec, uint32_t count, UpdView u, uint32_t* list,
+                                unsigned int* listed);
+hipError_t launch_clear_listed(hipStream_t s, UpdView u, const uint32_t* list, uint32_t count);
+hipError_t launch_set_u32(hipStream_t s, unsigned int* p, uint32_t v);
 hipError_t launch_rec_gather(hipStream_t s, int grid, const uint32_t* list, UpdView sparse, const RecDest* dest,
                              const Status* st);
 hipError_t launch_put_dest(hipStream_t s, RecDest* dst, RecDest v);

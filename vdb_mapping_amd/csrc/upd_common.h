@@ -30,7 +30,7 @@ __device__ __forceinline__ int world_to_index1(double c, double res, double inv)
 // is exact because the update set is an OR of idempotent marks).
 constexpr uint32_t kMaxProbe = 512;
 __device__ __forceinline__ uint32_t upd_slot(const UpdView& u, uint64_t key, unsigned int* ovf) {
-  uint32_t h = (uint32_t)fmix64(key) & u.cap_mask;
+  uint32_t h = map_hash(key) & u.cap_mask;
   const uint32_t limit = u.cap_mask < kMaxProbe ? u.cap_mask + 1 : kMaxProbe;
   for (uint32_t probe = 0; probe < limit; ++probe) {
     const unsigned long long k =

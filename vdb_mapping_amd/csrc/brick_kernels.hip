@@ -814,6 +814,11 @@ hipError_t launch_rec_list(hipStream_t s, const unsigned long long* leaf_mask, u
   return hipGetLastError();
 }
 
+hipError_t launch_scan_u64(hipStream_t s, const uint64_t* in, uint64_t* out, uint32_t n, unsigned int* total) {
+  hipLaunchKernelGGL(k_scan_u64, dim3(1), dim3(256), 0, s, in, out, n, total, 0, (unsigned int*)nullptr);
+  return hipGetLastError();
+}
+
 hipError_t launch_split_emit(hipStream_t s, int grid, const uint32_t* split_slot,
                              unsigned long long* shared_bits, BrickView bv, UpdView rec,
                              unsigned long long* leaf_mask, uint32_t rec_cap, Status* st) {

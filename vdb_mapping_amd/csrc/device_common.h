@@ -175,6 +175,16 @@ struct RtView {
   uint32_t live;              // 1: the map changed since, active states are read from it alone
   int bmin[3], bmax[3];
 };
+// A map section by the leaf cells of its index box (edit_kernels.hip): cell
+// (x, y, z) of dims is the leaf at (lo + (x, y, z)) * 8, numbered x-major, the
+// order of sorted origins; box is the inclusive voxel box.
+struct SectionBox {
+  int lo[3];
+  uint32_t dims[3];
+  int box[6];
+};
+constexpr uint32_t kSectionCells = 16;  // cells per workgroup
+
 constexpr uint32_t kRtNodeWords = 128;  // words of RtView::bits per node
 // What a snapshot build hands back: bbox (min, max) of leaves with an active
 // voxel, nodes in the hash, leaves covered.

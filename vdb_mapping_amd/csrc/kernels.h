@@ -112,6 +112,14 @@ hipError_t launch_snapshot_nodes(hipStream_t s, MapView mp, uint32_t first, uint
                                  uint32_t old_nodes, const Status* stmap, bool full);
 hipError_t launch_snapshot_bits(hipStream_t s, MapView mp, uint32_t first, uint32_t leaf_count, RtView rt,
                                 const RtInfo* info, TileView tv);
+// Map section by the cells of its box: cell[c] = pool index of the section leaf or kNone, their count to *total
+// (edit_kernels.hip); then the leaves, in cell order, up to cap of them.
+hipError_t launch_section_cells(hipStream_t s, MapView mp, const SectionBox& sb, uint32_t cells, bool full,
+                                uint32_t* cell, uint64_t* bsum, uint64_t* boff, unsigned int* total, TileView tv);
+hipError_t launch_section_rows(hipStream_t s, MapView mp, const SectionBox& sb, uint32_t cells, bool full,
+                               const uint32_t* cell, const uint64_t* boff, uint32_t cap, int* origins, float* values,
+                               unsigned long long* masks);
+hipError_t launch_scan_u64(hipStream_t s, const uint64_t* in, uint64_t* out, uint32_t n, unsigned int* total);
 hipError_t launch_raytrace(hipStream_t s, int num_cu, RtView rt, MapView mp, double inv, double res,
                            int64_t n, const double* origins, const double* dirs,
                            const double* lens, uint8_t* success, double* ends, unsigned int* err);

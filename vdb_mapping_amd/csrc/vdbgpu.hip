@@ -243,6 +243,14 @@ struct vdbgpu_map {
   uint32_t group_cap = 0;      // groups: work items + split bricks
   double* tbl = nullptr;
   uint32_t tbl_n = 0;
+  // map sections by cells: cell table and its block sums, and the pinned
+  // staging buffer that the section's leaves are written to
+  uint32_t* sec_cell = nullptr;
+  uint64_t* sec_sums = nullptr;  // sums, then their scan
+  uint32_t sec_cells = 0;
+  char* h_sec = nullptr;
+  uint32_t sec_cap = 0;  // leaves the staging buffer holds
+  bool sec_again = false;  // a section was read before
 
   // direct edits (addPointsToGrid / removePointsFromGrid) and artificial areas
   Source edit;                 // marked voxels of one edit call (cleared after it)
@@ -2091,6 +2099,8 @@ uint64_t walk_scratch(vdbgpu_map* m, bool release) {
   one(m->gneed, m->gcap);
   one(m->glist, m->gcap);
   one(m->gidx, m->gcap);
+  one(m->sec_cell, m->sec_cells);
+  one(m->sec_sums, (size_t)m->sec_cells / kSectionCells * 2);
   one(m->q_in, (size_t)m->q_cap * 7);
   one(m->q_succ, (size_t)m->q_cap);
   one(m->q_end, (size_t)m->q_cap * 3);
@@ -2104,6 +2114,9 @@ uint64_t walk_scratch(vdbgpu_map* m, bool release) {
   for (auto& kv : m->sources) upd(kv.second);
   upd(m->edit);
   if (release) {
+    if (m->h_sec) (void)hipHostFree(m->h_sec);
+    m->h_sec = nullptr;
+    m->sec_cells = m->sec_cap = 0;
     m->points_bytes = 0;
     m->ray_cap = 0;
     m->chunk_cap = 0;
@@ -2310,6 +2323,9 @@ void vdbgpu_destroy(vdbgpu_map* m) {
   dfree(m, &m->q_in, (size_t)m->q_cap * 7);
   dfree(m, &m->q_succ, (size_t)m->q_cap);
   dfree(m, &m->q_end, (size_t)m->q_cap * 3);
+  dfree(m, &m->sec_cell, m->sec_cells);
+  dfree(m, &m->sec_sums, (size_t)m->sec_cells / kSectionCells * 2);
+  if (m->h_sec) (void)hipHostFree(m->h_sec);
   if (m->noop4096) (void)hipFree(m->noop4096);
   if (m->d_scans) (void)hipFree(m->d_scans);
   if (m->d_ctl) (void)hipFree(m->d_ctl);
@@ -3408,11 +3424,113 @@ int64_t vdbgpu_export_artificial(vdbgpu_map* m, int32_t* origins, uint64_t* mask
 
 // ---------------------------------------------------------- map sections --
 
+}  // extern "C"
+
+namespace {
+
+// Boxes of more leaf cells than this scan the pool instead (and are sorted on
+// the host); the staging buffer stays below 280 MB.
+constexpr uint64_t kMaxSectionCells = 1u << 17;
+
+// The box's leaf cells, clipped to the leaf key range; their number in *cells.
+SectionBox section_box(const int32_t bbox[6], uint64_t* cells) {
+  SectionBox sb{};
+  *cells = 1;
+  for (int a = 0; a < 3; ++a) {
+    sb.box[a] = bbox[a];
+    sb.box[3 + a] = bbox[3 + a];
+    const int64_t lo = std::max<int64_t>(bbox[a], -kCoordLimit) >> 3;
+    const int64_t hi = std::min<int64_t>(bbox[3 + a], kCoordLimit - 1) >> 3;
+    sb.lo[a] = (int)lo;
+    sb.dims[a] = hi < lo || bbox[3 + a] < bbox[a] ? 0u : (uint32_t)(hi - lo + 1);
+    // (at most 2^21 per axis; capped so that the product cannot wrap)
+    *cells = std::min<uint64_t>(*cells * sb.dims[a], 1ull << 40);
+  }
+  return sb;
+}
+
+// Section of at most kMaxSectionCells cells. A map's first section is gathered
+// in device memory and copied. From the second on (a program that reads one
+// after every scan) the leaves are written straight into a pinned staging
+// buffer, guessed to hold them as it held the last section; when it does not,
+// it grows and they are written again. Pinning it costs about a millisecond,
+// which a single read would not win back.
+int64_t export_section_cells(vdbgpu_map* m, const SectionBox& sb, uint32_t cells, bool full, int32_t* origins,
+                             float* values, uint64_t* masks, int64_t cap) {
+  const uint32_t want = (cells + 255) / 256 * 256;
+  if (want > m->sec_cells) {
+    dfree(m, &m->sec_cell, m->sec_cells);
+    dfree(m, &m->sec_sums, (size_t)m->sec_cells / kSectionCells * 2);
+    m->sec_cells = 0;
+    CKN(dalloc(m, &m->sec_cell, want));
+    CKN(dalloc(m, &m->sec_sums, (size_t)want / kSectionCells * 2));
+    m->sec_cells = want;
+  }
+  uint64_t* boff = m->sec_sums + m->sec_cells / kSectionCells;
+  CKN(launch_section_cells(m->stream, map_view(m), sb, cells, full, m->sec_cell, m->sec_sums, boff,
+                           &m->d_st[2].entries, tile_view(m)));
+  const bool out = origins || values || masks;
+  auto rows = [&]() -> hipError_t {
+    char* p = nullptr;
+    const hipError_t e = hipHostGetDevicePointer((void**)&p, m->h_sec, 0);
+    if (e != hipSuccess) return e;
+    return launch_section_rows(m->stream, map_view(m), sb, cells, full, m->sec_cell, boff, m->sec_cap,
+                               (int*)(p + (size_t)m->sec_cap * 2112), values ? (float*)p : nullptr,
+                               (unsigned long long*)(p + (size_t)m->sec_cap * 2048));
+  };
+  if (out && m->sec_cap) CKN(rows());
+  if (read_status(m)) return -1;
+  const uint32_t n = m->h_st[2].entries;
+  if (!out) return n;
+  if ((int64_t)n > cap) return -(int64_t)n;
+  if (n == 0) return 0;
+  if (!m->sec_again) {
+    m->sec_again = true;
+    char* d = nullptr;
+    CKN(dalloc(m, &d, (size_t)n * 2124));
+    int* d_o = (int*)(d + (size_t)n * 2112);
+    unsigned long long* d_a = (unsigned long long*)(d + (size_t)n * 2048);
+    const hipError_t e = [&]() -> hipError_t {
+      hipError_t e = launch_section_rows(m->stream, map_view(m), sb, cells, full, m->sec_cell, boff, n, d_o,
+                                         values ? (float*)d : nullptr, d_a);
+      if (!e && values) e = hipMemcpyAsync(values, d, (size_t)n * 2048, hipMemcpyDeviceToHost, m->stream);
+      if (!e && masks) e = hipMemcpyAsync(masks, d_a, (size_t)n * 64, hipMemcpyDeviceToHost, m->stream);
+      if (!e && origins) e = hipMemcpyAsync(origins, d_o, (size_t)n * 12, hipMemcpyDeviceToHost, m->stream);
+      return e ? e : hipStreamSynchronize(m->stream);
+    }();
+    dfree(m, &d, (size_t)n * 2124);
+    CKN(e);
+    return n;
+  }
+  if (n > m->sec_cap) {
+    if (m->h_sec) (void)hipHostFree(m->h_sec);
+    m->h_sec = nullptr;
+    m->sec_cap = 0;
+    const uint32_t room = std::min(cells, std::max<uint32_t>(256, n + n / 4));
+    CKN(hipHostMalloc((void**)&m->h_sec, (size_t)room * 2124, hipHostMallocDefault));
+    m->sec_cap = room;
+    CKN(rows());
+    CKN(hipStreamSynchronize(m->stream));
+  }
+  if (values) std::memcpy(values, m->h_sec, (size_t)n * 2048);
+  if (masks) std::memcpy(masks, m->h_sec + (size_t)m->sec_cap * 2048, (size_t)n * 64);
+  if (origins) std::memcpy(origins, m->h_sec + (size_t)m->sec_cap * 2112, (size_t)n * 12);
+  return n;
+}
+
+}  // namespace
+
+extern "C" {
+
 int64_t vdbgpu_export_section(vdbgpu_map* m, const int32_t bbox[6], int32_t full_grid, int32_t* origins,
                               float* values, uint64_t* masks, int64_t cap) {
   if (!m || !bbox) return -1;
   Guard g(m);
   if (g.rc) return -1;
+  uint64_t cells = 0;
+  const SectionBox sb = section_box(bbox, &cells);
+  if (cells > 0 && cells <= kMaxSectionCells && m->mcap)
+    return export_section_cells(m, sb, (uint32_t)cells, full_grid != 0, origins, values, masks, cap);
   CKN(hipStreamSynchronize(m->cast));
   if (read_status(m)) return -1;
   const uint32_t L = m->h_st[1].leaf_count;

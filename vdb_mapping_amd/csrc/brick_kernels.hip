@@ -5,9 +5,12 @@
 // workgroup owns a brick's visited/hit bitmap (8 KiB of LDS) while it walks
 // that brick's segments. The result is the scan's update set as a list of
 // leaf records (key + 8 visited + 8 hit mask words), every update leaf
-// exactly once, written with plain stores at fixed positions (no shared
-// counters); k_map_insert and k_apply take the dense list of filled
-// positions built from the per-item leaf masks. No global atomics touch voxel bits except for the few
+// exactly once, written with plain stores into the scan's record set (a brick
+// takes its run of records with one atomic on one of 16 counters), which the
+// map stream reads, possibly several scans later. (Records at 64 fixed
+// positions per work item, listed and copied densely afterwards, needed no
+// counters but four launches and a copy: 105 us of an outdoor scan's cast.)
+// No global atomics touch voxel bits except for the few
 // bricks so crowded (more than kItemSegs segments, around the sensor) that
 // several workgroups share them.
 //
@@ -21,15 +24,11 @@
 //                   table, enumerate again, write each segment record at its
 //                   brick's next position
 //   k_brick_walk    one workgroup per work item: walk the item's segments
-//                   into the LDS bitmap, write the brick's leaf records at
-//                   the item's 64 fixed positions, or OR into the shared
-//                   bitmap of a split brick
-//   k_split_emit    leaf records of split bricks (positions after the items)
-//   k_mask_sums, k_mask_list  dense list of the filled record positions from
-//                   the per-item leaf masks (scan, no shared counters)
-//   k_rec_gather    the listed records copied densely into the scan's record
-//                   set, named in device memory (read by the map stream,
-//                   possibly several scans later)
+//                   into the LDS bitmap, append the brick's leaf records to
+//                   the scan's record set (named in device memory), or OR
+//                   into the shared bitmap of a split brick
+//   k_split_emit    leaf records of split bricks
+//   k_rec_total     record counts of the regions, overflow
 //
 // Segment record (uint4), self-contained so the walk loads nothing else:
 //   x = n0 | n1 << 14, y = n2 | c0 << 14, z = c1 | c2 << 14  (|delta| per axis
@@ -141,21 +140,35 @@ __device__ __forceinline__ uint64_t block_sum_u64(uint64_t v, uint64_t* s_w) {
   return t;
 }
 
-// Leaf records of the brick bitmap `bits` (brick origin o) at the fixed
-// positions base .. base + 63 (leaf l of the brick at base + l), for every
-// leaf with a visited voxel; *leaf_mask gets the set of filled positions
-// (bit l). Called by the whole workgroup.
-__device__ void emit_leaves(const unsigned long long* bits, int ox, int oy, int oz, UpdView rec,
-                            uint32_t base, uint32_t* s_pos, unsigned long long* leaf_mask) {
+// Regions in use for a scan of n_items work items: enough counters that the
+// appends of tens of thousands of bricks do not queue on one (a single one made
+// the walk 0.75 -> 1.27 ms), one for small scans, whose few bricks would fill
+// many regions unevenly.
+__device__ __forceinline__ uint32_t rec_regions(uint32_t n_items) {
+  return n_items >= kRecRegionItems ? kRecRegions : 1u;
+}
+
+// Leaf records of the brick bitmap `bits` (brick origin o), appended to region
+// `reg` of the record set: one atomic per brick on the region's counter, every
+// leaf with a visited voxel a record (key, 8 visited and 8 hit words) after the
+// next. A brick that does not fit is counted but not written (k_rec_total
+// flags it). Called by the whole workgroup.
+__device__ void emit_leaves(const unsigned long long* bits, int ox, int oy, int oz, const RecDest& d, uint32_t reg,
+                            uint32_t stride, unsigned int* rcnt, uint32_t* s_pos) {
   const int tid = threadIdx.x;
   if (tid < 64) {  // lane l = leaf l of the brick
     uint64_t any = 0;
 #pragma unroll
     for (int j = 0; j < 8; ++j) any |= bits[tid * 8 + j];
     const uint64_t m = __ballot(any != 0);
-    if (tid == 0) *leaf_mask = m;
-    s_pos[tid] = any ? base + tid : kNone;
-    if (any) rec.keys[base + tid] = leaf_key(ox + (tid >> 4) * 8, oy + ((tid >> 2) & 3) * 8, oz + (tid & 3) * 8);
+    const uint32_t n = (uint32_t)__popcll(m);
+    uint32_t base = 0;
+    if (tid == 0 && n) base = atomicAdd(&rcnt[reg * kRecCountStride], n);
+    base = __shfl(base, 0, 64);
+    const bool ok = any != 0 && base + n <= stride;
+    const uint32_t pos = reg * stride + base + (uint32_t)__popcll(m & ((1ull << tid) - 1));
+    s_pos[tid] = ok ? pos : kNone;
+    if (ok) d.keys[pos] = leaf_key(ox + (tid >> 4) * 8, oy + ((tid >> 2) & 3) * 8, oz + (tid & 3) * 8);
   }
   __syncthreads();
   // 16 records x 16 words per pass: contiguous 128-byte rows
@@ -163,7 +176,7 @@ __device__ void emit_leaves(const unsigned long long* bits, int ox, int oy, int 
   for (int p = 0; p < 4; ++p) {
     const int l = p * 16 + (tid >> 4), w = tid & 15;
     const uint32_t pos = s_pos[l];
-    if (pos != kNone) rec.masks[(size_t)pos * 16 + w] = bits[(w < 8 ? 0 : 512) + l * 8 + (w & 7)];
+    if (pos != kNone) d.masks[(size_t)pos * 16 + w] = bits[(w < 8 ? 0 : 512) + l * 8 + (w & 7)];
   }
 }
 
@@ -519,8 +532,8 @@ __global__ __launch_bounds__(kWalkThreads, 8) void k_brick_walk(const BrickItem*
                                                              const ScanInfo* __restrict__ scans,
                                                              const double* __restrict__ tbl, BrickView bv,
                                                              unsigned long long* __restrict__ shared_bits,
-                                                             UpdView rec, unsigned long long* __restrict__ leaf_mask,
-                                                             uint32_t rec_cap, Status* st) {
+                                                             const RecDest* __restrict__ dest,
+                                                             unsigned int* __restrict__ rcnt, Status* st) {
   __shared__ unsigned long long bits[kWalkWords];
   __shared__ uint32_t s_pos[64];
   __shared__ uint32_t s_hist[128];
@@ -529,10 +542,8 @@ __global__ __launch_bounds__(kWalkThreads, 8) void k_brick_walk(const BrickItem*
   __shared__ uint32_t s_used;
   if (stopped(st, &s_stop)) return;
   const uint32_t n_items = st->items;
-  if ((uint64_t)n_items * 64 > rec_cap) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) atomicOr(&st->overflow, kOvfRecords);
-    return;
-  }
+  const RecDest d = *dest;
+  const uint32_t regions = rec_regions(n_items), stride = d.cap / regions;
   const uint32_t t = threadIdx.x;
   // static assignment: item it -> workgroup it % grid (no shared queue counter)
   for (uint32_t it = blockIdx.x; it < n_items; it += gridDim.x) {
@@ -598,14 +609,13 @@ __global__ __launch_bounds__(kWalkThreads, 8) void k_brick_walk(const BrickItem*
     __syncthreads();
     merge_layouts(bits, s_used);
     if (item.shared == kNone) {
-      emit_leaves(bits, ox, oy, oz, rec, it * 64, s_pos, &leaf_mask[it]);
+      emit_leaves(bits, ox, oy, oz, d, it & (regions - 1), stride, rcnt, s_pos);
     } else {
       unsigned long long* dst = shared_bits + (size_t)item.shared * kBrickWords;
       for (int w = t; w < kBrickWords; w += kWalkThreads) {
         const uint64_t v = bits[w];
         if (v) atomicOr(&dst[w], (unsigned long long)v);
       }
-      if (t == 0) leaf_mask[it] = 0;  // its records come from k_split_emit
     }
     __syncthreads();
   }
@@ -613,18 +623,15 @@ __global__ __launch_bounds__(kWalkThreads, 8) void k_brick_walk(const BrickItem*
 
 __global__ __launch_bounds__(256) void k_split_emit(const uint32_t* __restrict__ split_slot,
                                                     unsigned long long* __restrict__ shared_bits,
-                                                    BrickView bv, UpdView rec,
-                                                    unsigned long long* __restrict__ leaf_mask,
-                                                    uint32_t rec_cap, Status* st) {
+                                                    BrickView bv, const RecDest* __restrict__ dest,
+                                                    unsigned int* __restrict__ rcnt, Status* st) {
   __shared__ unsigned long long bits[kBrickWords];
   __shared__ uint32_t s_pos[64];
   __shared__ unsigned int s_stop;
   if (stopped(st, &s_stop)) return;
-  const uint32_t ns = st->splits, n_items = st->items;
-  if ((uint64_t)(n_items + ns) * 64 > rec_cap) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) atomicOr(&st->overflow, kOvfRecords);
-    return;
-  }
+  const uint32_t ns = st->splits;
+  const RecDest d = *dest;
+  const uint32_t regions = rec_regions(st->items), stride = d.cap / regions;
   for (uint32_t k = blockIdx.x; k < ns; k += gridDim.x) {
     unsigned long long* src = shared_bits + (size_t)k * kBrickWords;
     for (int w = threadIdx.x; w < kBrickWords; w += blockDim.x) {
@@ -634,96 +641,33 @@ __global__ __launch_bounds__(256) void k_split_emit(const uint32_t* __restrict__
     __syncthreads();
     int b[3];
     brick_coords(bv.keys[split_slot[k]], b);
-    emit_leaves(bits, b[0] * kBrickDim, b[1] * kBrickDim, b[2] * kBrickDim, rec, (n_items + k) * 64, s_pos,
-                &leaf_mask[n_items + k]);
+    emit_leaves(bits, b[0] * kBrickDim, b[1] * kBrickDim, b[2] * kBrickDim, d, k & (regions - 1), stride, rcnt,
+                s_pos);
     __syncthreads();
   }
 }
 
-// Record list from the per-group (64 positions) leaf masks: per 256 groups
-// the number of filled positions, then after the scan of those sums every
-// group writes its positions in order. No shared counters.
-__global__ __launch_bounds__(256) void k_mask_sums(const unsigned long long* __restrict__ leaf_mask,
-                                                   uint64_t* __restrict__ bsum, const Status* st) {
-  __shared__ uint64_t s_w[4];
-  __shared__ unsigned int s_stop;
-  if (stopped(st, &s_stop)) return;
-  const uint32_t ng = st->items + st->splits;
-  const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
-  const uint64_t c = g < ng ? (uint64_t)__popcll(leaf_mask[g]) : 0;
-  const uint64_t t = block_sum_u64(c, s_w);
-  if (threadIdx.x == 0) bsum[blockIdx.x] = t;
-}
-
-__global__ __launch_bounds__(256) void k_mask_list(const unsigned long long* __restrict__ leaf_mask,
-                                                   const uint64_t* __restrict__ boff,
-                                                   uint32_t* __restrict__ list, const Status* st) {
-  __shared__ uint64_t s_w[4];
-  __shared__ unsigned int s_stop;
-  if (stopped(st, &s_stop)) return;
-  const uint32_t ng = st->items + st->splits;
-  const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
-  const uint64_t m = g < ng ? leaf_mask[g] : 0;
-  const uint64_t x = (uint64_t)__popcll(m);
-  uint64_t v = x;
+// The scan's record counts (one wave): total, prefix over the regions, and the
+// overflow flag when a region did not hold its records.
+__global__ void k_rec_total(const RecDest* dest, const unsigned int* rcnt, Status* st) {
+  const uint32_t l = threadIdx.x;
+  if (st->error | st->overflow) return;
+  const uint32_t stride = dest->cap / rec_regions(st->items);
+  const uint32_t c = l < kRecRegions ? rcnt[l * kRecCountStride] : 0u;
+  uint32_t v = c, most = c;
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
-    const uint64_t t = __shfl_up(v, o, 64);
-    if (bw_lane() >= o) v += t;
+    const uint32_t t = __shfl_up(v, o, 64);
+    if ((int)l >= o) v += t;
+    most = max(most, __shfl_xor(most, o, 64));
   }
-  const int wv = threadIdx.x >> 6;
-  if (bw_lane() == 63) s_w[wv] = v;
-  __syncthreads();
-  uint64_t add = 0;
-  for (int w = 0; w < wv; ++w) add += s_w[w];
-  uint32_t pos = (uint32_t)(boff[blockIdx.x] + add + v - x);
-  for (uint64_t r = m; r; r &= r - 1) list[pos++] = g * 64 + (uint32_t)__builtin_ctzll(r);
-}
-
-// Dense copy of the listed records (key and 16 mask words each, sixteen lanes
-// per record) into the record set the map stream reads; the positional set is
-// then free for the next scan's walk. Copies nothing when the count exceeds
-// dcap (the host grows the set and runs it again).
-__global__ __launch_bounds__(256) void k_rec_gather(const uint32_t* __restrict__ list, UpdView sparse,
-                                                    const RecDest* __restrict__ dest, const Status* st) {
-  if (st->error | st->overflow) return;
-  const uint32_t n = st->records;
-  const RecDest d = *dest;
-  if (n > d.cap) return;
-  const UpdView dense{d.keys, d.masks, 0};
-  // eight lanes per record, 16 bytes each (the 128 mask bytes); each lane
-  // group keeps kGatherRecs records in flight (list, then record loads, then
-  // stores, issued together)
-  constexpr int kGatherRecs = 4;
-  const int l = (int)(threadIdx.x & 7);
-  const uint64_t G = ((uint64_t)gridDim.x * blockDim.x) >> 3;
-  const uint4* __restrict__ src = reinterpret_cast<const uint4*>(sparse.masks);
-  uint4* __restrict__ dst = reinterpret_cast<uint4*>(dense.masks);
-  for (uint64_t i0 = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 3; i0 < n; i0 += kGatherRecs * G) {
-    uint32_t pos[kGatherRecs];
-#pragma unroll
-    for (int r = 0; r < kGatherRecs; ++r) pos[r] = i0 + r * G < n ? list[i0 + r * G] : kNone;
-    uint4 v[kGatherRecs];
-    unsigned long long key[kGatherRecs];
-#pragma unroll
-    for (int r = 0; r < kGatherRecs; ++r) {
-      if (pos[r] == kNone) continue;
-      v[r] = src[(size_t)pos[r] * 8 + l];
-      if (l == 0) key[r] = sparse.keys[pos[r]];
-    }
-#pragma unroll
-    for (int r = 0; r < kGatherRecs; ++r) {
-      if (pos[r] == kNone) continue;
-      const uint64_t i = i0 + r * G;
-      dst[i * 8 + l] = v[r];
-      if (l == 0) dense.keys[i] = key[r];
-    }
+  if (l < kRecRegions) st->rec_pre[l] = v - c;
+  if (l == 63) {
+    st->records = v;
+    st->rec_stride = stride;
+    st->rec_most = most;
+    if (most > stride) atomicOr(&st->overflow, kOvfRecords);
   }
-}
-
-// The record set of the next cast (one lane).
-__global__ void k_put_dest(RecDest* dst, RecDest v) {
-  if (threadIdx.x == 0) *dst = v;
 }
 
 // The map's leaf count into host-visible memory (one lane; no copy engine).
@@ -731,32 +675,15 @@ __global__ void k_snap_count(const Status* st, uint32_t* host_dst) {
   if (threadIdx.x == 0) __hip_atomic_store(host_dst, st->leaf_count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-__global__ __launch_bounds__(256) void k_iota_u32(uint32_t* p, uint32_t n) {
-  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-  if (i < n) p[i] = i;
-}
-
 // ---------------------------------------------------------------- launchers --
 
-hipError_t launch_rec_gather(hipStream_t s, int grid, const uint32_t* list, UpdView sparse, const RecDest* dest,
-                             const Status* st) {
-  hipLaunchKernelGGL(k_rec_gather, dim3(grid), dim3(256), 0, s, list, sparse, dest, st);
-  return hipGetLastError();
-}
-
-hipError_t launch_put_dest(hipStream_t s, RecDest* dst, RecDest v) {
-  hipLaunchKernelGGL(k_put_dest, dim3(1), dim3(64), 0, s, dst, v);
+hipError_t launch_rec_total(hipStream_t s, const RecDest* dest, const unsigned int* rcnt, Status* st) {
+  hipLaunchKernelGGL(k_rec_total, dim3(1), dim3(64), 0, s, dest, rcnt, st);
   return hipGetLastError();
 }
 
 hipError_t launch_snap_count(hipStream_t s, const Status* st, uint32_t* host_dst) {
   hipLaunchKernelGGL(k_snap_count, dim3(1), dim3(64), 0, s, st, host_dst);
-  return hipGetLastError();
-}
-
-hipError_t launch_iota_u32(hipStream_t s, uint32_t* p, uint32_t n) {
-  if (!n) return hipSuccess;
-  hipLaunchKernelGGL(k_iota_u32, dim3((n + 255) / 256), dim3(256), 0, s, p, n);
   return hipGetLastError();
 }
 
@@ -793,24 +720,10 @@ hipError_t launch_seg_fill(hipStream_t s, int grid, const int4* rayinfo, const S
 
 hipError_t launch_brick_walk(hipStream_t s, int grid, const BrickItem* items, const uint4* segs,
                              const int4* rayinfo, const ScanInfo* scans, const double* tbl,
-                             BrickView bv, unsigned long long* shared_bits, UpdView rec,
-                             unsigned long long* leaf_mask, uint32_t rec_cap, Status* st) {
+                             BrickView bv, unsigned long long* shared_bits, const RecDest* dest,
+                             unsigned int* rcnt, Status* st) {
   hipLaunchKernelGGL(k_brick_walk, dim3(grid), dim3(kWalkThreads), 0, s, items, segs, rayinfo, scans, tbl, bv,
-                     shared_bits, rec, leaf_mask, rec_cap, st);
-  return hipGetLastError();
-}
-
-// nb_cap: 256-group blocks the bsum/boff arrays hold (>= (items + splits) / 256).
-hipError_t launch_rec_list(hipStream_t s, const unsigned long long* leaf_mask, uint64_t* bsum, uint64_t* boff,
-                           uint32_t nb_cap, uint32_t* list, Status* st) {
-  hipLaunchKernelGGL(k_mask_sums, dim3(nb_cap), dim3(256), 0, s, leaf_mask, bsum, st);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_scan_u64, dim3(1), dim3(256), 0, s, bsum, boff, nb_cap, &st->records, 0,
-                     (unsigned int*)nullptr);
-  e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_mask_list, dim3(nb_cap), dim3(256), 0, s, leaf_mask, boff, list, st);
+                     shared_bits, dest, rcnt, st);
   return hipGetLastError();
 }
 
@@ -820,10 +733,9 @@ hipError_t launch_scan_u64(hipStream_t s, const uint64_t* in, uint64_t* out, uin
 }
 
 hipError_t launch_split_emit(hipStream_t s, int grid, const uint32_t* split_slot,
-                             unsigned long long* shared_bits, BrickView bv, UpdView rec,
-                             unsigned long long* leaf_mask, uint32_t rec_cap, Status* st) {
-  hipLaunchKernelGGL(k_split_emit, dim3(grid), dim3(256), 0, s, split_slot, shared_bits, bv, rec,
-                     leaf_mask, rec_cap, st);
+                             unsigned long long* shared_bits, BrickView bv, const RecDest* dest,
+                             unsigned int* rcnt, Status* st) {
+  hipLaunchKernelGGL(k_split_emit, dim3(grid), dim3(256), 0, s, split_slot, shared_bits, bv, dest, rcnt, st);
   return hipGetLastError();
 }
 

@@ -59,6 +59,12 @@ constexpr int kEditFree = 1;      // setNodeToFree: (min log-odds, off)
 constexpr int kEditState = 2;     // setNodeState: on = value > t_max
 constexpr int kEditActivate = 3;  // setActiveState(on)
 
+// A scan's update-leaf records lie in up to kRecRegions equal regions of its
+// record set, each filled from its start (see emit_leaves).
+constexpr uint32_t kRecRegions = 16;
+constexpr uint32_t kRecRegionItems = 4096;  // work items from which all regions are used
+constexpr uint32_t kRecCountStride = 32;    // words between the regions' counters (a line each)
+
 struct Status {
   unsigned long long total;     // visits of the scan (sum of counts)
   unsigned long long voxels;    // visited voxels in the update set (compact)
@@ -72,9 +78,25 @@ struct Status {
   unsigned int segs;            // brick segments of the scan (brick path)
   unsigned int items;           // brick work items
   unsigned int splits;          // bricks shared by several work items
-  unsigned int records;         // update-leaf records listed by the brick path
-  unsigned int reserved;
+  unsigned int records;         // update-leaf records of the scan (brick path)
+  unsigned int rec_stride;      // records per region of its record set
+  unsigned int rec_most;        // records of the fullest region
+  unsigned int rec_pre[kRecRegions];  // records of the regions before each
   unsigned int pad;
+};
+
+// Record e of a scan (in region order) lies at at(e) of its record set.
+struct RecIndex {
+  uint32_t pre[kRecRegions];
+  uint32_t stride;
+  __host__ __device__ __forceinline__ uint32_t at(uint32_t e) const {
+    uint32_t d = 0;
+#if defined(__HIPCC__)
+#pragma unroll
+#endif
+    for (uint32_t r = 1; r < kRecRegions; ++r) d = e >= pre[r] ? r * stride - pre[r] : d;
+    return e + d;
+  }
 };
 
 // One scan of a batch: sensor origin, max range, its rays [ray0, ray0 + nrays)
@@ -101,9 +123,9 @@ struct UpdView {
   uint32_t cap_mask;
 };
 
-// Where the brick path copies a scan's records (one record set of the ring):
-// kept in device memory, so a replayed cast graph copies into the set of the
-// scan it runs for.
+// Where the brick path puts a scan's records (one record set of the ring):
+// kept in device memory, so a replayed cast graph fills the set of the scan it
+// runs for.
 struct RecDest {
   unsigned long long* keys;
   unsigned long long* masks;  // 16 words per record

@@ -503,7 +503,7 @@ __global__ __launch_bounds__(256) void k_compact(UpdView u, uint32_t cap,
 // outdoor scan's 1.7 M records take 44 us instead of 86. One record per lane:
 // two or four per lane left fewer waves to hide the probes (47 and 59 us).
 __global__ __launch_bounds__(kListBlockMax) void k_map_insert(UpdView u, const uint32_t* __restrict__ list,
-                                                              uint32_t count, MapView mp,
+                                                              RecIndex ri, uint32_t count, MapView mp,
                                                               uint32_t* __restrict__ eidx,
                                                               uint32_t create_hit, uint32_t create_miss,
                                                               unsigned long long* noop_set,
@@ -518,7 +518,7 @@ __global__ __launch_bounds__(kListBlockMax) void k_map_insert(UpdView u, const u
     uint32_t h = kNone, idx = kNone;
     uint64_t key = 0;
     if (e < count) {
-      const uint32_t slot = list ? list[e] : e;
+      const uint32_t slot = list ? list[e] : ri.at(e);
       key = u.keys[slot];
       // every listed leaf has a visited voxel: with both ops creating, it needs
       // its leaf whatever its masks hold (the usual case: p_hit, p_miss != 0.5)
@@ -607,7 +607,7 @@ __device__ __forceinline__ void update_voxel(float& x, uint32_t& ab, int k, bool
 // updated voxels.
 constexpr int kApplyLeaves = 4;  // leaves in flight per wave
 
-__global__ __launch_bounds__(256) void k_apply(UpdView u, const uint32_t* __restrict__ list,
+__global__ __launch_bounds__(256) void k_apply(UpdView u, const uint32_t* __restrict__ list, RecIndex ri,
                                                const uint32_t* __restrict__ eidx, uint32_t count,
                                                MapView mp, float l_hit, float l_miss, float t_min,
                                                float t_max, float c_max, float c_min, Status* st,
@@ -626,7 +626,7 @@ __global__ __launch_bounds__(256) void k_apply(UpdView u, const uint32_t* __rest
 #pragma unroll
     for (int q = 0; q < kApplyLeaves; ++q) {
       const uint32_t e = e0 + q;
-      slot[q] = e < count ? list[e] : kNone;
+      slot[q] = e < count ? (list ? list[e] : ri.at(e)) : kNone;
       idx[q] = e < count ? eidx[e] : kNone;
     }
 #pragma unroll
@@ -709,8 +709,8 @@ __global__ __launch_bounds__(256) void k_apply(UpdView u, const uint32_t* __rest
 // Its cost is the append counter (see list_block): 66 -> 52 us a scan on the
 // outdoor stream with 1,024 records per append instead of 256.
 __global__ __launch_bounds__(kListBlockMax) void k_group_add(const uint32_t* __restrict__ eidx,
-                                                             const uint32_t* __restrict__ list, uint32_t count,
-                                                             uint32_t t, uint32_t* gslot, uint32_t* rgrp,
+                                                             const uint32_t* __restrict__ list, RecIndex ri,
+                                                             uint32_t count, uint32_t t, uint32_t* gslot, uint32_t* rgrp,
                                                              uint32_t rgrp_stride, uint32_t* glist, uint32_t* grec,
                                                              unsigned int* ngroups) {
   __shared__ uint32_t s_wave[kListBlockMax / 64];
@@ -721,15 +721,16 @@ __global__ __launch_bounds__(kListBlockMax) void k_group_add(const uint32_t* __r
   if (e != kNone) code = atomicCAS(&gslot[e], kNone, (t << kGroupScanShift) | i);
   const bool opener = e != kNone && code == kNone;
   const uint32_t g = block_append(opener, ngroups, s_wave, &s_base);
+  const uint32_t pos = e == kNone ? kNone : (list ? list[i] : ri.at(i));
   if (opener) {
     glist[g] = e;
     rgrp[(size_t)t * rgrp_stride + i] = g;
 #pragma unroll
-    for (int k = 0; k < kDeferMax; ++k) grec[(size_t)g * kDeferMax + k] = k == (int)t ? list[i] : kNone;
+    for (int k = 0; k < kDeferMax; ++k) grec[(size_t)g * kDeferMax + k] = k == (int)t ? pos : kNone;
   } else if (e != kNone && (code >> kGroupScanShift) < t) {
     // opened by an earlier scan's launch (a scan's records name distinct leaves)
     const uint32_t go = rgrp[(size_t)(code >> kGroupScanShift) * rgrp_stride + (code & kGroupRecMask)];
-    grec[(size_t)go * kDeferMax + t] = list[i];
+    grec[(size_t)go * kDeferMax + t] = pos;
   }
 }
 
@@ -889,7 +890,7 @@ __global__ __launch_bounds__(256) void k_apply_groups(GroupScans gs, const uint3
 // each. A record's slot has one owner in a launch, so the words need no
 // atomics; words without a bit (most hit words) are neither read nor written.
 // The host has made room (the load stays under tuning.load_factor).
-__global__ __launch_bounds__(256) void k_merge_records(UpdView rec, uint32_t count, UpdView u,
+__global__ __launch_bounds__(256) void k_merge_records(UpdView rec, RecIndex ri, uint32_t count, UpdView u,
                                                        uint32_t* __restrict__ list, unsigned int* listed) {
   __shared__ uint32_t s_wave[4], s_base, s_slot[256];
   const uint32_t base = blockIdx.x * 256u;
@@ -897,7 +898,7 @@ __global__ __launch_bounds__(256) void k_merge_records(UpdView rec, uint32_t cou
   bool fresh = false;
   uint32_t slot = kNone;
   if (e < count) {
-    const uint64_t key = rec.keys[e];
+    const uint64_t key = rec.keys[ri.at(e)];
     uint32_t h = map_hash(key) & u.cap_mask;
     for (uint32_t p = 0; p <= u.cap_mask; ++p) {
       unsigned long long k = __hip_atomic_load(&u.keys[h], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -922,7 +923,7 @@ __global__ __launch_bounds__(256) void k_merge_records(UpdView rec, uint32_t cou
   for (int r = 0; r < 8; ++r) {
     const uint32_t i = (uint32_t)(r * 32 + row), to = s_slot[i];
     if (to == kNone) continue;
-    const ulonglong2 v = src[(size_t)(base + i) * 8 + l];
+    const ulonglong2 v = src[(size_t)ri.at(base + i) * 8 + l];
     if (!(v.x | v.y)) continue;
     ulonglong2 w = dst[(size_t)to * 8 + l];
     w.x |= v.x;
@@ -978,16 +979,20 @@ __global__ __launch_bounds__(256) void k_rehash_map(MapView mp, uint32_t leaf_co
 
 // Per-scan set-up of a single-scan cast in one launch: the scan record and
 // the size block (by value, so no host-to-device copy is queued behind the
-// previous scan's map update), a zeroed scan status, and optionally the
-// brick table cleared (keys EMPTY, counts and cursors 0).
+// previous scan's map update), a zeroed scan status, and for a brick cast the
+// brick table cleared (keys EMPTY, counts and cursors 0), the record set named
+// and its counters cleared.
 __global__ void k_stage_scan(ScanInfo sc, BatchCtl ctl, ScanInfo* __restrict__ d_scans,
                              BatchCtl* __restrict__ d_ctl, Status* st, unsigned long long* bkeys,
-                             unsigned long long* bcnt, uint64_t nb) {
+                             unsigned long long* bcnt, uint64_t nb, RecDest dest, RecDest* d_dest,
+                             unsigned int* rcnt) {
   const uint64_t i0 = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i0 == 0) {
     d_scans[0] = sc;
     *d_ctl = ctl;
+    if (d_dest) *d_dest = dest;
   }
+  if (d_dest && i0 < kRecRegions) rcnt[i0 * kRecCountStride] = 0u;
   if (i0 < sizeof(Status) / 4) reinterpret_cast<uint32_t*>(st)[i0] = 0u;
   const uint64_t G = (uint64_t)gridDim.x * blockDim.x;
   for (uint64_t i = i0; i < nb; i += G) {
@@ -1102,31 +1107,33 @@ hipError_t launch_compact(hipStream_t s, UpdView u, uint32_t cap, uint32_t* list
   return hipGetLastError();
 }
 
-hipError_t launch_map_insert(hipStream_t s, UpdView u, const uint32_t* list, uint32_t count, MapView mp,
+hipError_t launch_map_insert(hipStream_t s, UpdView u, const uint32_t* list, const RecIndex& ri, uint32_t count,
+                             MapView mp,
                              uint32_t* eidx, bool create_hit, bool create_miss,
                              unsigned long long* noop_set, uint32_t noop_mask, Status* st) {
   if (!count) return hipSuccess;
   const int block = list_block(count);
   const int grid = (int)std::min<uint32_t>((1u << 20) / block, (count + block - 1) / block);
-  hipLaunchKernelGGL(k_map_insert, dim3(grid), dim3(block), 0, s, u, list, count, mp, eidx,
+  hipLaunchKernelGGL(k_map_insert, dim3(grid), dim3(block), 0, s, u, list, ri, count, mp, eidx,
                      (uint32_t)create_hit, (uint32_t)create_miss, noop_set, noop_mask, st);
   return hipGetLastError();
 }
 
-hipError_t launch_apply(hipStream_t s, int grid, UpdView u, const uint32_t* list,
+hipError_t launch_apply(hipStream_t s, int grid, UpdView u, const uint32_t* list, const RecIndex& ri,
                         const uint32_t* eidx, uint32_t count, MapView mp, const float lo[6],
                         Status* st, bool clear) {
-  hipLaunchKernelGGL(k_apply, dim3(grid), dim3(256), 0, s, u, list, eidx, count, mp, lo[0], lo[1],
+  hipLaunchKernelGGL(k_apply, dim3(grid), dim3(256), 0, s, u, list, ri, eidx, count, mp, lo[0], lo[1],
                      lo[2], lo[3], lo[4], lo[5], st, (uint32_t)clear);
   return hipGetLastError();
 }
 
-hipError_t launch_group_add(hipStream_t s, const uint32_t* eidx, const uint32_t* list, uint32_t count, uint32_t t,
+hipError_t launch_group_add(hipStream_t s, const uint32_t* eidx, const uint32_t* list, const RecIndex& ri,
+                            uint32_t count, uint32_t t,
                             uint32_t* gslot, uint32_t* rgrp, uint32_t rgrp_stride, uint32_t* glist, uint32_t* grec,
                             unsigned int* ngroups) {
   if (!count) return hipSuccess;
   const int block = list_block(count);
-  hipLaunchKernelGGL(k_group_add, dim3((count + block - 1) / block), dim3(block), 0, s, eidx, list, count, t, gslot, rgrp,
+  hipLaunchKernelGGL(k_group_add, dim3((count + block - 1) / block), dim3(block), 0, s, eidx, list, ri, count, t, gslot, rgrp,
                      rgrp_stride, glist, grec, ngroups);
   return hipGetLastError();
 }
@@ -1139,10 +1146,11 @@ hipError_t launch_apply_groups(hipStream_t s, int grid, const GroupScans& gs, co
   return hipGetLastError();
 }
 
-hipError_t launch_merge_records(hipStream_t s, UpdView rec, uint32_t count, UpdView u, uint32_t* list,
+hipError_t launch_merge_records(hipStream_t s, UpdView rec, const RecIndex& ri, uint32_t count, UpdView u,
+                                uint32_t* list,
                                 unsigned int* listed) {
   if (!count) return hipSuccess;
-  hipLaunchKernelGGL(k_merge_records, dim3((count + 255) / 256), dim3(256), 0, s, rec, count, u, list, listed);
+  hipLaunchKernelGGL(k_merge_records, dim3((count + 255) / 256), dim3(256), 0, s, rec, ri, count, u, list, listed);
   return hipGetLastError();
 }
 
@@ -1171,10 +1179,11 @@ hipError_t launch_rehash_map(hipStream_t s, int grid, MapView mp, uint32_t leaf_
 
 hipError_t launch_stage_scan(hipStream_t s, const ScanInfo& sc, const BatchCtl& ctl, ScanInfo* d_scans,
                              BatchCtl* d_ctl, Status* st, unsigned long long* bkeys, unsigned long long* bcnt,
-                             uint64_t nb) {
+                             uint64_t nb, const RecDest& dest, RecDest* d_dest, unsigned int* rcnt) {
   const uint64_t blocks = (nb + 255) / 256;
   const int grid = (int)(blocks < 1 ? 1 : (blocks < 4096 ? blocks : 4096));
-  hipLaunchKernelGGL(k_stage_scan, dim3(grid), dim3(256), 0, s, sc, ctl, d_scans, d_ctl, st, bkeys, bcnt, nb);
+  hipLaunchKernelGGL(k_stage_scan, dim3(grid), dim3(256), 0, s, sc, ctl, d_scans, d_ctl, st, bkeys, bcnt, nb,
+                     dest, d_dest, rcnt);
   return hipGetLastError();
 }
 

@@ -39,18 +39,17 @@ hipError_t launch_fold(hipStream_t s, int grid, UpdView u, GroupView gv, const u
 hipError_t launch_clear_keys(hipStream_t s, int grid, UpdView u, const uint32_t* list,
                              const Status* st);
 hipError_t launch_zero_words(hipStream_t s, unsigned long long* p, uint32_t n);
-hipError_t launch_map_insert(hipStream_t s, UpdView u, const uint32_t* list, uint32_t count, MapView mp,
+// list: positions of the records (hash slots), or null: record e at ri.at(e)
+hipError_t launch_map_insert(hipStream_t s, UpdView u, const uint32_t* list, const RecIndex& ri, uint32_t count,
+                             MapView mp,
                              uint32_t* eidx, bool create_hit, bool create_miss,
                              unsigned long long* noop_set, uint32_t noop_mask, Status* st);
 // Records (one per leaf) OR-ed into an update set with room for them; the slots they open are appended to list.
-hipError_t launch_merge_records(hipStream_t s, UpdView rec, uint32_t count, UpdView u, uint32_t* list,
-                                unsigned int* listed);
+hipError_t launch_merge_records(hipStream_t s, UpdView rec, const RecIndex& ri, uint32_t count, UpdView u,
+                                uint32_t* list, unsigned int* listed);
 hipError_t launch_clear_listed(hipStream_t s, UpdView u, const uint32_t* list, uint32_t count);
 hipError_t launch_set_u32(hipStream_t s, unsigned int* p, uint32_t v);
-hipError_t launch_rec_gather(hipStream_t s, int grid, const uint32_t* list, UpdView sparse, const RecDest* dest,
-                             const Status* st);
-hipError_t launch_put_dest(hipStream_t s, RecDest* dst, RecDest v);
-hipError_t launch_iota_u32(hipStream_t s, uint32_t* p, uint32_t n);
+hipError_t launch_rec_total(hipStream_t s, const RecDest* dest, const unsigned int* rcnt, Status* st);
 hipError_t launch_snap_count(hipStream_t s, const Status* st, uint32_t* host_dst);
 // Deferred brick-path scans applied as one group pass (integrate_kernels.hip).
 constexpr int kDeferMax = 8;                       // scans per group pass
@@ -60,13 +59,14 @@ struct GroupScans {
   const unsigned long long* masks[kDeferMax];  // record masks of scan t (16 words per position)
   int nscan;
 };
-hipError_t launch_group_add(hipStream_t s, const uint32_t* eidx, const uint32_t* list, uint32_t count, uint32_t t,
+hipError_t launch_group_add(hipStream_t s, const uint32_t* eidx, const uint32_t* list, const RecIndex& ri,
+                            uint32_t count, uint32_t t,
                             uint32_t* gslot, uint32_t* rgrp, uint32_t rgrp_stride, uint32_t* glist, uint32_t* grec,
                             unsigned int* ngroups);
 hipError_t launch_apply_groups(hipStream_t s, int grid, const GroupScans& gs, const uint32_t* glist,
                                const uint32_t* grec, const unsigned int* ngroups, uint32_t* gslot, MapView mp,
                                const float lo[6], Status* st);
-hipError_t launch_apply(hipStream_t s, int grid, UpdView u, const uint32_t* list,
+hipError_t launch_apply(hipStream_t s, int grid, UpdView u, const uint32_t* list, const RecIndex& ri,
                         const uint32_t* eidx, uint32_t count, MapView mp, const float lo[6],
                         Status* st, bool clear);
 hipError_t launch_rehash_update(hipStream_t s, int grid, UpdView from, uint32_t from_cap,
@@ -76,7 +76,7 @@ hipError_t launch_rehash_map(hipStream_t s, int grid, MapView mp, uint32_t leaf_
 hipError_t launch_fill_u64(hipStream_t s, unsigned long long* p, uint64_t n, uint64_t v);
 hipError_t launch_stage_scan(hipStream_t s, const ScanInfo& sc, const BatchCtl& ctl, ScanInfo* d_scans,
                              BatchCtl* d_ctl, Status* st, unsigned long long* bkeys, unsigned long long* bcnt,
-                             uint64_t nb);
+                             uint64_t nb, const RecDest& dest, RecDest* d_dest, unsigned int* rcnt);
 hipError_t launch_dirty_list(hipStream_t s, int grid, uint8_t* dirty, uint32_t leaf_count,
                              uint32_t* list, Status* st);
 hipError_t launch_gather_leaves(hipStream_t s, int grid, const uint32_t* list, uint32_t count,
@@ -99,13 +99,11 @@ hipError_t launch_seg_fill(hipStream_t s, int grid, const int4* rayinfo, const S
                            uint32_t seg_cap, Status* st);
 hipError_t launch_brick_walk(hipStream_t s, int grid, const BrickItem* items, const uint4* segs,
                              const int4* rayinfo, const ScanInfo* scans, const double* tbl,
-                             BrickView bv, unsigned long long* shared_bits, UpdView rec,
-                             unsigned long long* leaf_mask, uint32_t rec_cap, Status* st);
-hipError_t launch_rec_list(hipStream_t s, const unsigned long long* leaf_mask, uint64_t* bsum, uint64_t* boff,
-                           uint32_t nb_cap, uint32_t* list, Status* st);
+                             BrickView bv, unsigned long long* shared_bits, const RecDest* dest,
+                             unsigned int* rcnt, Status* st);
 hipError_t launch_split_emit(hipStream_t s, int grid, const uint32_t* split_slot,
-                             unsigned long long* shared_bits, BrickView bv, UpdView rec,
-                             unsigned long long* leaf_mask, uint32_t rec_cap, Status* st);
+                             unsigned long long* shared_bits, BrickView bv, const RecDest* dest,
+                             unsigned int* rcnt, Status* st);
 
 hipError_t launch_snapshot_nodes(hipStream_t s, MapView mp, uint32_t first, uint64_t leaf_bound, RtView rt,
                                  RtInfo* info, const unsigned long long* noop, uint32_t noop_cap,

@@ -190,22 +190,17 @@ struct vdbgpu_map {
   unsigned long long* wsc = nullptr;
   uint64_t wtab_cap = 0;
   uint32_t split_cap = 0;
-  // update-leaf records: the walk fills positional records (64 positions per
-  // work item, cast stream only), listed and copied densely into one record
-  // set of a ring; the cast of scan i+1 fills one set while the map stream
-  // still applies earlier scans from the others (two sets, or 2 defer + 2
-  // when scans are applied in groups)
+  // update-leaf records: the walk appends them to one record set of a ring; the
+  // cast of scan i+1 fills one set while the map stream still applies earlier
+  // scans from the others (two sets, or 2 defer + 2 when scans are applied in
+  // groups)
   static constexpr int kRecSets = 2 * kDeferMax + 2;
-  unsigned long long* rkeys = nullptr;
-  unsigned long long* rmasks = nullptr;
-  uint32_t* rlist = nullptr;  // filled record positions (dense)
   unsigned long long* dkeys[kRecSets] = {};   // record set: leaf keys
   unsigned long long* dmasks[kRecSets] = {};  // record set: 16 mask words per record
   uint32_t* reidx[kRecSets] = {};             // record set: map leaf index of each record
+  RecIndex rindex[kRecSets] = {};             // record set: where its scan's records lie
   uint32_t dcap[kRecSets] = {};
   uint32_t dense_hint = 0;     // record-set size for a first use (largest scan seen, +25%)
-  uint32_t* ident = nullptr;   // 0, 1, 2, ...: the list of a dense record set
-  uint32_t ident_cap = 0;
   hipEvent_t rec_free[kRecSets] = {};  // recorded on the map stream after the last read
   // leaf count after the map insert of each record set's scan (pinned, copied
   // on the map stream before ins_done), for a tight leaf-count bound
@@ -236,11 +231,6 @@ struct vdbgpu_map {
   uint32_t* grec = nullptr;   // per group: record position of each scan (kDeferMax)
   uint64_t grp_cap = 0;
   unsigned int* ngroups = nullptr;
-  uint32_t rec_cap = 0;        // record positions: 64 per work item and per split brick
-  unsigned long long* leaf_mask = nullptr;  // filled positions per 64-position group
-  uint64_t* lbsum = nullptr;
-  uint64_t* lboff = nullptr;
-  uint32_t group_cap = 0;      // groups: work items + split bricks
   double* tbl = nullptr;
   uint32_t tbl_n = 0;
   // map sections by cells: cell table and its block sums, and the pinned
@@ -268,10 +258,10 @@ struct vdbgpu_map {
   Status* h_st = nullptr;
   // brick-path casts whose status the host has not read: two host slots
   Status* h_cst = nullptr;
-  RecDest* d_dest = nullptr;  // the record set the next cast copies into
+  RecDest* d_dest = nullptr;  // the record set the next cast fills
+  unsigned int* d_rcnt = nullptr;  // its regions' record counters
   hipEvent_t cst_done[2] = {};
   int cst_next = 0;
-  uint64_t cast_seq = 0;    // brick casts enqueued (re-runs included)
   // brick casts of batched inserts replayed from captured graphs, one per
   // exact set of launch arguments (least recently used dropped first)
   struct CastGraph {
@@ -868,7 +858,8 @@ int launch_fold_stage(vdbgpu_map* m, Source& src, bool from_groups) {
 // visit bound of the scans in *visits_bound.
 int stage_scans(vdbgpu_map* m, hipStream_t stream, const float* xyz, int64_t stride, bool on_device,
                 const std::vector<ScanInfo>& scans, uint32_t n_total, bool batched,
-                uint64_t* visits_bound, bool clear_bricks = false) {
+                uint64_t* visits_bound, const RecDest* dest = nullptr) {
+  const bool clear_bricks = dest != nullptr;  // a brick cast: its record set, the brick table cleared
   int r;
   if ((r = ensure_rays(m, n_total))) return r;
   uint32_t ext_max = 1;
@@ -900,17 +891,14 @@ int stage_scans(vdbgpu_map* m, hipStream_t stream, const float* xyz, int64_t str
     CK(launch_stage_scan(stream, scans[0], ctl, m->d_scans, m->d_ctl, &m->d_st[0],
                          clear_bricks ? m->bkeys : nullptr,
                          clear_bricks ? reinterpret_cast<unsigned long long*>(m->bcnt) : nullptr,
-                         clear_bricks ? m->bcap : 0));
+                         clear_bricks ? m->bcap : 0, dest ? *dest : RecDest{}, dest ? m->d_dest : nullptr,
+                         m->d_rcnt));
   } else {
     std::copy(scans.begin(), scans.end(), m->h_scans);
     *m->h_ctl = ctl;
     CK(hipMemcpyAsync(m->d_scans, m->h_scans, scans.size() * sizeof(ScanInfo), hipMemcpyHostToDevice, stream));
     CK(hipMemcpyAsync(m->d_ctl, m->h_ctl, sizeof(BatchCtl), hipMemcpyHostToDevice, stream));
     CK(hipMemsetAsync(&m->d_st[0], 0, sizeof(Status), stream));
-    if (clear_bricks) {
-      CK(launch_fill_u64(stream, m->bkeys, m->bcap, kEmpty));
-      CK(launch_fill_u64(stream, reinterpret_cast<unsigned long long*>(m->bcnt), m->bcap, 0));
-    }
   }
   const bool vec4 = stride == 16 && (reinterpret_cast<uintptr_t>(pts) & 15) == 0;
   Timer t(m, kPrep, stream);
@@ -1114,7 +1102,7 @@ int do_accumulate(vdbgpu_map* m, Source& src, const float* xyz, int64_t n, int64
 }
 
 // Brick path tables large enough for the given counts (grown, never shrunk).
-int ensure_bricks(vdbgpu_map* m, uint32_t bcap, uint32_t seg_cap, uint32_t split_cap, uint32_t rec_cap) {
+int ensure_bricks(vdbgpu_map* m, uint32_t bcap, uint32_t seg_cap, uint32_t split_cap) {
   if (bcap > m->bcap) {
     dfree(m, &m->bkeys, m->bcap);
     dfree(m, &m->bcnt, (size_t)m->bcap * 2);
@@ -1145,25 +1133,6 @@ int ensure_bricks(vdbgpu_map* m, uint32_t bcap, uint32_t seg_cap, uint32_t split
     CK(dalloc(m, &m->split_slot, split_cap));
     CK(dalloc(m, &m->shared_bits, (size_t)split_cap * 1024));
     CK(launch_fill_u64(m->cast, m->shared_bits, (uint64_t)split_cap * 1024, 0));
-  }
-  if (rec_cap > m->rec_cap) {  // positional records: read by the cast stream only
-    dfree(m, &m->rkeys, m->rec_cap);
-    dfree(m, &m->rmasks, (size_t)m->rec_cap * 16);
-    dfree(m, &m->rlist, m->rec_cap);
-    m->rec_cap = rec_cap;
-    CK(dalloc(m, &m->rkeys, rec_cap));
-    CK(dalloc(m, &m->rmasks, (size_t)rec_cap * 16));
-    CK(dalloc(m, &m->rlist, rec_cap));
-  }
-  const uint32_t groups = (m->item_cap + m->split_cap + 255) & ~255u;
-  if (groups > m->group_cap) {
-    dfree(m, &m->leaf_mask, m->group_cap);
-    dfree(m, &m->lbsum, m->group_cap / 256);
-    dfree(m, &m->lboff, m->group_cap / 256);
-    m->group_cap = groups;
-    CK(dalloc(m, &m->leaf_mask, groups));
-    CK(dalloc(m, &m->lbsum, groups / 256));
-    CK(dalloc(m, &m->lboff, groups / 256));
   }
   return VDBGPU_OK;
 }
@@ -1241,8 +1210,8 @@ int flush_pending(vdbgpu_map* m) {
       // workgroups than the CUs hold at once (four leaves per wave, four waves
       // per SIMD), so the last ones fill in behind the slow ones (synchronous
       // p50 2.63 ms at 16 per CU against 2.65 at 8 and 4)
-      CK(launch_apply(m->stream, std::min<int>(m->num_cu * 16, (int)((recs + 1) / 2)), rec, m->ident, m->reidx[X],
-                      recs, map_view(m), m->lo, &m->d_st[3], false));
+      CK(launch_apply(m->stream, std::min<int>(m->num_cu * 16, (int)((recs + 1) / 2)), rec, nullptr, m->rindex[X],
+                      m->reidx[X], recs, map_view(m), m->lo, &m->d_st[3], false));
     }
     m->npend = 0;
     int r;
@@ -1267,7 +1236,7 @@ int flush_pending(vdbgpu_map* m) {
     Timer t(m, kCompact);
     for (int p = 0; p < P; ++p) {  // in scan order: a scan's records join the groups earlier ones opened
       const int X = m->pend_set[p];
-      CK(launch_group_add(m->stream, m->reidx[X], m->ident, m->pend_recs[p], (uint32_t)p, m->gslot, m->rgrp, rs,
+      CK(launch_group_add(m->stream, m->reidx[X], nullptr, m->rindex[X], m->pend_recs[p], (uint32_t)p, m->gslot, m->rgrp, rs,
                           m->gl, m->grec, m->ngroups));
       gs.masks[p] = m->dmasks[X];
     }
@@ -1301,8 +1270,7 @@ struct BrickCast {
   ScanInfo sc{};
   int X = 0;     // record set
   int slot = 0;  // host status slot: m->h_cst[2 slot] (scan), [2 slot + 1] (map snapshot)
-  uint32_t cap = 0;    // capacity of set X when the records were copied into it
-  uint64_t seq = 0;    // m->cast_seq of its latest enqueue
+  uint32_t cap = 0;    // capacity of set X when it was cast
   uint64_t epoch = 0;  // m->cast_epoch then
 };
 
@@ -1315,8 +1283,7 @@ int brick_tables(vdbgpu_map* m, int64_t n, double R) {
     const uint64_t vb = (uint64_t)n * (1 + 3 * (uint64_t)ext);
     const uint64_t segs0 = std::min<uint64_t>(vb, 16ull * (uint64_t)n);
     if ((r = ensure_bricks(m, (uint32_t)std::max<uint64_t>(4096, next_pow2((uint64_t)n / 2)),
-                           (uint32_t)std::max<uint64_t>(1u << 16, std::min<uint64_t>(segs0, 0xC0000000ull)), 256,
-                           (uint32_t)std::max<uint64_t>(1u << 16, std::min<uint64_t>(8ull * n, 0xC0000000ull)))))
+                           (uint32_t)std::max<uint64_t>(1u << 16, std::min<uint64_t>(segs0, 0xC0000000ull)), 256)))
       return r;
   }
   const int nb = (int)((n + kPrepBlock - 1) / kPrepBlock);
@@ -1331,13 +1298,12 @@ int brick_tables(vdbgpu_map* m, int64_t n, double R) {
   return VDBGPU_OK;
 }
 
-// The brick stages of a staged scan on the cast stream: cut, walk, record
-// list and the copy into the record set named in m->d_dest. `nb` = workgroups
+// The brick stages of a staged scan on the cast stream: cut, walk (records
+// into the set named in m->d_dest) and record counts. `nb` = workgroups
 // of the cut (lanes past the scan's rays do nothing).
 int cast_chain(vdbgpu_map* m, int nb) {
   hipStream_t cs = m->cast;
   const BrickView bv{m->bkeys, m->bcnt, m->bcnt + m->bcap, m->bcap - 1};
-  const UpdView rec{m->rkeys, m->rmasks, 0};
   {
     Timer t(m, kTraverse, cs);
     CK(launch_seg_count(cs, nb, m->rayinfo, m->d_scans, m->d_ctl, m->tbl, bv, m->wkey, m->wsc, &m->d_st[0]));
@@ -1351,14 +1317,12 @@ int cast_chain(vdbgpu_map* m, int nb) {
     // 64 work-groups per CU over the grid-stride item loop: bricks cost very
     // different amounts, and the finer split shortens the tail.
     CK(launch_brick_walk(cs, m->num_cu * 64, m->items, m->segs, m->rayinfo, m->d_scans, m->tbl, bv,
-                         m->shared_bits, rec, m->leaf_mask, m->rec_cap, &m->d_st[0]));
+                         m->shared_bits, m->d_dest, m->d_rcnt, &m->d_st[0]));
   }
   {
     Timer t(m, kCompact, cs);
-    CK(launch_split_emit(cs, m->num_cu, m->split_slot, m->shared_bits, bv, rec, m->leaf_mask,
-                         m->rec_cap, &m->d_st[0]));
-    CK(launch_rec_list(cs, m->leaf_mask, m->lbsum, m->lboff, m->group_cap / 256, m->rlist, &m->d_st[0]));
-    CK(launch_rec_gather(cs, m->num_cu * 8, m->rlist, rec, m->d_dest, &m->d_st[0]));
+    CK(launch_split_emit(cs, m->num_cu, m->split_slot, m->shared_bits, bv, m->d_dest, m->d_rcnt, &m->d_st[0]));
+    CK(launch_rec_total(cs, m->d_dest, m->d_rcnt, &m->d_st[0]));
   }
   return VDBGPU_OK;
 }
@@ -1381,9 +1345,8 @@ int launch_cast_graph(vdbgpu_map* m, int nb) {
   const std::vector<uint64_t> key = {
       (uint64_t)grid, (uint64_t)m->num_cu, u(m->rayinfo), u(m->d_scans), u(m->d_ctl), u(m->tbl), u(m->bkeys),
       u(m->bcnt), m->bcap, u(m->wkey), u(m->wsc), m->wtab_cap, u(m->segs), m->seg_cap, u(m->bbsum), u(m->bboff),
-      u(m->items), m->item_cap, u(m->split_slot), m->split_cap, u(m->shared_bits), u(m->rkeys), u(m->rmasks),
-      u(m->leaf_mask), m->rec_cap, u(m->lbsum), u(m->lboff), m->group_cap, u(m->rlist), u(m->d_dest),
-      u(m->d_st)};
+      u(m->items), m->item_cap, u(m->split_slot), m->split_cap, u(m->shared_bits), u(m->d_dest),
+      u(m->d_rcnt), u(m->d_st)};
   vdbgpu_map::CastGraph* hit = nullptr;
   for (auto& g : m->cast_graphs)
     if (g.key == key) hit = &g;
@@ -1418,10 +1381,10 @@ int launch_cast_graph(vdbgpu_map* m, int nb) {
   return VDBGPU_OK;
 }
 
-// Enqueues the cast of c on the cast stream: staging (prep, brick table
-// cleared), record set c.X named for the copy, brick cut, walk, record list
-// and the copy (launched, or replayed from a graph), then the copy of its
-// status (and a snapshot of the map's leaf count) into host slot c.slot. A first attempt takes the next record set of the ring and
+// Enqueues the cast of c on the cast stream: staging (record set c.X named,
+// brick table cleared, prep), brick cut, walk and record counts (launched, or
+// replayed from a graph), then the copy of its status (and a snapshot of the
+// map's leaf count) into host slot c.slot. A first attempt takes the next record set of the ring and
 // waits until the map stream has applied the scan that used it last; a re-run
 // (attempt > 0, tables grown) stages the scan again, since a later cast may
 // have used the shared tables meanwhile.
@@ -1429,8 +1392,6 @@ int brick_enqueue(vdbgpu_map* m, BrickCast& c, int attempt) {
   int r;
   hipStream_t cs = m->cast;
   const int nb = (int)((c.n + kPrepBlock - 1) / kPrepBlock);
-  uint64_t vb = 0;
-  if ((r = stage_scans(m, cs, c.xyz, c.stride, c.on_device, {c.sc}, (uint32_t)c.n, false, &vb, true))) return r;
   if (attempt == 0) {
     // record set X: free once the map stream has applied the scan that last used it
     c.X = m->rec_cur;
@@ -1438,6 +1399,11 @@ int brick_enqueue(vdbgpu_map* m, BrickCast& c, int attempt) {
     c.slot = m->cst_next;
     m->cst_next ^= 1;
     CK(hipStreamWaitEvent(cs, m->rec_free[c.X], 0));
+    if (m->dense_hint == 0 && m->dcap[c.X] == 0) {
+      // the map's first scan: a guess of its records, for this set alone
+      if ((r = grow_set(m, c.X, (uint32_t)std::max<int64_t>(4096, std::min<int64_t>(c.n / 4, 1 << 20))))) return r;
+      m->dense_hint = 0;
+    }
     if (m->dcap[c.X] < m->dense_hint) {  // a first use of set X: size it like the others
       CK(hipStreamSynchronize(cs));      // (the map stream is done with it)
       if ((r = grow_set(m, c.X, m->dense_hint))) return r;
@@ -1448,7 +1414,9 @@ int brick_enqueue(vdbgpu_map* m, BrickCast& c, int attempt) {
     }
   }
   c.cap = m->dcap[c.X];  // (a later first use may size an empty set X before this is checked)
-  CK(launch_put_dest(cs, m->d_dest, RecDest{m->dkeys[c.X], m->dmasks[c.X], c.cap, 0}));
+  const RecDest dest{m->dkeys[c.X], m->dmasks[c.X], c.cap, 0};
+  uint64_t vb = 0;
+  if ((r = stage_scans(m, cs, c.xyz, c.stride, c.on_device, {c.sc}, (uint32_t)c.n, false, &vb, &dest))) return r;
   if (m->graph_casts && !m->profiling) {
     if ((r = launch_cast_graph(m, nb))) return r;
   } else if ((r = cast_chain(m, nb))) {
@@ -1458,19 +1426,17 @@ int brick_enqueue(vdbgpu_map* m, BrickCast& c, int attempt) {
   // applying earlier scans meanwhile
   CK(hipMemcpyAsync(m->h_cst + 2 * c.slot, m->d_st, 2 * sizeof(Status), hipMemcpyDeviceToHost, cs));
   CK(hipEventRecord(m->cst_done[c.slot], cs));
-  c.seq = ++m->cast_seq;
   c.epoch = m->cast_epoch;
   return VDBGPU_OK;
 }
 
 // Waits for the status of the cast of c and checks it: errors fail the scan,
-// table overflows grow the tables and cast the scan again (nothing of it has
-// been applied), a record set too small grows and takes the records again.
-// A cast enqueued before an overflow of an earlier cast was found started
-// from split-brick bitmaps holding that cast's partial ORs: it runs again.
-// When another cast has run since c's, the shared tables no longer hold c's
-// records, so a set too small also means casting again. A scan with records
-// is left staged for the map stream (commit_staged).
+// table overflows, or a record set too small, grow the tables or the set and
+// cast the scan again (nothing of it has been applied). A cast enqueued before
+// a table overflow of an earlier cast was found started from split-brick
+// bitmaps holding that cast's partial ORs: it runs again. (A full record set
+// stops no walk, so it leaves the bitmaps empty as every cast does.) A scan
+// with records is left staged for the map stream (commit_staged).
 int brick_check(vdbgpu_map* m, BrickCast& c) {
   int r;
   const int X = c.X;
@@ -1482,35 +1448,41 @@ int brick_check(vdbgpu_map* m, BrickCast& c) {
       if ((r = brick_enqueue(m, c, attempt))) return r;
       continue;
     }
-    const bool later = c.seq != m->cast_seq;
     const Status* h = m->h_cst + 2 * c.slot;
     m->leaf_count_ub = leaf_bound(m, h[1].leaf_count, m->rec_seq[X]);
     if (h[1].map_full)
       return fail(m, VDBGPU_DEVICE_ERROR, "leaf pool overflow in a map insert (internal bound violated)");
     const Status st = h[0];
     if ((r = scan_error(m, st, false))) return r;
-    if (st.overflow == 0 && (st.records <= c.cap || !later)) break;
-    if (st.overflow) {
+    if (st.overflow == 0) break;
+    if (st.overflow & ~kOvfRecords) {
       const uint32_t bcap = (st.overflow & kOvfBricks) ? (uint32_t)std::min<uint64_t>(1u << 30, (uint64_t)m->bcap * 4) : m->bcap;
       const uint32_t seg_cap = st.segs > m->seg_cap ? grow_cap(st.segs, m->seg_cap) : m->seg_cap;
       const uint32_t split_cap = st.splits > m->split_cap ? grow_cap(st.splits, m->split_cap) : m->split_cap;
-      const uint64_t positions = (uint64_t)(st.items + st.splits) * 64;
-      const uint32_t rec_cap = positions > m->rec_cap ? grow_cap(positions, m->rec_cap) : m->rec_cap;
       if ((st.overflow & kOvfBricks) && bcap == m->bcap) return fail(m, VDBGPU_DEVICE_ERROR, "brick table cannot grow");
-      if ((r = ensure_bricks(m, bcap, seg_cap, split_cap, rec_cap))) return r;
+      if ((r = ensure_bricks(m, bcap, seg_cap, split_cap))) return r;
+      // the records are at most 64 per item and split brick: room for them now
+      // saves a growing map's scan another cast
+      const uint64_t most = (uint64_t)(st.items + st.splits) * 64;
+      if (!(st.overflow & kOvfBricks) && most > m->dcap[X] && most <= 64ull * (uint64_t)c.n &&
+          (r = grow_set(m, X, (uint32_t)std::min<uint64_t>(most, 0xC0000000ull))))
+        return r;
       // split-brick bitmaps may hold partial ORs of the stopped run: cleared,
       // and any cast enqueued since runs again
       CK(launch_fill_u64(m->cast, m->shared_bits, (uint64_t)m->split_cap * 1024, 0));
       ++m->cast_epoch;
-    } else if (st.records > m->dcap[X] &&
-               (r = grow_set(m, X, (uint32_t)std::min<uint64_t>(st.records + (uint64_t)st.records / 4,
-                                                                0xC0000000ull)))) {
-      return r;
+    } else {
+      // the walk counted every record: room for the fullest region (or the whole
+      // scan, where it used one), a quarter more
+      const uint64_t regions = st.items >= kRecRegionItems ? kRecRegions : 1;
+      const uint64_t want = std::max<uint64_t>(st.records, regions * st.rec_most);
+      if ((r = grow_set(m, X, (uint32_t)std::min<uint64_t>(want + want / 4 + regions, 0xC0000000ull)))) return r;
     }
     if ((r = brick_enqueue(m, c, attempt))) return r;
   }
   const Status& st = m->h_cst[2 * c.slot];
-  const uint32_t recs = st.records;  // listed in m->rlist, copied to set X when it had room
+  const uint32_t recs = st.records;
+  m->dense_hint = std::max(m->dense_hint, std::min<uint32_t>(c.cap, recs + recs / 4 + 64));
   m->stats.scans += 1;
   m->stats.rays += st.rays;
   m->stats.visits += st.total;
@@ -1519,16 +1491,8 @@ int brick_check(vdbgpu_map* m, BrickCast& c) {
     m->rec_seq[X] = m->ledger_seq;
     return VDBGPU_OK;
   }
-  if (recs > c.cap) {  // set X (no pending scan holds it) grows; the copy runs again
-    if (recs > m->dcap[X] &&
-        (r = grow_set(m, X, (uint32_t)std::min<uint64_t>(recs + (uint64_t)recs / 4, 0xC0000000ull))))
-      return r;
-    c.cap = m->dcap[X];
-    CK(launch_put_dest(m->cast, m->d_dest, RecDest{m->dkeys[X], m->dmasks[X], c.cap, 0}));
-    CK(launch_rec_gather(m->cast, m->num_cu * 8, m->rlist, UpdView{m->rkeys, m->rmasks, 0}, m->d_dest,
-                         &m->d_st[0]));
-    CK(hipStreamSynchronize(m->cast));
-  }
+  for (uint32_t g = 0; g < kRecRegions; ++g) m->rindex[X].pre[g] = st.rec_pre[g];
+  m->rindex[X].stride = st.rec_stride;
   m->staged = true;
   m->staged_set = X;
   m->staged_recs = recs;
@@ -1596,7 +1560,7 @@ int run_brick_accumulate(vdbgpu_map* m, Source& src, const float* xyz, int64_t n
     }
   }
   if (!src.counting) CK(launch_set_u32(m->stream, src.d_count, src.pending));
-  CK(launch_merge_records(m->stream, UpdView{m->dkeys[X], m->dmasks[X], 0}, recs, upd_view(src), src.list,
+  CK(launch_merge_records(m->stream, UpdView{m->dkeys[X], m->dmasks[X], 0}, m->rindex[X], recs, upd_view(src), src.list,
                           src.d_count));
   CK(hipEventRecord(m->rec_free[X], m->stream));
   m->rec_seq[X] = m->ledger_seq;
@@ -1616,18 +1580,12 @@ int commit_staged(vdbgpu_map* m) {
   int r;
   const uint32_t art_new = m->art_leaves ? 0 : m->art_count;  // leaves the activation may create
   if ((r = ensure_map(m, m->leaf_count_ub + recs + art_new))) return r;
-  if (recs > m->ident_cap) {
-    dfree(m, &m->ident, m->ident_cap);
-    m->ident_cap = m->dcap[X];
-    CK(dalloc(m, &m->ident, m->ident_cap));
-    CK(launch_iota_u32(m->stream, m->ident, m->ident_cap));
-  }
   bool ch, cm;
   create_flags(m, &ch, &cm);
   const UpdView rec{m->dkeys[X], m->dmasks[X], 0};
   {
     Timer t(m, kCompact);
-    CK(launch_map_insert(m->stream, rec, m->ident, recs, map_view(m), m->reidx[X], ch, cm, m->noop4096,
+    CK(launch_map_insert(m->stream, rec, nullptr, m->rindex[X], recs, map_view(m), m->reidx[X], ch, cm, m->noop4096,
                          vdbgpu_map::kNoopCap - 1, &m->d_st[1]));
   }
   m->leaf_count_ub += recs;
@@ -1662,7 +1620,7 @@ int commit_staged(vdbgpu_map* m) {
   const int g2 = std::min<int>(m->num_cu * 3, (int)((recs + 1) / 2));
   {
     Timer t(m, kApply);
-    CK(launch_apply(m->stream, g2, rec, m->ident, m->reidx[X], recs, map_view(m), m->lo, &m->d_st[3], false));
+    CK(launch_apply(m->stream, g2, rec, nullptr, m->rindex[X], m->reidx[X], recs, map_view(m), m->lo, &m->d_st[3], false));
   }
   if ((r = check_tiles(m))) return r;
   if ((r = activate_artificial(m))) return r;  // enters its new leaves in the ledger
@@ -1816,9 +1774,9 @@ int integrate_groups(vdbgpu_map* m, const std::vector<Source*>& ready, bool ch, 
       for (size_t i = i0; i < i1; ++i) {
         Source& s = *ready[i];
         const uint32_t p = (uint32_t)(i - i0);
-        CK(launch_map_insert(m->stream, upd_view(s), s.list, s.pending, map_view(m), m->eidx + off, ch, cm,
+        CK(launch_map_insert(m->stream, upd_view(s), s.list, RecIndex{}, s.pending, map_view(m), m->eidx + off, ch, cm,
                              m->noop4096, vdbgpu_map::kNoopCap - 1, &m->d_st[1]));
-        CK(launch_group_add(m->stream, m->eidx + off, s.list, s.pending, p, m->gslot, m->rgrp, rs, m->gl, m->grec,
+        CK(launch_group_add(m->stream, m->eidx + off, s.list, RecIndex{}, s.pending, p, m->gslot, m->rgrp, rs, m->gl, m->grec,
                             m->ngroups));
         gs.masks[p] = s.masks;
         off += s.pending;
@@ -1879,12 +1837,12 @@ int do_integrate(vdbgpu_map* m) {
     const int g2 = std::min<int>(m->num_cu * 16, (int)((s.pending + 1) / 2));  // 128 lanes per leaf
     {
       Timer t(m, kCompact);
-      CK(launch_map_insert(m->stream, upd_view(s), s.list, s.pending, map_view(m), m->eidx, ch, cm,
+      CK(launch_map_insert(m->stream, upd_view(s), s.list, RecIndex{}, s.pending, map_view(m), m->eidx, ch, cm,
                            m->noop4096, vdbgpu_map::kNoopCap - 1, &m->d_st[1]));
     }
     {
       Timer t(m, kApply);
-      CK(launch_apply(m->stream, g2, upd_view(s), s.list, m->eidx, s.pending, map_view(m), m->lo,
+      CK(launch_apply(m->stream, g2, upd_view(s), s.list, RecIndex{}, m->eidx, s.pending, map_view(m), m->lo,
                       &m->d_st[3], true));
     }
     m->leaf_count_ub += s.pending;
@@ -1965,7 +1923,7 @@ int mark_set(vdbgpu_map* m, Source& s, uint32_t cap0, Mark&& mark, uint32_t* cou
 int apply_edit(vdbgpu_map* m, Source& s, uint32_t count, uint32_t* eidx, int op, float val, bool need,
                bool clear) {
   if (count == 0) return VDBGPU_OK;
-  CK(launch_map_insert(m->stream, upd_view(s), s.list, count, map_view(m), eidx, need, need, m->noop4096,
+  CK(launch_map_insert(m->stream, upd_view(s), s.list, RecIndex{}, count, map_view(m), eidx, need, need, m->noop4096,
                        vdbgpu_map::kNoopCap - 1, &m->d_st[1]));
   CK(launch_set_voxels(m->stream, upd_view(s), s.list, eidx, count, map_view(m), op, val, m->lo[3], clear));
   m->touched = true;
@@ -2078,18 +2036,11 @@ uint64_t walk_scratch(vdbgpu_map* m, bool release) {
   one(m->shared_bits, (size_t)m->split_cap * 1024);
   one(m->wkey, m->wtab_cap);
   one(m->wsc, m->wtab_cap);
-  one(m->rkeys, m->rec_cap);
-  one(m->rmasks, (size_t)m->rec_cap * 16);
-  one(m->rlist, m->rec_cap);
-  one(m->leaf_mask, m->group_cap);
-  one(m->lbsum, m->group_cap / 256);
-  one(m->lboff, m->group_cap / 256);
   for (int X = 0; X < vdbgpu_map::kRecSets; ++X) {
     one(m->dkeys[X], m->dcap[X]);
     one(m->dmasks[X], (size_t)m->dcap[X] * 16);
     one(m->reidx[X], m->dcap[X]);
   }
-  one(m->ident, m->ident_cap);
   one(m->gslot, m->gslot_cap);
   one(m->rgrp, m->rgrp_cap);
   one(m->gl, m->grp_cap);
@@ -2121,10 +2072,9 @@ uint64_t walk_scratch(vdbgpu_map* m, bool release) {
     m->ray_cap = 0;
     m->chunk_cap = 0;
     m->eidx_cap = 0;
-    m->bcap = m->seg_cap = m->item_cap = m->split_cap = m->rec_cap = m->group_cap = 0;
+    m->bcap = m->seg_cap = m->item_cap = m->split_cap = 0;
     m->wtab_cap = 0;
     for (int X = 0; X < vdbgpu_map::kRecSets; ++X) m->dcap[X] = 0;
-    m->ident_cap = 0;
     m->gslot_cap = 0;
     m->rgrp_cap = 0;
     m->grp_cap = 0;
@@ -2230,6 +2180,7 @@ int32_t vdbgpu_create(double resolution, vdbgpu_map** out) {
       hipHostMalloc((void**)&m->h_st, 4 * sizeof(Status), hipHostMallocDefault) != hipSuccess ||
       hipHostMalloc((void**)&m->h_cst, 4 * sizeof(Status), hipHostMallocDefault) != hipSuccess ||
       hipMalloc((void**)&m->d_dest, sizeof(RecDest)) != hipSuccess ||
+      hipMalloc((void**)&m->d_rcnt, kRecRegions * kRecCountStride * sizeof(unsigned int)) != hipSuccess ||
       hipEventCreateWithFlags(&m->cst_done[0], hipEventDisableTiming) != hipSuccess ||
       hipEventCreateWithFlags(&m->cst_done[1], hipEventDisableTiming) != hipSuccess ||
       hipMemsetAsync(m->d_st, 0, 4 * sizeof(Status), m->stream) != hipSuccess) {
@@ -2293,24 +2244,17 @@ void vdbgpu_destroy(vdbgpu_map* m) {
   dfree(m, &m->shared_bits, (size_t)m->split_cap * 1024);
   dfree(m, &m->wkey, m->wtab_cap);
   dfree(m, &m->wsc, m->wtab_cap);
-  dfree(m, &m->rkeys, m->rec_cap);
-  dfree(m, &m->rmasks, (size_t)m->rec_cap * 16);
-  dfree(m, &m->rlist, m->rec_cap);
   for (int i = 0; i < vdbgpu_map::kRecSets; ++i) {
     free_set(m, i);
     if (m->rec_free[i]) (void)hipEventDestroy(m->rec_free[i]);
     if (m->ins_done[i]) (void)hipEventDestroy(m->ins_done[i]);
   }
   if (m->h_lc) (void)hipHostFree(m->h_lc);
-  dfree(m, &m->ident, m->ident_cap);
   dfree(m, &m->gslot, m->gslot_cap);
   dfree(m, &m->rgrp, m->rgrp_cap);
   dfree(m, &m->gl, m->grp_cap);
   dfree(m, &m->grec, m->grp_cap * kDeferMax);
   dfree(m, &m->ngroups, 1);
-  dfree(m, &m->leaf_mask, m->group_cap);
-  dfree(m, &m->lbsum, m->group_cap / 256);
-  dfree(m, &m->lboff, m->group_cap / 256);
   dfree(m, &m->roff, m->ray_cap);
   dfree(m, &m->first_ray, m->chunk_cap);
   dfree(m, &m->tbl, (uint64_t)m->tbl_n * (m->tbl_n + 1) / 2);
@@ -2340,6 +2284,7 @@ void vdbgpu_destroy(vdbgpu_map* m) {
   if (m->h_st) (void)hipHostFree(m->h_st);
   drop_cast_graphs(m);
   if (m->d_dest) (void)hipFree(m->d_dest);
+  if (m->d_rcnt) (void)hipFree(m->d_rcnt);
   if (m->h_cst) (void)hipHostFree(m->h_cst);
   for (hipEvent_t e : m->cst_done)
     if (e) (void)hipEventDestroy(e);

@@ -622,8 +622,10 @@ __global__ __launch_bounds__(256) void k_section_prep(const int* __restrict__ or
 
 // evalActiveVoxelBoundingBox: min / max voxel coordinate of the active
 // voxels, folded into box[0..2] (atomicMin) and box[3..5] (atomicMax). One
-// lane per (leaf, word).
+// lane per (leaf, word); one atomic per workgroup and side, and only when it
+// still moves that side.
 __global__ __launch_bounds__(256) void k_active_bbox(MapView mp, uint32_t leaf_count, int* box) {
+  __shared__ int s_box[4][6];
   const uint64_t G = (uint64_t)gridDim.x * blockDim.x;
   int lo[3] = {INT_MAX, INT_MAX, INT_MAX}, hi[3] = {INT_MIN, INT_MIN, INT_MIN};
   for (uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; t < (uint64_t)leaf_count * 8; t += G) {
@@ -647,18 +649,151 @@ __global__ __launch_bounds__(256) void k_active_bbox(MapView mp, uint32_t leaf_c
     hi[2] = max(hi[2], o[2] + 31 - __builtin_clz(cols));
   }
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
+  for (int o = 1; o < 64; o <<= 1) {
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
       lo[a] = min(lo[a], __shfl_xor(lo[a], o, 64));
       hi[a] = max(hi[a], __shfl_xor(hi[a], o, 64));
     }
   }
-  if (lane_id() == 0 && lo[0] != INT_MAX) {
+  if (lane_id() == 0) {
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-      atomicMin(&box[a], lo[a]);
-      atomicMax(&box[3 + a], hi[a]);
+      s_box[threadIdx.x >> 6][a] = lo[a];
+      s_box[threadIdx.x >> 6][3 + a] = hi[a];
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x < 6) {
+    const int a = threadIdx.x;
+    int v = s_box[0][a];
+    for (int w = 1; w < 4; ++w) v = a < 3 ? min(v, s_box[w][a]) : max(v, s_box[w][a]);
+    const int cur = __hip_atomic_load(&box[a], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (a < 3 ? v < cur : v > cur) {
+      if (a < 3)
+        atomicMin(&box[a], v);
+      else
+        atomicMax(&box[a], v);
+    }
+  }
+}
+
+// Active points of the map (saveMapToPCD, VM:218-256) in OpenVDB's
+// cbeginValueOn order, on the device.
+//
+// Position of a leaf in that order: root children by origin, then 128^3 nodes
+// and leaves by offset, all x-major; 12 + 5 + 4 bits per axis of its biased
+// leaf coordinates, most significant level first.
+__device__ __forceinline__ uint64_t tree_order(const int o[3]) {
+  uint32_t u[3];
+#pragma unroll
+  for (int a = 0; a < 3; ++a) u[a] = (uint32_t)((o[a] >> 3) + (1 << 20));
+  uint64_t k = 0;
+#pragma unroll
+  for (int a = 0; a < 3; ++a) k = k << 12 | (u[a] >> 9);
+#pragma unroll
+  for (int a = 0; a < 3; ++a) k = k << 5 | ((u[a] >> 4) & 31u);
+#pragma unroll
+  for (int a = 0; a < 3; ++a) k = k << 4 | (u[a] & 15u);
+  return k;
+}
+
+// Leaves with an active value, their order keys and counts; cbeginValueOn
+// yields an active tile once, at its origin (an inactive one not at all).
+__global__ __launch_bounds__(256) void k_point_leaves(MapView mp, const Status* __restrict__ stmap, TileView tv,
+                                                      uint64_t* __restrict__ keys, uint32_t* __restrict__ cnt,
+                                                      uint32_t* __restrict__ idx, Status* st) {
+  __shared__ uint32_t s_wave[4], s_base;
+  __shared__ unsigned long long s_sum[4];
+  const uint32_t leaf_count = stmap->leaf_count;
+  const uint32_t G = gridDim.x * blockDim.x;
+  unsigned long long sum = 0;
+  for (uint32_t base = blockIdx.x * blockDim.x; base < leaf_count; base += G) {
+    const uint32_t i = base + threadIdx.x;
+    uint32_t c = 0;
+    if (i < leaf_count) {
+      const unsigned long long* w = mp.active + (size_t)i * 8;
+      if (tile_at(tv, i)) {
+        c = (uint32_t)(w[0] & 1u);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) c += (uint32_t)__popcll(w[j]);
+      }
+    }
+    const uint32_t pos = block_append(c != 0, &st->entries, s_wave, &s_base);
+    if (c) {
+      int o[3];
+      key_origin(mp.leaf_keys[i], o);
+      keys[pos] = tree_order(o);
+      cnt[pos] = c;
+      idx[pos] = i;
+      sum += c;
+    }
+  }
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) sum += __shfl_xor(sum, o, 64);
+  if (lane_id() == 0) s_sum[threadIdx.x >> 6] = sum;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    sum = s_sum[0] + s_sum[1] + s_sum[2] + s_sum[3];
+    if (sum) atomicAdd(&st->total, sum);
+  }
+}
+
+// First point of each listed leaf: the counts of the leaves before it, by
+// comparing it with all of them (slice blockIdx.y of the list, 256 at a time
+// in LDS). n^2 compares, but a list of 32,768 leaves takes 60 us and needs no
+// sort; the host takes over above kMaxPointLeaves.
+__global__ __launch_bounds__(256) void k_point_offsets(const uint64_t* __restrict__ keys,
+                                                       const uint32_t* __restrict__ cnt, uint32_t n,
+                                                       unsigned long long* off) {
+  __shared__ uint64_t s_key[256];
+  __shared__ uint32_t s_cnt[256];
+  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+  const uint64_t mine = i < n ? keys[i] : 0;
+  unsigned long long sum = 0;
+  for (uint32_t base = blockIdx.y * 256u; base < n; base += gridDim.y * 256u) {
+    __syncthreads();
+    const uint32_t j = base + threadIdx.x;
+    s_key[threadIdx.x] = j < n ? keys[j] : ~0ull;  // after every key
+    s_cnt[threadIdx.x] = j < n ? cnt[j] : 0u;
+    __syncthreads();
+    uint32_t part = 0;  // <= 256 * 512
+#pragma unroll 8
+    for (int k = 0; k < 256; ++k) part += s_key[k] < mine ? s_cnt[k] : 0u;
+    sum += part;
+  }
+  if (i < n && sum) atomicAdd(&off[i], sum);
+}
+
+// One wave per listed leaf: the centres of its active voxels, in offset order.
+__global__ __launch_bounds__(256) void k_point_rows(MapView mp, TileView tv, const uint32_t* __restrict__ idx,
+                                                    const unsigned long long* __restrict__ off, uint32_t n, double res,
+                                                    float* __restrict__ xyz) {
+  const uint32_t waves = gridDim.x * (blockDim.x >> 6);
+  const int lane = lane_id();
+  for (uint32_t i = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); i < n; i += waves) {
+    const uint32_t L = idx[i];
+    uint32_t row = (uint32_t)(mp.active[(size_t)L * 8 + (lane >> 3)] >> ((lane & 7) * 8)) & 0xFFu;
+    if (tile_at(tv, L)) row = lane == 0 ? row & 1u : 0u;
+    uint32_t v = (uint32_t)__popc(row);
+    const uint32_t c = v;
+#pragma unroll
+    for (int s = 1; s < 64; s <<= 1) {
+      const uint32_t t = __shfl_up(v, s, 64);
+      if (lane >= s) v += t;
+    }
+    int o[3];
+    key_origin(mp.leaf_keys[L], o);
+    float* p = xyz + 3 * (off[i] + v - c);
+    for (uint32_t r = row; r; r &= r - 1) {
+      const int q[3] = {o[0] + (lane >> 3), o[1] + (lane & 7), o[2] + __builtin_ctz(r)};
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        double w = (double)q[a] * res;  // indexToWorld (ScaleMap::applyMap)
+        w += 0.5 * res;
+        *p++ = (float)w;
+      }
     }
   }
 }
@@ -678,24 +813,30 @@ __global__ __launch_bounds__(256) void k_box_keys(int lx, int ly, int lz, uint32
 }
 
 // The background of createMapFromPointCloud: inside the box, every inactive
-// voxel of the leaves eidx[i] gets value v (its state stays off). One lane
-// per (leaf, word).
+// voxel of the leaves eidx[i] gets value v (its state stays off). One wave per
+// leaf, eight voxels per lane as two float4 where all of them are written (the
+// usual leaf): one lane per word, storing voxel by voxel, took 84 us for 32,000
+// leaves.
 __global__ __launch_bounds__(256) void k_box_fill(const unsigned long long* __restrict__ keys,
                                                   const uint32_t* __restrict__ eidx, uint32_t n, const int* box,
                                                   MapView mp, float v) {
-  const uint64_t G = (uint64_t)gridDim.x * blockDim.x;
-  for (uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; t < (uint64_t)n * 8; t += G) {
-    const uint32_t i = (uint32_t)(t >> 3);
-    const int j = (int)(t & 7);
+  const uint32_t waves = gridDim.x * (blockDim.x >> 6);
+  const int lane = lane_id();
+  for (uint32_t i = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); i < n; i += waves) {
     const uint32_t idx = eidx[i];
     if (idx == kNone) continue;
     int o[3];
     key_origin(keys[i], o);
-    const uint64_t m = box_word(o, box, j) & ~(uint64_t)mp.active[(size_t)idx * 8 + j];
-    if (!m) continue;
-    float* pv = mp.values + (size_t)idx * 512 + j * 64;
-    for (uint64_t b = m; b; b &= b - 1) pv[__builtin_ctzll(b)] = v;
-    mp.dirty[idx] = 1;
+    const uint32_t act = (uint32_t)(mp.active[(size_t)idx * 8 + (lane >> 3)] >> ((lane & 7) * 8)) & 0xFFu;
+    const uint32_t m = box_row(o, box, lane >> 3, lane & 7) & ~act;
+    float* pv = mp.values + (size_t)idx * 512 + lane * 8;
+    if (m == 0xFFu) {
+      reinterpret_cast<float4*>(pv)[0] = make_float4(v, v, v, v);
+      reinterpret_cast<float4*>(pv)[1] = make_float4(v, v, v, v);
+    } else {
+      for (uint32_t b = m; b; b &= b - 1) pv[__builtin_ctz(b)] = v;
+    }
+    if (__ballot(m != 0) != 0 && lane == 0) mp.dirty[idx] = 1;
   }
 }
 
@@ -816,7 +957,7 @@ hipError_t launch_section_prep(hipStream_t s, const int* origins, const float* v
 
 hipError_t launch_active_bbox(hipStream_t s, MapView mp, uint32_t leaf_count, int* box) {
   if (leaf_count == 0) return hipSuccess;
-  const int grid = (int)std::min<uint64_t>(4096, ((uint64_t)leaf_count * 8 + 255) / 256);
+  const int grid = (int)std::min<uint64_t>(1024, ((uint64_t)leaf_count * 8 + 255) / 256);
   hipLaunchKernelGGL(k_active_bbox, dim3(grid), dim3(256), 0, s, mp, leaf_count, box);
   return hipGetLastError();
 }
@@ -834,8 +975,29 @@ hipError_t launch_box_keys(hipStream_t s, const int lo[3], const uint32_t dims[3
 hipError_t launch_box_fill(hipStream_t s, const unsigned long long* keys, const uint32_t* eidx, uint32_t n,
                            const int* box, MapView mp, float v) {
   if (n == 0) return hipSuccess;
-  const int grid = (int)std::min<uint64_t>(8192, ((uint64_t)n * 8 + 255) / 256);
+  const int grid = (int)std::min<uint32_t>(8192, (n + 3) / 4);
   hipLaunchKernelGGL(k_box_fill, dim3(grid), dim3(256), 0, s, keys, eidx, n, box, mp, v);
+  return hipGetLastError();
+}
+
+hipError_t launch_point_leaves(hipStream_t s, MapView mp, uint64_t leaf_bound, const Status* stmap, TileView tv,
+                               uint64_t* keys, uint32_t* cnt, uint32_t* idx, Status* st) {
+  const int grid = (int)std::min<uint64_t>(2048, (leaf_bound + 255) / 256 + 1);
+  hipLaunchKernelGGL(k_point_leaves, dim3(grid), dim3(256), 0, s, mp, stmap, tv, keys, cnt, idx, st);
+  return hipGetLastError();
+}
+
+hipError_t launch_points(hipStream_t s, MapView mp, TileView tv, const uint64_t* keys, const uint32_t* cnt,
+                         const uint32_t* idx, uint32_t n, unsigned long long* off, double res, float* xyz) {
+  if (n == 0) return hipSuccess;
+  const uint32_t nb = (n + 255) / 256;
+  hipError_t e = launch_fill_u64(s, off, n, 0);
+  if (e != hipSuccess) return e;
+  // slices: about four workgroups per CU
+  const uint32_t slices = std::max(1u, std::min(nb, 1024u / nb));
+  hipLaunchKernelGGL(k_point_offsets, dim3(nb, slices), dim3(256), 0, s, keys, cnt, n, off);
+  if ((e = hipGetLastError()) != hipSuccess) return e;
+  hipLaunchKernelGGL(k_point_rows, dim3(std::min(8192u, (n + 3) / 4)), dim3(256), 0, s, mp, tv, idx, off, n, res, xyz);
   return hipGetLastError();
 }
 

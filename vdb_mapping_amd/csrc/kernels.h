@@ -117,6 +117,12 @@ hipError_t launch_section_cells(hipStream_t s, MapView mp, const SectionBox& sb,
 hipError_t launch_section_rows(hipStream_t s, MapView mp, const SectionBox& sb, uint32_t cells, bool full,
                                const uint32_t* cell, const uint64_t* boff, uint32_t cap, int* origins, float* values,
                                unsigned long long* masks);
+// Active points in value-on order (edit_kernels.hip): the leaves that hold some (st->entries of them, st->total
+// points), then the points.
+hipError_t launch_point_leaves(hipStream_t s, MapView mp, uint64_t leaf_bound, const Status* stmap, TileView tv,
+                               uint64_t* keys, uint32_t* cnt, uint32_t* idx, Status* st);
+hipError_t launch_points(hipStream_t s, MapView mp, TileView tv, const uint64_t* keys, const uint32_t* cnt,
+                         const uint32_t* idx, uint32_t n, unsigned long long* off, double res, float* xyz);
 hipError_t launch_scan_u64(hipStream_t s, const uint64_t* in, uint64_t* out, uint32_t n, unsigned int* total);
 hipError_t launch_raytrace(hipStream_t s, int num_cu, RtView rt, MapView mp, double inv, double res,
                            int64_t n, const double* origins, const double* dirs,

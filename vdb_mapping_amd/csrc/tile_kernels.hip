@@ -2,7 +2,7 @@
 // tolerance 0) at the leaf level, and of the rule that turns a tile back into a
 // leaf.
 //
-//   k_prune       one wave per pool leaf: a leaf whose 512 values compare equal
+//   k_prune       32 pool leaves per workgroup: a leaf whose 512 values compare equal
 //                 and whose voxels are all on or all off becomes a tile of that
 //                 value and state (bit in tv.bits / tv.on, value in tv.val) and
 //                 is appended to the tile list
@@ -37,20 +37,41 @@ __device__ __forceinline__ bool leaf_uniform(const MapView& mp, uint32_t L, floa
 
 }  // namespace
 
+// One workgroup per 32 leaves (a word of the tile bits), eight per wave: their
+// bits are gathered in LDS, so a word costs two plain stores and one append. A
+// bit, a state and an append atomic per tile ran one after another: 295 us for
+// the 32,000 background leaves of a room.
 __global__ __launch_bounds__(256) void k_prune(MapView mp, uint32_t leaf_count, TileView tv,
                                                uint32_t* __restrict__ list, unsigned int* counter) {
-  const uint32_t waves = gridDim.x * (blockDim.x >> 6);
-  for (uint32_t L = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); L < leaf_count; L += waves) {
-    const uint64_t w0 = mp.active[(size_t)L * 8];
-    if (w0 != 0 && w0 != ~0ull) continue;
-    const float v0 = mp.values[(size_t)L * 512];
-    if (!leaf_uniform(mp, L, v0, w0)) continue;
-    if (__lane_id() == 0) {
-      atomicOr(&tv.bits[L >> 5], 1u << (L & 31));
-      if (w0) atomicOr(&tv.on[L >> 5], 1u << (L & 31));
-      tv.val[L] = v0;
-      list[atomicAdd(counter, 1u)] = L;
+  __shared__ uint32_t s_bits, s_on, s_base;
+  for (uint32_t word = blockIdx.x; (uint64_t)word * 32 < leaf_count; word += gridDim.x) {
+    if (threadIdx.x == 0) s_bits = s_on = 0;
+    __syncthreads();
+#pragma unroll
+    for (uint32_t k = 0; k < 8; ++k) {
+      const uint32_t q = (threadIdx.x >> 6) * 8 + k, L = word * 32 + q;
+      if (L >= leaf_count) continue;  // the whole wave
+      const uint64_t w0 = mp.active[(size_t)L * 8];
+      if (w0 != 0 && w0 != ~0ull) continue;
+      const float v0 = mp.values[(size_t)L * 512];
+      if (!leaf_uniform(mp, L, v0, w0)) continue;
+      if (__lane_id() == 0) {
+        atomicOr(&s_bits, 1u << q);
+        if (w0) atomicOr(&s_on, 1u << q);
+        tv.val[L] = v0;
+      }
     }
+    __syncthreads();
+    const uint32_t bits = s_bits;
+    if (threadIdx.x == 0) {
+      tv.bits[word] = bits;
+      tv.on[word] = s_on;
+      s_base = bits ? atomicAdd(counter, (unsigned int)__popc(bits)) : 0u;
+    }
+    __syncthreads();
+    if (threadIdx.x < 32 && ((bits >> threadIdx.x) & 1u))
+      list[s_base + __popc(bits & ((1u << threadIdx.x) - 1))] = word * 32 + threadIdx.x;
+    __syncthreads();
   }
 }
 
@@ -72,7 +93,7 @@ __global__ __launch_bounds__(256) void k_tile_check(MapView mp, const uint32_t* 
 hipError_t launch_prune(hipStream_t s, MapView mp, uint32_t leaf_count, TileView tv, uint32_t* list,
                         unsigned int* counter) {
   if (leaf_count == 0) return hipSuccess;
-  const int grid = (int)std::min<uint32_t>(8192, (leaf_count + 3) / 4);
+  const int grid = (int)std::min<uint32_t>(8192, (leaf_count + 31) / 32);
   hipLaunchKernelGGL(k_prune, dim3(grid), dim3(256), 0, s, mp, leaf_count, tv, list, counter);
   return hipGetLastError();
 }

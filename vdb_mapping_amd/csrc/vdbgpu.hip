@@ -33,6 +33,7 @@ namespace {
 constexpr uint32_t kMaxTableN = 8192;       // longest per-axis ray extent in voxels
 constexpr uint32_t kMinUpdateCap = 1u << 12;
 constexpr uint32_t kMaxRays = 1u << 30;
+constexpr uint32_t kMaxPointLeaves = 1u << 19;  // leaves with active voxels that are ordered on the device
 constexpr int64_t kBrickAccumulateRays = 1 << 22;
 // Rays per squared voxel of range from which an accumulated cloud takes the
 // brick path. Three clouds and their integrate, brick against hash traversal:
@@ -233,6 +234,15 @@ struct vdbgpu_map {
   unsigned int* ngroups = nullptr;
   double* tbl = nullptr;
   uint32_t tbl_n = 0;
+  // export of the active points: listed leaves (order key, count, pool index,
+  // first point) and the points
+  uint64_t* pt_key = nullptr;
+  uint32_t* pt_cnt = nullptr;
+  uint32_t* pt_idx = nullptr;
+  unsigned long long* pt_off = nullptr;
+  uint64_t pt_cap = 0;
+  float* pt_xyz = nullptr;
+  uint64_t pt_xyz_cap = 0;
   // map sections by cells: cell table and its block sums, and the pinned
   // staging buffer that the section's leaves are written to
   uint32_t* sec_cell = nullptr;
@@ -292,6 +302,16 @@ namespace {
     if (e_ != hipSuccess) {                                                      \
       m->last_error = std::string(#expr) + ": " + hipGetErrorString(e_);         \
       return VDBGPU_DEVICE_ERROR;                                                \
+    }                                                                            \
+  } while (0)
+
+// CK for the exports: a HIP error returns -1.
+#define CKN(expr)                                                                \
+  do {                                                                           \
+    hipError_t e_ = (expr);                                                      \
+    if (e_ != hipSuccess) {                                                      \
+      m->last_error = std::string(#expr) + ": " + hipGetErrorString(e_);         \
+      return -1;                                                                 \
     }                                                                            \
   } while (0)
 
@@ -2050,6 +2070,11 @@ uint64_t walk_scratch(vdbgpu_map* m, bool release) {
   one(m->gneed, m->gcap);
   one(m->glist, m->gcap);
   one(m->gidx, m->gcap);
+  one(m->pt_key, m->pt_cap);
+  one(m->pt_cnt, m->pt_cap);
+  one(m->pt_idx, m->pt_cap);
+  one(m->pt_off, m->pt_cap);
+  one(m->pt_xyz, m->pt_xyz_cap);
   one(m->sec_cell, m->sec_cells);
   one(m->sec_sums, (size_t)m->sec_cells / kSectionCells * 2);
   one(m->q_in, (size_t)m->q_cap * 7);
@@ -2068,6 +2093,7 @@ uint64_t walk_scratch(vdbgpu_map* m, bool release) {
     if (m->h_sec) (void)hipHostFree(m->h_sec);
     m->h_sec = nullptr;
     m->sec_cells = m->sec_cap = 0;
+    m->pt_cap = m->pt_xyz_cap = 0;
     m->points_bytes = 0;
     m->ray_cap = 0;
     m->chunk_cap = 0;
@@ -2267,6 +2293,11 @@ void vdbgpu_destroy(vdbgpu_map* m) {
   dfree(m, &m->q_in, (size_t)m->q_cap * 7);
   dfree(m, &m->q_succ, (size_t)m->q_cap);
   dfree(m, &m->q_end, (size_t)m->q_cap * 3);
+  dfree(m, &m->pt_key, m->pt_cap);
+  dfree(m, &m->pt_cnt, m->pt_cap);
+  dfree(m, &m->pt_idx, m->pt_cap);
+  dfree(m, &m->pt_off, m->pt_cap);
+  dfree(m, &m->pt_xyz, m->pt_xyz_cap);
   dfree(m, &m->sec_cell, m->sec_cells);
   dfree(m, &m->sec_sums, (size_t)m->sec_cells / kSectionCells * 2);
   if (m->h_sec) (void)hipHostFree(m->h_sec);
@@ -3148,7 +3179,42 @@ int64_t vdbgpu_export_active_points(vdbgpu_map* m, float* xyz, int64_t cap) {
   if (!m) return -1;
   Guard g(m);
   if (g.rc) return -1;
-  if (hipStreamSynchronize(m->cast) != hipSuccess || read_status(m)) return -1;
+  const uint64_t bound = m->leaf_count_ub;
+  if (bound == 0) return 0;
+  if (bound > m->pt_cap) {
+    dfree(m, &m->pt_key, m->pt_cap);
+    dfree(m, &m->pt_cnt, m->pt_cap);
+    dfree(m, &m->pt_idx, m->pt_cap);
+    dfree(m, &m->pt_off, m->pt_cap);
+    m->pt_cap = 0;
+    CKN(dalloc(m, &m->pt_key, bound));
+    CKN(dalloc(m, &m->pt_cnt, bound));
+    CKN(dalloc(m, &m->pt_idx, bound));
+    CKN(dalloc(m, &m->pt_off, bound));
+    m->pt_cap = bound;
+  }
+  CKN(launch_zero_words(m->stream, (unsigned long long*)&m->d_st[2], sizeof(Status) / 8));
+  CKN(launch_point_leaves(m->stream, map_view(m), bound, &m->d_st[1], tile_view(m), m->pt_key, m->pt_cnt, m->pt_idx,
+                          &m->d_st[2]));
+  if (read_status(m)) return -1;
+  const uint32_t listed = m->h_st[2].entries;
+  const int64_t points = (int64_t)m->h_st[2].total;
+  if (!xyz) return points;
+  if (points > cap) return -points;
+  if (points == 0) return 0;
+  if (listed <= kMaxPointLeaves) {
+    if ((uint64_t)points * 3 > m->pt_xyz_cap) {
+      dfree(m, &m->pt_xyz, m->pt_xyz_cap);
+      m->pt_xyz_cap = 0;
+      CKN(dalloc(m, &m->pt_xyz, (uint64_t)points * 3));
+      m->pt_xyz_cap = (uint64_t)points * 3;
+    }
+    CKN(launch_points(m->stream, map_view(m), tile_view(m), m->pt_key, m->pt_cnt, m->pt_idx, listed, m->pt_off,
+                      m->res, m->pt_xyz));
+    CKN(hipMemcpyAsync(xyz, m->pt_xyz, (size_t)points * 12, hipMemcpyDeviceToHost, m->stream));
+    CKN(hipStreamSynchronize(m->stream));
+    return points;
+  }
   const uint32_t n = m->h_st[1].leaf_count;
   std::vector<unsigned long long> keys(n), act((size_t)n * 8);
   if (n && (hipMemcpy(keys.data(), m->leaf_keys, n * sizeof(unsigned long long), hipMemcpyDeviceToHost) ||
@@ -3331,16 +3397,6 @@ int32_t vdbgpu_restore_map_integrity(vdbgpu_map* m) {
   if (g.rc) return g.rc;
   return restore_integrity(m);
 }
-
-// CK for the exports: a HIP error returns -1.
-#define CKN(expr)                                                                \
-  do {                                                                           \
-    hipError_t e_ = (expr);                                                      \
-    if (e_ != hipSuccess) {                                                      \
-      m->last_error = std::string(#expr) + ": " + hipGetErrorString(e_);         \
-      return -1;                                                                 \
-    }                                                                            \
-  } while (0)
 
 int64_t vdbgpu_export_artificial(vdbgpu_map* m, int32_t* origins, uint64_t* masks, int64_t cap) {
   if (!m) return -1;

@@ -45,14 +45,34 @@ VDB_HD bool ev_before(const double* __restrict__ tbl, int b, uint32_t nb, uint32
   return fb < fa || (fb == fa && b > a);
 }
 
+// Quotient (and remainder r) of X by n, exact, with inv = 1.0f / n at hand: for
+// quotients up to 2^15 the float product is within 2^15 * 2^-21 of X / n (the
+// roundings of X, of inv, on the device one unit in the last place, and of the
+// product), so its floor is off by one at most and the remainder says which
+// way. Ten instructions; the division they stand for takes more than twice as
+// many, and the brick cut makes four of them per segment.
+VDB_HD uint32_t div_by(uint32_t X, uint32_t n, float inv, uint32_t& r) {
+  uint32_t q = (uint32_t)((float)X * inv);
+  int32_t d = (int32_t)(X - q * n);
+  if (d < 0) {
+    --q;
+    d += (int32_t)n;
+  } else if (d >= (int32_t)n) {
+    ++q;
+    d -= (int32_t)n;
+  }
+  r = (uint32_t)d;
+  return q;
+}
+
 // Number of axis-b crossings (b has |delta| nb) that precede event (a, ca):
 // #{c : (2c+1) na < (2ca+1) nb} plus the rational tie, if any, when the
-// tie-break puts it first.
+// tie-break puts it first. inv_na = 1.0f / na.
 VDB_HD uint32_t count_before(const double* __restrict__ tbl, int b, uint32_t nb, int a, uint32_t na,
-                             uint32_t ca) {
+                             uint32_t ca, float inv_na) {
   if (nb == 0) return 0;
-  const uint32_t X = (2 * ca + 1) * nb;  // < 2^28
-  const uint32_t q = X / na, r = X - q * na;
+  uint32_t r;
+  const uint32_t q = div_by((2 * ca + 1) * nb, na, inv_na, r);  // < 2^28, quotient < 2 nb + 1
   uint32_t cnt = r == 0 ? q / 2 : (q + 1) / 2;
   if (cnt > nb) cnt = nb;
   if (r == 0 && (q & 1)) {
@@ -217,16 +237,20 @@ struct SegEnum {
   uint32_t cur[3];     // crossing counts at the current segment's first visit
   uint32_t nxt[3];     // next brick-boundary crossing index per axis (kNoCross: none)
   uint32_t G[3];       // global step index of that crossing
+  uint32_t p1[3], p2[3];  // crossings of the other two axes before it
+  float inv[3];        // 1 / n
   uint32_t g0;         // first visit of the current segment
   uint32_t cnt;
   bool done;
 
-  // Global step index of crossing nxt[a] of axis a (a is a constant after
+  // Global step index of crossing nxt[a] of axis a, with the other axes' counts
+  // before it, which are what `take` needs when it comes (a is a constant after
   // unrolling: the state stays in registers).
-  VDB_HD uint32_t event_index(const double* __restrict__ tbl, int a) const {
+  VDB_HD uint32_t event_index(const double* __restrict__ tbl, int a) {
     const int o1 = a == 0 ? 1 : 0, o2 = a == 2 ? 1 : 2;
-    return 1 + nxt[a] + count_before(tbl, o1, n[o1], a, n[a], nxt[a]) +
-           count_before(tbl, o2, n[o2], a, n[a], nxt[a]);
+    p1[a] = count_before(tbl, o1, n[o1], a, n[a], nxt[a], inv[a]);
+    p2[a] = count_before(tbl, o2, n[o2], a, n[a], nxt[a], inv[a]);
+    return 1 + nxt[a] + p1[a] + p2[a];
   }
   // Step past the brick crossing of axis A: crossing counts after it (axis A
   // made crossing nxt[A], the others theirs before it), brick, next crossing.
@@ -234,8 +258,8 @@ struct SegEnum {
   VDB_HD void take(const double* __restrict__ tbl) {
     constexpr int O1 = A == 0 ? 1 : 0, O2 = A == 2 ? 1 : 2;
     const uint32_t ca = nxt[A];
-    cur[O1] = count_before(tbl, O1, n[O1], A, n[A], ca);
-    cur[O2] = count_before(tbl, O2, n[O2], A, n[A], ca);
+    cur[O1] = p1[A];
+    cur[O2] = p2[A];
     cur[A] = ca + 1;
     b[A] += step[A];
     nxt[A] = ca + kBrickDim < n[A] ? ca + kBrickDim : kNoCross;
@@ -253,6 +277,7 @@ struct SegEnum {
       step[a] = d > 0 ? 1 : (d < 0 ? -1 : 0);
       b[a] = (count == 0 ? e[a] : s[a]) >> kBrickLog;
       cur[a] = 0;
+      inv[a] = n[a] ? 1.0f / (float)n[a] : 0.0f;
       const uint32_t lo = (uint32_t)s[a] & (kBrickDim - 1);
       // crossing index whose step enters the next brick along this axis
       const uint32_t first = step[a] > 0 ? (kBrickDim - 1) - lo : lo;

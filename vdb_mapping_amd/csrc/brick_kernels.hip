@@ -49,12 +49,11 @@ constexpr int kLdsBricks = kSegTab;  // per-workgroup brick aggregation table
 constexpr int kLdsBrickProbe = 32;
 constexpr uint32_t kMaxBrickProbe = 512;
 constexpr int kBrickWords = 1024;  // 64 leaves x (8 visited + 8 hit) words
-// The walk's LDS bitmap: [0, 512) visited words of layout X, [512, 1024) hit
-// words (leaf-major, as emitted), [1024, 1536) layout Y, [1536, 2048) layout Z.
-// A segment marks its voxels in the layout whose word axis it steps along
-// least (see walk_segment); the layouts are merged into leaf-major visited
-// words before the records are written.
-constexpr int kWalkWords = 2048;
+// The walk's LDS bitmap: one 32-bit word per (x, y) row of the brick, bit z,
+// rows of a plane 33 words apart so that the rows of a column do not share a
+// bank. Merged into leaf-major visited words before the records are written.
+constexpr int kWalkPlane = 33;
+constexpr int kWalkWords = 32 * kWalkPlane;
 
 __device__ __forceinline__ int bw_lane() { return (int)__lane_id(); }
 
@@ -400,30 +399,35 @@ __global__ __launch_bounds__(256) void k_seg_fill(const int4* __restrict__ rayin
   }
 }
 
-// Walk one segment record into the brick bitmap `bits`.
+// Walk one segment record into the brick's rows `vis` (and its end voxel into
+// the leaf-major hit words).
 //
-// Word layouts: a segment's voxels go into the layout whose word axis A is
-// the axis it steps along least, so most steps stay inside one 64-bit word
-// and the word is OR-ed into LDS only when the walk leaves it. With (a, b, c)
-// the voxel's brick-local coordinates along (A, B, C) -- (x, y, z) for layout
-// X, (y, x, z) for Y, (z, x, y) for Z -- the word is a * 16 + (b >> 3) * 4 +
-// (c >> 3) and the bit (b & 7) * 8 + (c & 7). The walk state is one packed
-// code u = a << 12 | b << 6 | c (6-bit fields; bit 5 of a field is a guard: a
-// field that leaves [0, 31] sets it, and the OR of every code is checked at
-// the end), stepped by one add per visit. The path is monotone along every
-// axis, so it stays inside the brick when no field ever left it.
+// The walk state is one code u = (x * 33 + y) * 32 + z of the brick-local
+// voxel, stepped by one add per visit: u >> 5 is the row's word, the low five
+// bits of u its bit, so a visit is an OR of 1 << z into LDS. The loop is bound
+// by VALU issue, and this is the least of it found: gathering the bits of a
+// 64-bit word in registers and OR-ing it when the walk left it (in three
+// layouts, each segment in the one whose words it left least) saved LDS
+// operations but cost the loop some fifteen more instructions (a 262,144-ray
+// outdoor scan alone: 496 us, now 390).
+// The word index is clamped to the bitmap. The path is monotone along every
+// axis, so it stayed inside the brick exactly when the end lies where m - 1
+// steps of the right signs lead (a field that left [0, 31] has carried into
+// the next: its apparent step then has the wrong sign or the steps the wrong
+// sum).
 //
 // The step order is the exact integer DDA of dda_math.h (signs of the three
 // pairwise differences); the rational-tie rule runs only when a lane of the
 // wave meets a tie, with the crossing counts recovered from the walk state.
-__device__ __forceinline__ uint32_t walk_word(uint32_t u) {
-  return ((u >> 8) & 0x1F0u) | ((u >> 7) & 0xCu) | ((u >> 3) & 3u);
+__device__ __forceinline__ void walk_voxel(uint32_t u, uint32_t& x, uint32_t& y, uint32_t& z) {
+  const uint32_t w = u >> 5;
+  x = (w * 1986u) >> 16;  // w / 33 for w < 1056
+  y = w - x * 33u;
+  z = u & 31u;
 }
-__device__ __forceinline__ uint32_t walk_bit(uint32_t u) { return ((u >> 3) & 0x38u) | (u & 7u); }
-constexpr uint32_t kWalkFields = 0x1F7DFu;  // the valid bits of a walk code
 
-__device__ __forceinline__ void walk_segment(const uint4 sr, const double* __restrict__ tbl,
-                                             unsigned long long* bits, uint32_t& used, Status* st) {
+__device__ __forceinline__ void walk_segment(const uint4 sr, const double* __restrict__ tbl, uint32_t* vis,
+                                             unsigned long long* hit, Status* st) {
   const uint32_t n0 = sr.x & 0x3FFFu, n1 = (sr.x >> 14) & 0x3FFFu, n2 = sr.y & 0x3FFFu;
   const uint32_t c00 = (sr.y >> 14) & 0x3FFFu, c10 = sr.z & 0x3FFFu, c20 = (sr.z >> 14) & 0x3FFFu;
   const uint32_t lx0 = sr.w & 31u, ly0 = (sr.w >> 5) & 31u, lz0 = (sr.w >> 10) & 31u;
@@ -431,35 +435,22 @@ __device__ __forceinline__ void walk_segment(const uint4 sr, const double* __res
   const int sgx = n0 == 0 ? 0 : (((sr.w >> 24) & 1u) ? -1 : 1);
   const int sgy = n1 == 0 ? 0 : (((sr.w >> 25) & 1u) ? -1 : 1);
   const int sgz = n2 == 0 ? 0 : (((sr.w >> 26) & 1u) ? -1 : 1);
-  // word axis: the one with the fewest steps
-  const int L = (n0 <= n1 && n0 <= n2) ? 0 : (n1 <= n2 ? 1 : 2);
-  used |= 1u << L;
-  const int shx = L == 0 ? 12 : 6, shy = L == 1 ? 12 : (L == 0 ? 6 : 0), shz = L == 2 ? 12 : 0;
-  uint32_t u = lx0 << shx | ly0 << shy | lz0 << shz;
-  const int ix = sgx * (1 << shx), iy = sgy * (1 << shy), iz = sgz * (1 << shz);
-  const uint32_t base = L == 0 ? 0u : (L == 1 ? 1024u : 1536u);
+  uint32_t u = (lx0 * kWalkPlane + ly0) * 32u + lz0;
+  const int ix = sgx * kWalkPlane * 32, iy = sgy * 32, iz = sgz;
   const int tn0 = 2 * (int)n0, tn1 = 2 * (int)n1, tn2 = 2 * (int)n2;
   int dyx = (int)((2 * c10 + 1) * n0) - (int)((2 * c00 + 1) * n1);
   int dzx = (int)((2 * c20 + 1) * n0) - (int)((2 * c00 + 1) * n2);
   int dzy = (int)((2 * c20 + 1) * n1) - (int)((2 * c10 + 1) * n2);
-  uint32_t esc = u, cw = walk_word(u);
-  uint64_t cb = 0;
   for (uint32_t k = 0;;) {
-    const uint32_t w = walk_word(u);
-    if (w != cw) {
-      atomicOr(&bits[base + cw], (unsigned long long)cb);
-      cw = w;
-      cb = 0;
-    }
-    cb |= 1ull << walk_bit(u);
+    atomicOr(&vis[min(u >> 5, (uint32_t)kWalkWords - 1)], 1u << (u & 31u));
     if (++k >= m) break;  // m == 0: the endpoint of a zero-length ray
     bool y = dyx < 0;
     const int dzm = y ? dzy : dzx;
     bool z = dzm < 0;
     if (__any(dyx == 0 || dzm == 0)) {
       // exact rule for every lane: crossing counts from the walk state
-      const uint32_t fa = (u >> 12) & 31u, fb = (u >> 6) & 31u, fc = u & 31u;
-      const uint32_t lx = L == 0 ? fa : fb, ly = L == 1 ? fa : (L == 0 ? fb : fc), lz = L == 2 ? fa : fc;
+      uint32_t lx, ly, lz;
+      walk_voxel(u, lx, ly, lz);
       IntDda t;
       t.n0 = n0, t.n1 = n1, t.n2 = n2;
       t.c0 = c00 + (uint32_t)abs((int)lx - (int)lx0);
@@ -476,49 +467,37 @@ __device__ __forceinline__ void walk_segment(const uint4 sr, const double* __res
     dzx += y ? 0 : (z ? tn0 : -tn2);
     dzy += x ? 0 : (z ? tn1 : -tn2);
     u += (uint32_t)(z ? iz : (y ? iy : ix));
-    esc |= u;
   }
-  atomicOr(&bits[base + cw], (unsigned long long)cb);
-  if (esc & ~kWalkFields) {
+  uint32_t lx, ly, lz;
+  walk_voxel(u, lx, ly, lz);
+  const int ex = ((int)lx - (int)lx0) * sgx, ey = ((int)ly - (int)ly0) * sgy, ez = ((int)lz - (int)lz0) * sgz;
+  if (u >> 5 >= (uint32_t)kWalkWords || ly > 31u || ex < 0 || ey < 0 || ez < 0 || ex + ey + ez != (int)max(m, 1u) - 1) {
     atomicOr(&st->error, kErrBrick);  // the scan is rejected
   } else if (sr.w & 0x80000000u) {
     // setValueOn(end, true) (VDBMapping.hpp:533-536): the last visit is the end voxel
-    const uint32_t fa = (u >> 12) & 31u, fb = (u >> 6) & 31u, fc = u & 31u;
-    const uint32_t lx = L == 0 ? fa : fb, ly = L == 1 ? fa : (L == 0 ? fb : fc), lz = L == 2 ? fa : fc;
     const uint32_t hw = ((lx >> 3) << 7) | ((ly >> 3) << 5) | ((lz >> 3) << 3) | (lx & 7u);
-    atomicOr(&bits[512 + hw], 1ull << (((ly & 7u) << 3) | (lz & 7u)));
+    atomicOr(&hit[hw], 1ull << (((ly & 7u) << 3) | (lz & 7u)));
   }
 }
 
-// Merge the layouts of the walk bitmap into leaf-major visited words at
-// [0, 512) (word j of leaf l at l * 8 + j, bit (y & 7) * 8 + (z & 7)); `used`
-// names the layouts any segment of the item marked. Called by the whole
-// workgroup (two words per thread); ends with a barrier.
-__device__ void merge_layouts(unsigned long long* bits, uint32_t used) {
-  uint64_t out[2];
+// The brick's rows as leaf-major visited words (word j of leaf l at l * 8 + j,
+// bit (y & 7) * 8 + (z & 7)). Called by the whole workgroup: a thread reads the
+// eight rows of one leaf plane and writes the words of two of the four leaves
+// along z; ends with a barrier.
+__device__ void merge_rows(const uint32_t* vis, unsigned long long* bits) {
+  const int t = (int)(threadIdx.x & 127u), half = (int)(threadIdx.x >> 7);
+  const int lx = t >> 5, j = (t >> 2) & 7, ly = t & 3;
+  const uint32_t* row = vis + (lx * 8 + j) * kWalkPlane + ly * 8;
+  uint64_t out0 = 0, out1 = 0;
 #pragma unroll
-  for (int r = 0; r < 2; ++r) {
-    const int q = (int)threadIdx.x + r * 256;
-    const int l = q >> 3, j = q & 7;
-    const int lx = l >> 4, ly = (l >> 2) & 3, lz = l & 3;
-    uint64_t v = (used & 1u) ? bits[(lx * 8 + j) * 16 + ly * 4 + lz] : 0ull;
-    if (used & 2u) {  // layout Y: byte j of the word at y = 8 ly + yy is byte yy here
-      const unsigned long long* p = bits + 1024 + (ly * 8) * 16 + lx * 4 + lz;
-#pragma unroll
-      for (int yy = 0; yy < 8; ++yy) v |= ((p[yy * 16] >> (8 * j)) & 0xFFull) << (8 * yy);
-    }
-    if (used & 4u) {  // layout Z: bit yy of byte j of the word at z = 8 lz + zz is bit 8 yy + zz here
-      const unsigned long long* p = bits + 1536 + (lz * 8) * 16 + lx * 4 + ly;
-      uint64_t mz = 0;
-#pragma unroll
-      for (int zz = 0; zz < 8; ++zz) mz |= ((p[zz * 16] >> (8 * j)) & 0xFFull) << (8 * zz);
-      v |= transpose8(mz);
-    }
-    out[r] = v;
+  for (int yy = 0; yy < 8; ++yy) {
+    const uint32_t w = row[yy] >> (16 * half);
+    out0 |= (uint64_t)(w & 0xFFu) << (8 * yy);
+    out1 |= (uint64_t)((w >> 8) & 0xFFu) << (8 * yy);
   }
-  __syncthreads();
-#pragma unroll
-  for (int r = 0; r < 2; ++r) bits[threadIdx.x + r * 256] = out[r];
+  unsigned long long* dst = bits + ((lx * 4 + ly) * 4 + 2 * half) * 8 + j;
+  dst[0] = out0;
+  dst[8] = out1;
   __syncthreads();
 }
 
@@ -534,12 +513,12 @@ __global__ __launch_bounds__(kWalkThreads, 8) void k_brick_walk(const BrickItem*
                                                              unsigned long long* __restrict__ shared_bits,
                                                              const RecDest* __restrict__ dest,
                                                              unsigned int* __restrict__ rcnt, Status* st) {
-  __shared__ unsigned long long bits[kWalkWords];
+  __shared__ unsigned long long bits[kBrickWords];
+  __shared__ uint32_t vis[kWalkWords];
   __shared__ uint32_t s_pos[64];
   __shared__ uint32_t s_hist[128];
   __shared__ uint16_t s_order[kItemSegs];
   __shared__ unsigned int s_stop;
-  __shared__ uint32_t s_used;
   if (stopped(st, &s_stop)) return;
   const uint32_t n_items = st->items;
   const RecDest d = *dest;
@@ -551,9 +530,9 @@ __global__ __launch_bounds__(kWalkThreads, 8) void k_brick_walk(const BrickItem*
     int b[3];
     brick_coords(bv.keys[item.slot], b);
     const int ox = b[0] * kBrickDim, oy = b[1] * kBrickDim, oz = b[2] * kBrickDim;
-    for (int w = t; w < kWalkWords; w += kWalkThreads) bits[w] = 0;
+    for (int w = t; w < kWalkWords; w += kWalkThreads) vis[w] = 0;
+    for (int w = t; w < 512; w += kWalkThreads) bits[512 + w] = 0;  // hits; the visited words are merged in
     if (t < 128) s_hist[t] = 0;
-    if (t == 0) s_used = 0;
     // Counting sort of the item's segments by visit count, longest first, so
     // the lanes of a wave walk segments of about the same length. Segment k
     // belongs to thread k % 256; its length is loaded once, for both passes.
@@ -592,7 +571,6 @@ __global__ __launch_bounds__(kWalkThreads, 8) void k_brick_walk(const BrickItem*
     // w takes the 64 of block (w + r) mod 4, so over the rounds every wave
     // walks long and short ones alike. The next round's record is loaded
     // before the current one is walked.
-    uint32_t used = 0;
     const uint32_t lane = t & 63u, wave = t >> 6;
     uint32_t k = (((wave + 0) & 3u) << 6) + lane;
     uint4 sr = k < nseg ? segs[item.seg0 + s_order[k]] : make_uint4(0, 0, 0, 0);
@@ -601,13 +579,12 @@ __global__ __launch_bounds__(kWalkThreads, 8) void k_brick_walk(const BrickItem*
       ++r;
       const uint32_t kn = r * kWalkThreads + (((wave + r) & 3u) << 6) + lane;
       const uint4 sn = kn < nseg ? segs[item.seg0 + s_order[kn]] : make_uint4(0, 0, 0, 0);
-      walk_segment(sr, tbl, bits, used, st);
+      walk_segment(sr, tbl, vis, bits + 512, st);
       k = kn;
       sr = sn;
     }
-    if (used) atomicOr(&s_used, used);
     __syncthreads();
-    merge_layouts(bits, s_used);
+    merge_rows(vis, bits);
     if (item.shared == kNone) {
       emit_leaves(bits, ox, oy, oz, d, it & (regions - 1), stride, rcnt, s_pos);
     } else {

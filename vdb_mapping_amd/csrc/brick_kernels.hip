@@ -231,11 +231,11 @@ __global__ __launch_bounds__(256) void k_seg_count(const int4* __restrict__ rayi
 
 // Per 256 slots: (work items << 32) | segments.
 __global__ __launch_bounds__(256) void k_brick_sums(BrickView bv, uint64_t* __restrict__ bsum,
-                                                    const Status* st) {
+                                                    uint32_t item_segs) {
   __shared__ uint64_t s_w[4];
   const uint32_t slot = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t c = bv.cnt[slot];
-  const uint64_t v = ((uint64_t)((c + kItemSegs - 1) / kItemSegs) << 32) | c;
+  const uint64_t v = ((uint64_t)((c + item_segs - 1) / item_segs) << 32) | c;
   const uint64_t t = block_sum_u64(v, s_w);
   if (threadIdx.x == 0) bsum[blockIdx.x] = t;
 }
@@ -280,11 +280,11 @@ __global__ __launch_bounds__(256) void k_brick_offsets(BrickView bv, const uint6
                                                        BrickItem* __restrict__ items,
                                                        uint32_t seg_cap, uint32_t item_cap,
                                                        uint32_t* __restrict__ split_slot,
-                                                       uint32_t split_cap, Status* st) {
+                                                       uint32_t split_cap, uint32_t item_segs, Status* st) {
   __shared__ uint64_t s_w[4];
   const uint32_t slot = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t c = bv.cnt[slot];
-  const uint32_t ni = (c + kItemSegs - 1) / kItemSegs;
+  const uint32_t ni = (c + item_segs - 1) / item_segs;
   const uint64_t x = ((uint64_t)ni << 32) | c;
   uint64_t v = x;
 #pragma unroll
@@ -319,8 +319,8 @@ __global__ __launch_bounds__(256) void k_brick_offsets(BrickView bv, const uint6
     split_slot[shared] = slot;
   }
   for (uint32_t j = 0; j < ni; ++j) {
-    const uint32_t a = seg0 + j * kItemSegs;
-    const uint32_t b = min(a + kItemSegs, seg0 + c);
+    const uint32_t a = seg0 + j * item_segs;
+    const uint32_t b = min(a + item_segs, seg0 + c);
     items[item0 + j] = BrickItem{slot, a, b, shared};
   }
 }
@@ -673,16 +673,16 @@ hipError_t launch_seg_count(hipStream_t s, int grid, const int4* rayinfo, const 
 
 hipError_t launch_brick_offsets(hipStream_t s, BrickView bv, uint64_t* bsum, uint64_t* boff,
                                 BrickItem* items, uint32_t seg_cap, uint32_t item_cap,
-                                uint32_t* split_slot, uint32_t split_cap, Status* st) {
+                                uint32_t* split_slot, uint32_t split_cap, uint32_t item_segs, Status* st) {
   const uint32_t nb = (bv.cap_mask + 1) / 256;
-  hipLaunchKernelGGL(k_brick_sums, dim3(nb), dim3(256), 0, s, bv, bsum, st);
+  hipLaunchKernelGGL(k_brick_sums, dim3(nb), dim3(256), 0, s, bv, bsum, item_segs);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(k_scan_u64, dim3(1), dim3(256), 0, s, bsum, boff, nb, &st->items, 32, &st->segs);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(k_brick_offsets, dim3(nb), dim3(256), 0, s, bv, boff, items, seg_cap, item_cap,
-                     split_slot, split_cap, st);
+                     split_slot, split_cap, item_segs, st);
   return hipGetLastError();
 }
 

@@ -501,14 +501,16 @@ __global__ __launch_bounds__(256) void k_compact(UpdView u, uint32_t cap,
 // modify op changes the tile's value or active state).
 // Random accesses bound it: with the leaf hash in groups of four (map_hash) an
 // outdoor scan's 1.7 M records take 44 us instead of 86. One record per lane:
-// two or four per lane left fewer waves to hide the probes (47 and 59 us).
-__global__ __launch_bounds__(kListBlockMax) void k_map_insert(UpdView u, const uint32_t* __restrict__ list,
+// two or four per lane left fewer waves to hide the probes (47 and 59 us), and
+// workgroups of 1,024 waited for a CU that the next scan's walk had left (225 us
+// beside it, 58 with 256).
+__global__ __launch_bounds__(256) void k_map_insert(UpdView u, const uint32_t* __restrict__ list,
                                                               RecIndex ri, uint32_t count, MapView mp,
                                                               uint32_t* __restrict__ eidx,
                                                               uint32_t create_hit, uint32_t create_miss,
                                                               unsigned long long* noop_set,
                                                               uint32_t noop_mask, Status* st) {
-  __shared__ uint32_t s_wave[kListBlockMax / 64], s_base;
+  __shared__ uint32_t s_wave[4], s_base;
   const uint32_t G = gridDim.x * blockDim.x;
   const uint32_t e0 = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t rounds = (count + G - 1) / G;
@@ -1112,7 +1114,7 @@ hipError_t launch_map_insert(hipStream_t s, UpdView u, const uint32_t* list, con
                              uint32_t* eidx, bool create_hit, bool create_miss,
                              unsigned long long* noop_set, uint32_t noop_mask, Status* st) {
   if (!count) return hipSuccess;
-  const int block = list_block(count);
+  const int block = 256;
   const int grid = (int)std::min<uint32_t>((1u << 20) / block, (count + block - 1) / block);
   hipLaunchKernelGGL(k_map_insert, dim3(grid), dim3(block), 0, s, u, list, ri, count, mp, eidx,
                      (uint32_t)create_hit, (uint32_t)create_miss, noop_set, noop_mask, st);

@@ -92,7 +92,8 @@ hipError_t launch_seg_count(hipStream_t s, int grid, const int4* rayinfo, const 
                             unsigned long long* wsc, Status* st);
 hipError_t launch_brick_offsets(hipStream_t s, BrickView bv, uint64_t* bsum, uint64_t* boff,
                                 BrickItem* items, uint32_t seg_cap, uint32_t item_cap,
-                                uint32_t* split_slot, uint32_t split_cap, Status* st);
+                                uint32_t* split_slot, uint32_t split_cap, uint32_t item_segs,
+                                Status* st);
 hipError_t launch_seg_fill(hipStream_t s, int grid, const int4* rayinfo, const ScanInfo* scans,
                            const BatchCtl* ctl, const double* tbl, BrickView bv,
                            const unsigned long long* wkey, const unsigned long long* wsc, uint4* segs,

@@ -1139,8 +1139,8 @@ int ensure_bricks(vdbgpu_map* m, uint32_t bcap, uint32_t seg_cap, uint32_t split
     m->seg_cap = seg_cap;
     CK(dalloc(m, &m->segs, seg_cap));
   }
-  // work items: at most one partial item per brick plus seg_cap / kItemSegs full ones
-  const uint32_t item_need = m->bcap + m->seg_cap / kItemSegs + 1;
+  // work items: at most one partial item per brick plus seg_cap / kSmallItemSegs full ones
+  const uint32_t item_need = m->bcap + m->seg_cap / kSmallItemSegs + 1;
   if (item_need > m->item_cap) {
     dfree(m, &m->items, m->item_cap);
     m->item_cap = item_need;
@@ -1321,14 +1321,14 @@ int brick_tables(vdbgpu_map* m, int64_t n, double R) {
 // The brick stages of a staged scan on the cast stream: cut, walk (records
 // into the set named in m->d_dest) and record counts. `nb` = workgroups
 // of the cut (lanes past the scan's rays do nothing).
-int cast_chain(vdbgpu_map* m, int nb) {
+int cast_chain(vdbgpu_map* m, int nb, uint32_t item_segs) {
   hipStream_t cs = m->cast;
   const BrickView bv{m->bkeys, m->bcnt, m->bcnt + m->bcap, m->bcap - 1};
   {
     Timer t(m, kTraverse, cs);
     CK(launch_seg_count(cs, nb, m->rayinfo, m->d_scans, m->d_ctl, m->tbl, bv, m->wkey, m->wsc, &m->d_st[0]));
     CK(launch_brick_offsets(cs, bv, m->bbsum, m->bboff, m->items, m->seg_cap, m->item_cap,
-                            m->split_slot, m->split_cap, &m->d_st[0]));
+                            m->split_slot, m->split_cap, item_segs, &m->d_st[0]));
     CK(launch_seg_fill(cs, nb, m->rayinfo, m->d_scans, m->d_ctl, m->tbl, bv, m->wkey, m->wsc, m->segs,
                        m->seg_cap, &m->d_st[0]));
   }
@@ -1358,12 +1358,12 @@ void drop_cast_graphs(vdbgpu_map* m) {
 // grown table simply yields another graph. The record set comes from device
 // memory and the cut's grid is rounded up to a power of two, so that every
 // set of the ring and scans of different sizes share graphs.
-int launch_cast_graph(vdbgpu_map* m, int nb) {
+int launch_cast_graph(vdbgpu_map* m, int nb, uint32_t item_segs) {
   hipStream_t cs = m->cast;
   const int grid = (int)next_pow2((uint64_t)nb);
   auto u = [](const void* p) { return (uint64_t)(uintptr_t)p; };
   const std::vector<uint64_t> key = {
-      (uint64_t)grid, (uint64_t)m->num_cu, u(m->rayinfo), u(m->d_scans), u(m->d_ctl), u(m->tbl), u(m->bkeys),
+      (uint64_t)grid, (uint64_t)m->num_cu, item_segs, u(m->rayinfo), u(m->d_scans), u(m->d_ctl), u(m->tbl), u(m->bkeys),
       u(m->bcnt), m->bcap, u(m->wkey), u(m->wsc), m->wtab_cap, u(m->segs), m->seg_cap, u(m->bbsum), u(m->bboff),
       u(m->items), m->item_cap, u(m->split_slot), m->split_cap, u(m->shared_bits), u(m->d_dest),
       u(m->d_rcnt), u(m->d_st)};
@@ -1380,7 +1380,7 @@ int launch_cast_graph(vdbgpu_map* m, int nb) {
       m->cast_graphs.erase(m->cast_graphs.begin() + (long)lru);
     }
     CK(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
-    const int rc = cast_chain(m, grid);
+    const int rc = cast_chain(m, grid, item_segs);
     hipGraph_t graph = nullptr;
     const hipError_t ec = hipStreamEndCapture(cs, &graph);
     if (rc || ec != hipSuccess || !graph) {
@@ -1434,12 +1434,13 @@ int brick_enqueue(vdbgpu_map* m, BrickCast& c, int attempt) {
     }
   }
   c.cap = m->dcap[c.X];  // (a later first use may size an empty set X before this is checked)
+  const uint32_t item_segs = c.n <= (int64_t)kSmallScanRays ? kSmallItemSegs : kItemSegs;
   const RecDest dest{m->dkeys[c.X], m->dmasks[c.X], c.cap, 0};
   uint64_t vb = 0;
   if ((r = stage_scans(m, cs, c.xyz, c.stride, c.on_device, {c.sc}, (uint32_t)c.n, false, &vb, &dest))) return r;
   if (m->graph_casts && !m->profiling) {
-    if ((r = launch_cast_graph(m, nb))) return r;
-  } else if ((r = cast_chain(m, nb))) {
+    if ((r = launch_cast_graph(m, nb, item_segs))) return r;
+  } else if ((r = cast_chain(m, nb, item_segs))) {
     return r;
   }
   // the scan's status and a snapshot of the leaf count: the map stream keeps

@@ -51,6 +51,7 @@ constexpr uint32_t kOvfSegs = 4u;     // segment array
 constexpr uint32_t kOvfItems = 8u;    // work items
 constexpr uint32_t kOvfSplit = 16u;   // shared-brick bitmaps
 constexpr uint32_t kOvfRecords = 32u; // update-leaf records
+constexpr uint32_t kOvfSpans = 64u;   // fast-mode span lists
 // Segments per brick work item, at most and for small scans: a small scan has
 // too few bricks to fill the chip, and its crowded ones (all rays start in one)
 // are the walk's critical path, so they are cut finer (the walk of a room scan of
@@ -222,6 +223,13 @@ struct RtInfo {
   int bbox[6];
   unsigned int nodes, leaves;
 };
+// A run of existing leaves along a ray of a fast-mode cast.
+struct FastSpan {
+  double t0, t1;
+  uint32_t ray;
+  uint32_t len;  // about its voxels
+};
+constexpr uint32_t kFastSpans = 1024;  // spans per workgroup (256 rays) to start with, and per sort of the walk
 // Word and bit of the leaf at (x, y, z) in its 128^3 node.
 __host__ __device__ inline int rt_word(int x, int y, int z) {
   return (((x >> 5) & 3) << 4) | (((y >> 5) & 3) << 2) | ((z >> 5) & 3);

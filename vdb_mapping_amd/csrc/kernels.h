@@ -21,9 +21,11 @@ hipError_t launch_traverse(hipStream_t s, int grid, int block, const int4* rayin
                            const uint64_t* roff, const uint32_t* first_ray, const ScanInfo* scans,
                            const BatchCtl* ctl, const double* tbl, UpdView u, Status* st,
                            uint32_t chunk);
+// spans: cap per workgroup of the grid (fast_grid), count: one per workgroup, left: one per ray
+uint32_t fast_grid(int num_cu, uint32_t n, bool cast);
 hipError_t launch_fast_cast(hipStream_t s, int num_cu, uint32_t n, const int4* rayinfo, const ScanInfo* scans,
-                            const BatchCtl* ctl, RtView rt, MapView mp, UpdView u, bool cast,
-                            Status* st);
+                            const BatchCtl* ctl, RtView rt, MapView mp, UpdView u, bool cast, FastSpan* spans,
+                            uint32_t cap, uint32_t* count, int* left, Status* st);
 hipError_t launch_compact(hipStream_t s, UpdView u, uint32_t cap, uint32_t* list,
                           unsigned int* counter, const Status* st);
 hipError_t launch_group_build(hipStream_t s, int grid, UpdView u, const uint32_t* list, GroupView gv,

@@ -234,6 +234,13 @@ struct vdbgpu_map {
   unsigned int* ngroups = nullptr;
   double* tbl = nullptr;
   uint32_t tbl_n = 0;
+  // fast-mode casts: spans per workgroup of the search, their counts, and the
+  // rays' remaining steps
+  FastSpan* f_spans = nullptr;
+  uint32_t* f_count = nullptr;
+  uint32_t f_groups = 0, f_cap = kFastSpans;
+  int* f_left = nullptr;
+  uint32_t f_rays = 0;
   // export of the active points: listed leaves (order key, count, pool index,
   // first point) and the points
   uint64_t* pt_key = nullptr;
@@ -1064,11 +1071,29 @@ int run_fast(vdbgpu_map* m, Source& src, const float* xyz, int64_t n, int64_t st
   if (src.cap == 0) {
     if ((r = alloc_update(m, src, (uint32_t)std::max<uint64_t>(kMinUpdateCap, next_pow2(4 * (uint64_t)n))))) return r;
   }
+  const uint32_t groups = fast_grid(m->num_cu, (uint32_t)n, cast);
+  auto span_lists = [&](uint32_t cap) -> int {
+    dfree(m, &m->f_spans, (size_t)m->f_groups * m->f_cap);
+    dfree(m, &m->f_count, m->f_groups);
+    m->f_groups = 0;
+    CK(dalloc(m, &m->f_spans, (size_t)groups * cap));
+    CK(dalloc(m, &m->f_count, groups));
+    m->f_groups = groups;
+    m->f_cap = cap;
+    return VDBGPU_OK;
+  };
+  if (groups > m->f_groups && (r = span_lists(m->f_cap))) return r;
+  if ((uint32_t)n > m->f_rays) {
+    dfree(m, &m->f_left, m->f_rays);
+    m->f_rays = 0;
+    CK(dalloc(m, &m->f_left, (uint32_t)n));
+    m->f_rays = (uint32_t)n;
+  }
   for (int attempt = 0;; ++attempt) {
     {
       Timer t(m, kTraverse);
       CK(launch_fast_cast(m->stream, m->num_cu, (uint32_t)n, m->rayinfo, m->d_scans, m->d_ctl, rt_view(m), map_view(m),
-                          upd_view(src), cast, &m->d_st[0]));
+                          upd_view(src), cast, m->f_spans, m->f_cap, m->f_count, m->f_left, &m->d_st[0]));
     }
     {
       Timer t(m, kCompact);
@@ -1078,9 +1103,11 @@ int run_fast(vdbgpu_map* m, Source& src, const float* xyz, int64_t n, int64_t st
     if ((r = read_status(m))) return r;
     const Status& st = m->h_st[0];
     if ((r = scan_error(m, st, false))) return r;
-    if (!(st.overflow & kOvfHard)) break;
-    if (attempt > 8 || src.cap >= (1u << 30)) return fail(m, VDBGPU_DEVICE_ERROR, "update set cannot grow");
-    if ((r = grow_update(m, src, src.cap * 4))) return r;
+    if (!st.overflow) break;
+    if (attempt > 12 || src.cap >= (1u << 30) || m->f_cap >= (1u << 28))
+      return fail(m, VDBGPU_DEVICE_ERROR, "update set cannot grow");
+    if ((st.overflow & kOvfHard) && (r = grow_update(m, src, src.cap * 4))) return r;
+    if ((st.overflow & kOvfSpans) && (r = span_lists(m->f_cap * 4))) return r;
     CK(hipMemsetAsync(&m->d_st[0].overflow, 0, sizeof(unsigned int), m->stream));
     CK(hipMemsetAsync(&m->d_st[0].entries, 0, sizeof(unsigned int), m->stream));
   }
@@ -2071,6 +2098,9 @@ uint64_t walk_scratch(vdbgpu_map* m, bool release) {
   one(m->gneed, m->gcap);
   one(m->glist, m->gcap);
   one(m->gidx, m->gcap);
+  one(m->f_spans, (size_t)m->f_groups * m->f_cap);
+  one(m->f_count, m->f_groups);
+  one(m->f_left, m->f_rays);
   one(m->pt_key, m->pt_cap);
   one(m->pt_cnt, m->pt_cap);
   one(m->pt_idx, m->pt_cap);
@@ -2094,6 +2124,7 @@ uint64_t walk_scratch(vdbgpu_map* m, bool release) {
     if (m->h_sec) (void)hipHostFree(m->h_sec);
     m->h_sec = nullptr;
     m->sec_cells = m->sec_cap = 0;
+    m->f_groups = m->f_rays = 0;
     m->pt_cap = m->pt_xyz_cap = 0;
     m->points_bytes = 0;
     m->ray_cap = 0;
@@ -2294,6 +2325,9 @@ void vdbgpu_destroy(vdbgpu_map* m) {
   dfree(m, &m->q_in, (size_t)m->q_cap * 7);
   dfree(m, &m->q_succ, (size_t)m->q_cap);
   dfree(m, &m->q_end, (size_t)m->q_cap * 3);
+  dfree(m, &m->f_spans, (size_t)m->f_groups * m->f_cap);
+  dfree(m, &m->f_count, m->f_groups);
+  dfree(m, &m->f_left, m->f_rays);
   dfree(m, &m->pt_key, m->pt_cap);
   dfree(m, &m->pt_cnt, m->pt_cap);
   dfree(m, &m->pt_idx, m->pt_cap);

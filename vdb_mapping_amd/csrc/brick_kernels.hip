@@ -102,6 +102,19 @@ __device__ __forceinline__ int lds_brick(unsigned long long* lkey, uint64_t key,
 // absent or after kMaxBrickProbe probes (then the table is flagged full).
 __device__ __forceinline__ uint32_t brick_slot(const BrickView& bv, uint64_t key, bool insert,
                                                unsigned int* ovf) {
+  if (bv.cells) {
+    int b[3];
+    brick_coords(key, b);
+    const uint32_t D = 2u * (uint32_t)bv.half + 1;
+    const uint32_t x = (uint32_t)(b[0] - (bv.scan->s[0] >> kBrickLog) + bv.half),
+                   y = (uint32_t)(b[1] - (bv.scan->s[1] >> kBrickLog) + bv.half),
+                   z = (uint32_t)(b[2] - (bv.scan->s[2] >> kBrickLog) + bv.half);
+    // every ray ends within the range the cube was sized for; a brick outside
+    // would be an error, and is treated like a full table
+    if (x < D && y < D && z < D) return (x * D + y) * D + z;
+    atomicOr(ovf, kOvfBricks);
+    return kNone;
+  }
   uint32_t h = (uint32_t)fmix64(key) & bv.cap_mask;
   const uint32_t limit = bv.cap_mask < kMaxBrickProbe ? bv.cap_mask + 1 : kMaxBrickProbe;
   for (uint32_t p = 0; p < limit; ++p) {
@@ -117,6 +130,19 @@ __device__ __forceinline__ uint32_t brick_slot(const BrickView& bv, uint64_t key
   }
   if (insert) atomicOr(ovf, kOvfBricks);
   return kNone;
+}
+
+// Coordinates of the brick in a slot.
+__device__ __forceinline__ void brick_of(const BrickView& bv, uint32_t slot, int b[3]) {
+  if (bv.cells) {
+    const uint32_t D = 2u * (uint32_t)bv.half + 1;
+    const uint32_t z = slot % D, q = slot / D, y = q % D, x = q / D;
+    b[0] = (int)x - bv.half + (bv.scan->s[0] >> kBrickLog);
+    b[1] = (int)y - bv.half + (bv.scan->s[1] >> kBrickLog);
+    b[2] = (int)z - bv.half + (bv.scan->s[2] >> kBrickLog);
+  } else {
+    brick_coords(bv.keys[slot], b);
+  }
 }
 
 // Workgroup-uniform stop flag: error or any overflow already raised.
@@ -528,7 +554,7 @@ __global__ __launch_bounds__(kWalkThreads, 8) void k_brick_walk(const BrickItem*
   for (uint32_t it = blockIdx.x; it < n_items; it += gridDim.x) {
     const BrickItem item = items[it];
     int b[3];
-    brick_coords(bv.keys[item.slot], b);
+    brick_of(bv, item.slot, b);
     const int ox = b[0] * kBrickDim, oy = b[1] * kBrickDim, oz = b[2] * kBrickDim;
     for (int w = t; w < kWalkWords; w += kWalkThreads) vis[w] = 0;
     for (int w = t; w < 512; w += kWalkThreads) bits[512 + w] = 0;  // hits; the visited words are merged in
@@ -617,7 +643,7 @@ __global__ __launch_bounds__(256) void k_split_emit(const uint32_t* __restrict__
     }
     __syncthreads();
     int b[3];
-    brick_coords(bv.keys[split_slot[k]], b);
+    brick_of(bv, split_slot[k], b);
     emit_leaves(bits, b[0] * kBrickDim, b[1] * kBrickDim, b[2] * kBrickDim, d, k & (regions - 1), stride, rcnt,
                 s_pos);
     __syncthreads();
@@ -674,7 +700,7 @@ hipError_t launch_seg_count(hipStream_t s, int grid, const int4* rayinfo, const 
 hipError_t launch_brick_offsets(hipStream_t s, BrickView bv, uint64_t* bsum, uint64_t* boff,
                                 BrickItem* items, uint32_t seg_cap, uint32_t item_cap,
                                 uint32_t* split_slot, uint32_t split_cap, uint32_t item_segs, Status* st) {
-  const uint32_t nb = (bv.cap_mask + 1) / 256;
+  const uint32_t nb = bv.slots() / 256;
   hipLaunchKernelGGL(k_brick_sums, dim3(nb), dim3(256), 0, s, bv, bsum, item_segs);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;

@@ -150,12 +150,21 @@ struct GroupView {
   uint32_t cap_mask;
 };
 
-// Bricks (32^3 voxels) of one scan: key -> segment count and fill cursor.
+// Bricks (32^3 voxels) of one scan: slot -> segment count and fill cursor. A
+// slot is a cell of the cube of 2 half + 1 bricks around the sensor's brick
+// where that has at most kDenseBricks cells (ranges up to 1,600 voxels), x-major:
+// no key to compare or insert, a count is one atomic without a result, and the
+// bricks are listed in space order. Farther rays hash the brick's key.
+constexpr uint32_t kDenseBricks = 1u << 20;
 struct BrickView {
-  unsigned long long* keys;  // kEmpty = free
+  unsigned long long* keys;  // hash: kEmpty = free
   uint32_t* cnt;             // segments in the brick
   uint32_t* cur;             // next free segment position (fill stage)
-  uint32_t cap_mask;
+  uint32_t cap_mask;         // hash slots - 1
+  uint32_t cells;            // dense slots, a multiple of 256 (0: hash)
+  int half;                  // bricks to each side
+  const ScanInfo* scan;      // the scan (its origin voxel)
+  __host__ __device__ __forceinline__ uint32_t slots() const { return cells ? cells : cap_mask + 1; }
 };
 // One work item of the brick walk: segments [seg0, seg1) of brick `slot`;
 // `shared` indexes the global bitmap the items of a split brick OR into

@@ -1068,7 +1068,7 @@ __global__ __launch_bounds__(256) void k_rehash_map(MapView mp, uint32_t leaf_co
 // Per-scan set-up of a single-scan cast in one launch: the scan record and
 // the size block (by value, so no host-to-device copy is queued behind the
 // previous scan's map update), a zeroed scan status, and for a brick cast the
-// brick table cleared (keys EMPTY, counts and cursors 0), the record set named
+// brick table cleared (nb words of counts, keys EMPTY unless null), the record set named
 // and its counters cleared.
 __global__ void k_stage_scan(ScanInfo sc, BatchCtl ctl, ScanInfo* __restrict__ d_scans,
                              BatchCtl* __restrict__ d_ctl, Status* st, unsigned long long* bkeys,
@@ -1084,7 +1084,7 @@ __global__ void k_stage_scan(ScanInfo sc, BatchCtl ctl, ScanInfo* __restrict__ d
   if (i0 < sizeof(Status) / 4) reinterpret_cast<uint32_t*>(st)[i0] = 0u;
   const uint64_t G = (uint64_t)gridDim.x * blockDim.x;
   for (uint64_t i = i0; i < nb; i += G) {
-    bkeys[i] = kEmpty;
+    if (bkeys) bkeys[i] = kEmpty;
     bcnt[i] = 0;
   }
 }

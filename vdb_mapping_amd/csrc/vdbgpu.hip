@@ -885,7 +885,7 @@ int launch_fold_stage(vdbgpu_map* m, Source& src, bool from_groups) {
 // visit bound of the scans in *visits_bound.
 int stage_scans(vdbgpu_map* m, hipStream_t stream, const float* xyz, int64_t stride, bool on_device,
                 const std::vector<ScanInfo>& scans, uint32_t n_total, bool batched,
-                uint64_t* visits_bound, const RecDest* dest = nullptr) {
+                uint64_t* visits_bound, const RecDest* dest = nullptr, uint32_t dense_cells = 0) {
   const bool clear_bricks = dest != nullptr;  // a brick cast: its record set, the brick table cleared
   int r;
   if ((r = ensure_rays(m, n_total))) return r;
@@ -916,9 +916,9 @@ int stage_scans(vdbgpu_map* m, hipStream_t stream, const float* xyz, int64_t str
   if (scans.size() == 1) {
     // one launch: scan record and sizes by value, status zeroed, brick table cleared
     CK(launch_stage_scan(stream, scans[0], ctl, m->d_scans, m->d_ctl, &m->d_st[0],
-                         clear_bricks ? m->bkeys : nullptr,
+                         clear_bricks && !dense_cells ? m->bkeys : nullptr,
                          clear_bricks ? reinterpret_cast<unsigned long long*>(m->bcnt) : nullptr,
-                         clear_bricks ? m->bcap : 0, dest ? *dest : RecDest{}, dest ? m->d_dest : nullptr,
+                         clear_bricks ? (dense_cells ? dense_cells / 2 : m->bcap) : 0, dest ? *dest : RecDest{}, dest ? m->d_dest : nullptr,
                          m->d_rcnt));
   } else {
     std::copy(scans.begin(), scans.end(), m->h_scans);
@@ -1321,6 +1321,19 @@ struct BrickCast {
   uint64_t epoch = 0;  // m->cast_epoch then
 };
 
+// Bricks to each side of the sensor's that rays of range R can reach, and the
+// cells of that cube padded to workgroups of 256; 0 cells where it is too large
+// (then the bricks are hashed).
+int dense_half(const vdbgpu_map* m, double R, uint32_t* cells) {
+  *cells = 0;
+  const double ext = std::ceil(R * m->inv) + 2.0;  // voxels along an axis
+  if (!(ext < (double)kMaxTableN)) return 0;
+  const uint64_t half = ((uint64_t)ext >> 5) + 1, d = 2 * half + 1;
+  if (d * d * d > kDenseBricks) return 0;
+  *cells = (uint32_t)((d * d * d + 255) / 256 * 256);
+  return (int)half;
+}
+
 // Tables of the brick path sized for a scan of n rays of range R (the first
 // scan: from its visit bound; the per-block segment tables: for its blocks).
 int brick_tables(vdbgpu_map* m, int64_t n, double R) {
@@ -1333,6 +1346,9 @@ int brick_tables(vdbgpu_map* m, int64_t n, double R) {
                            (uint32_t)std::max<uint64_t>(1u << 16, std::min<uint64_t>(segs0, 0xC0000000ull)), 256)))
       return r;
   }
+  uint32_t cells = 0;
+  (void)dense_half(m, R, &cells);
+  if (cells > m->bcap && (r = ensure_bricks(m, (uint32_t)next_pow2(cells), m->seg_cap, m->split_cap))) return r;
   const int nb = (int)((n + kPrepBlock - 1) / kPrepBlock);
   if ((uint64_t)nb * kSegTab > m->wtab_cap) {  // (hipFree waits for the kernels using them)
     dfree(m, &m->wkey, m->wtab_cap);
@@ -1348,9 +1364,9 @@ int brick_tables(vdbgpu_map* m, int64_t n, double R) {
 // The brick stages of a staged scan on the cast stream: cut, walk (records
 // into the set named in m->d_dest) and record counts. `nb` = workgroups
 // of the cut (lanes past the scan's rays do nothing).
-int cast_chain(vdbgpu_map* m, int nb, uint32_t item_segs) {
+int cast_chain(vdbgpu_map* m, int nb, uint32_t item_segs, int half, uint32_t cells) {
   hipStream_t cs = m->cast;
-  const BrickView bv{m->bkeys, m->bcnt, m->bcnt + m->bcap, m->bcap - 1};
+  const BrickView bv{m->bkeys, m->bcnt, m->bcnt + m->bcap, m->bcap - 1, cells, half, m->d_scans};
   {
     Timer t(m, kTraverse, cs);
     CK(launch_seg_count(cs, nb, m->rayinfo, m->d_scans, m->d_ctl, m->tbl, bv, m->wkey, m->wsc, &m->d_st[0]));
@@ -1385,12 +1401,12 @@ void drop_cast_graphs(vdbgpu_map* m) {
 // grown table simply yields another graph. The record set comes from device
 // memory and the cut's grid is rounded up to a power of two, so that every
 // set of the ring and scans of different sizes share graphs.
-int launch_cast_graph(vdbgpu_map* m, int nb, uint32_t item_segs) {
+int launch_cast_graph(vdbgpu_map* m, int nb, uint32_t item_segs, int half, uint32_t cells) {
   hipStream_t cs = m->cast;
   const int grid = (int)next_pow2((uint64_t)nb);
   auto u = [](const void* p) { return (uint64_t)(uintptr_t)p; };
   const std::vector<uint64_t> key = {
-      (uint64_t)grid, (uint64_t)m->num_cu, item_segs, u(m->rayinfo), u(m->d_scans), u(m->d_ctl), u(m->tbl), u(m->bkeys),
+      (uint64_t)grid, (uint64_t)m->num_cu, item_segs, (uint64_t)half, cells, u(m->rayinfo), u(m->d_scans), u(m->d_ctl), u(m->tbl), u(m->bkeys),
       u(m->bcnt), m->bcap, u(m->wkey), u(m->wsc), m->wtab_cap, u(m->segs), m->seg_cap, u(m->bbsum), u(m->bboff),
       u(m->items), m->item_cap, u(m->split_slot), m->split_cap, u(m->shared_bits), u(m->d_dest),
       u(m->d_rcnt), u(m->d_st)};
@@ -1407,7 +1423,7 @@ int launch_cast_graph(vdbgpu_map* m, int nb, uint32_t item_segs) {
       m->cast_graphs.erase(m->cast_graphs.begin() + (long)lru);
     }
     CK(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
-    const int rc = cast_chain(m, grid, item_segs);
+    const int rc = cast_chain(m, grid, item_segs, half, cells);
     hipGraph_t graph = nullptr;
     const hipError_t ec = hipStreamEndCapture(cs, &graph);
     if (rc || ec != hipSuccess || !graph) {
@@ -1461,13 +1477,15 @@ int brick_enqueue(vdbgpu_map* m, BrickCast& c, int attempt) {
     }
   }
   c.cap = m->dcap[c.X];  // (a later first use may size an empty set X before this is checked)
+  uint32_t cells = 0;
+  const int half = dense_half(m, c.sc.R, &cells);
   const uint32_t item_segs = c.n <= (int64_t)kSmallScanRays ? kSmallItemSegs : kItemSegs;
   const RecDest dest{m->dkeys[c.X], m->dmasks[c.X], c.cap, 0};
   uint64_t vb = 0;
-  if ((r = stage_scans(m, cs, c.xyz, c.stride, c.on_device, {c.sc}, (uint32_t)c.n, false, &vb, &dest))) return r;
+  if ((r = stage_scans(m, cs, c.xyz, c.stride, c.on_device, {c.sc}, (uint32_t)c.n, false, &vb, &dest, cells))) return r;
   if (m->graph_casts && !m->profiling) {
-    if ((r = launch_cast_graph(m, nb, item_segs))) return r;
-  } else if ((r = cast_chain(m, nb, item_segs))) {
+    if ((r = launch_cast_graph(m, nb, item_segs, half, cells))) return r;
+  } else if ((r = cast_chain(m, nb, item_segs, half, cells))) {
     return r;
   }
   // the scan's status and a snapshot of the leaf count: the map stream keeps
@@ -1503,6 +1521,10 @@ int brick_check(vdbgpu_map* m, BrickCast& c) {
     const Status st = h[0];
     if ((r = scan_error(m, st, false))) return r;
     if (st.overflow == 0) break;
+    uint32_t cells = 0;
+    (void)dense_half(m, c.sc.R, &cells);
+    if ((st.overflow & kOvfBricks) && cells)
+      return fail(m, VDBGPU_DEVICE_ERROR, "a ray left the bricks of its range (internal bound violated)");
     if (st.overflow & ~kOvfRecords) {
       const uint32_t bcap = (st.overflow & kOvfBricks) ? (uint32_t)std::min<uint64_t>(1u << 30, (uint64_t)m->bcap * 4) : m->bcap;
       const uint32_t seg_cap = st.segs > m->seg_cap ? grow_cap(st.segs, m->seg_cap) : m->seg_cap;

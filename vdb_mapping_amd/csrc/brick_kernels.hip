@@ -17,8 +17,6 @@
 //   k_seg_count     one lane per ray: enumerate its bricks, count segments
 //                   per brick (aggregated per workgroup in an LDS table,
 //                   which is stored for the fill)
-//   k_brick_sums    per 256 brick slots: sums of segments and work items
-//   k_scan_u64      exclusive scan of those sums (one 256-thread workgroup)
 //   k_brick_offsets segment offset and work items of each brick
 //   k_seg_fill      reserve the run of each entry of the workgroup's stored
 //                   table, enumerate again, write each segment record at its
@@ -28,7 +26,7 @@
 //                   the scan's record set (named in device memory), or OR
 //                   into the shared bitmap of a split brick
 //   k_split_emit    leaf records of split bricks
-//   k_rec_total     record counts of the regions, overflow
+//   k_rec_total     ray, visit and record counts of the scan, overflow
 //
 // Segment record (uint4), self-contained so the walk loads nothing else:
 //   x = n0 | n1 << 14, y = n2 | c0 << 14, z = c1 | c2 << 14  (|delta| per axis
@@ -37,6 +35,8 @@
 //       negative-step bits x, y, z << 24 | end-voxel hit flag << 31
 // The walk of a segment starts at that voxel with the integer DDA state of
 // those counts and visits m (<= 94) voxels, all inside the brick (checked).
+#include <cstddef>
+
 #include "dda_math.h"
 #include "device_common.h"
 #include "kernels.h"
@@ -154,17 +154,6 @@ __device__ __forceinline__ bool stopped(const Status* st, unsigned int* s_stop) 
   return *s_stop != 0;
 }
 
-__device__ __forceinline__ uint64_t block_sum_u64(uint64_t v, uint64_t* s_w) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  if (bw_lane() == 0) s_w[threadIdx.x >> 6] = v;
-  __syncthreads();
-  uint64_t t = 0;
-  for (int w = 0; w < (int)(blockDim.x >> 6); ++w) t += s_w[w];
-  __syncthreads();
-  return t;
-}
-
 // Regions in use for a scan of n_items work items: enough counters that the
 // appends of tens of thousands of bricks do not queue on one (a single one made
 // the walk 0.75 -> 1.27 ms), one for small scans, whose few bricks would fill
@@ -255,24 +244,10 @@ __global__ __launch_bounds__(256) void k_seg_count(const int4* __restrict__ rayi
   }
 }
 
-// Per 256 slots: (work items << 32) | segments.
-__global__ __launch_bounds__(256) void k_brick_sums(BrickView bv, uint64_t* __restrict__ bsum,
-                                                    uint32_t item_segs) {
-  __shared__ uint64_t s_w[4];
-  const uint32_t slot = blockIdx.x * blockDim.x + threadIdx.x;
-  const uint32_t c = bv.cnt[slot];
-  const uint64_t v = ((uint64_t)((c + item_segs - 1) / item_segs) << 32) | c;
-  const uint64_t t = block_sum_u64(v, s_w);
-  if (threadIdx.x == 0) bsum[blockIdx.x] = t;
-}
-
-// Exclusive scan of nb packed sums (one workgroup); totals to st: the sum's
-// bits from total_shift up, and its low half where `low` is given (the
-// segments: one atomic per wave of the count on st->segs took 40 of its 103 us
-// for 262,144 rays).
+// Exclusive scan of nb sums (one workgroup); their total to *total.
 __global__ __launch_bounds__(256) void k_scan_u64(const uint64_t* __restrict__ bsum,
                                                   uint64_t* __restrict__ boff, uint32_t nb,
-                                                  unsigned int* total, int total_shift, unsigned int* low) {
+                                                  unsigned int* total) {
   __shared__ uint64_t wsum[4];
   uint64_t carry = 0;
   for (uint32_t base = 0; base < nb; base += 256) {
@@ -296,22 +271,29 @@ __global__ __launch_bounds__(256) void k_scan_u64(const uint64_t* __restrict__ b
     carry += tot;
     __syncthreads();
   }
-  if (threadIdx.x == 0) {
-    *total = (unsigned int)(carry >> total_shift);
-    if (low) *low = (unsigned int)carry;
-  }
+  if (threadIdx.x == 0) *total = (unsigned int)carry;
 }
 
-__global__ __launch_bounds__(256) void k_brick_offsets(BrickView bv, const uint64_t* __restrict__ boff,
-                                                       BrickItem* __restrict__ items,
+// Segment offset and work items of each brick, kOffsetSlots slots a workgroup
+// (four to a lane). A workgroup takes its run of segments and of items with one
+// atomic on the pair of totals; which run a brick gets does not matter, so no
+// scan over the workgroups is needed (it took two more launches, 9 us of a
+// 2,000-point scan's 160 us of GPU time). A range of 1,000 voxels has 268
+// workgroups, and only those with a segment touch the counter.
+__global__ __launch_bounds__(256) void k_brick_offsets(BrickView bv, BrickItem* __restrict__ items,
                                                        uint32_t seg_cap, uint32_t item_cap,
                                                        uint32_t* __restrict__ split_slot,
                                                        uint32_t split_cap, uint32_t item_segs, Status* st) {
+  static_assert(offsetof(Status, segs) % 8 == 0 && offsetof(Status, items) == offsetof(Status, segs) + 4,
+                "segs and items are one 64-bit counter");
   __shared__ uint64_t s_w[4];
-  const uint32_t slot = blockIdx.x * blockDim.x + threadIdx.x;
-  const uint32_t c = bv.cnt[slot];
-  const uint32_t ni = (c + item_segs - 1) / item_segs;
-  const uint64_t x = ((uint64_t)ni << 32) | c;
+  __shared__ uint64_t s_base;
+  const uint32_t slot0 = blockIdx.x * kOffsetSlots + threadIdx.x * 4;
+  const uint4 q = *reinterpret_cast<const uint4*>(bv.cnt + slot0);
+  const uint32_t c[4] = {q.x, q.y, q.z, q.w};
+  uint64_t x = 0;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) x += ((uint64_t)((c[k] + item_segs - 1) / item_segs) << 32) | c[k];
   uint64_t v = x;
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
@@ -321,33 +303,38 @@ __global__ __launch_bounds__(256) void k_brick_offsets(BrickView bv, const uint6
   const int wv = threadIdx.x >> 6;
   if (bw_lane() == 63) s_w[wv] = v;
   __syncthreads();
-  uint64_t add = 0;
-  for (int w = 0; w < wv; ++w) add += s_w[w];
-  const uint64_t off = boff[blockIdx.x] + add + v - x;
-  const uint32_t seg0 = (uint32_t)off, item0 = (uint32_t)(off >> 32);
-  bv.cur[slot] = seg0;
-  if (ni == 0) return;
-  if ((uint64_t)seg0 + c > seg_cap) {
-    atomicOr(&st->overflow, kOvfSegs);
-    return;
+  if (threadIdx.x == 0) {
+    const uint64_t sum = s_w[0] + s_w[1] + s_w[2] + s_w[3];
+    s_base = sum ? atomicAdd(reinterpret_cast<unsigned long long*>(&st->segs), (unsigned long long)sum) : 0ull;
   }
-  if ((uint64_t)item0 + ni > item_cap) {
-    atomicOr(&st->overflow, kOvfItems);
-    return;
-  }
-  uint32_t shared = kNone;
-  if (ni > 1) {
-    shared = atomicAdd(&st->splits, 1u);
-    if (shared >= split_cap) {
-      atomicOr(&st->overflow, kOvfSplit);
-      return;
+  __syncthreads();
+  uint64_t off = s_base + v - x;
+  for (int w = 0; w < wv; ++w) off += s_w[w];
+  uint32_t seg0 = (uint32_t)off, item0 = (uint32_t)(off >> 32);
+  const uint32_t s1 = seg0 + c[0], s2 = s1 + c[1];
+  *reinterpret_cast<uint4*>(bv.cur + slot0) = make_uint4(seg0, s1, s2, s2 + c[2]);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const uint32_t slot = slot0 + k, n = c[k], ni = (n + item_segs - 1) / item_segs;
+    if (ni == 0) continue;
+    if ((uint64_t)seg0 + n > seg_cap) {
+      atomicOr(&st->overflow, kOvfSegs);
+    } else if ((uint64_t)item0 + ni > item_cap) {
+      atomicOr(&st->overflow, kOvfItems);
+    } else {
+      const uint32_t shared = ni > 1 ? atomicAdd(&st->splits, 1u) : kNone;
+      if (ni > 1 && shared >= split_cap) {
+        atomicOr(&st->overflow, kOvfSplit);
+      } else {
+        if (ni > 1) split_slot[shared] = slot;
+        for (uint32_t j = 0; j < ni; ++j) {
+          const uint32_t a = seg0 + j * item_segs;
+          items[item0 + j] = BrickItem{slot, a, min(a + item_segs, seg0 + n), shared};
+        }
+      }
     }
-    split_slot[shared] = slot;
-  }
-  for (uint32_t j = 0; j < ni; ++j) {
-    const uint32_t a = seg0 + j * item_segs;
-    const uint32_t b = min(a + item_segs, seg0 + c);
-    items[item0 + j] = BrickItem{slot, a, b, shared};
+    seg0 += n;
+    item0 += ni;
   }
 }
 
@@ -650,10 +637,35 @@ __global__ __launch_bounds__(256) void k_split_emit(const uint32_t* __restrict__
   }
 }
 
-// The scan's record counts (one wave): total, prefix over the regions, and the
+// The scan's counts (one workgroup): its valid rays and visits from the sums of
+// k_prep's workgroups, its records with their prefix over the regions, and the
 // overflow flag when a region did not hold its records.
-__global__ void k_rec_total(const RecDest* dest, const unsigned int* rcnt, Status* st) {
+__global__ __launch_bounds__(256) void k_rec_total(const uint32_t* __restrict__ bsum, const BatchCtl* __restrict__ ctl,
+                                                   const RecDest* dest, const unsigned int* rcnt, Status* st) {
+  __shared__ unsigned long long s_v[4];
+  __shared__ unsigned int s_r[4];
   const uint32_t l = threadIdx.x;
+  unsigned long long visits = 0;
+  uint32_t rays = 0;
+  for (uint32_t i = l; i < ctl->nb; i += 256) {
+    visits += bsum[i] & kPrepVisitMask;
+    rays += bsum[i] >> kPrepValidShift;
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    visits += __shfl_xor(visits, o, 64);
+    rays += __shfl_xor(rays, o, 64);
+  }
+  if (bw_lane() == 0) {
+    s_v[l >> 6] = visits;
+    s_r[l >> 6] = rays;
+  }
+  __syncthreads();
+  if (l >= 64) return;
+  if (l == 0) {
+    st->total = s_v[0] + s_v[1] + s_v[2] + s_v[3];
+    st->rays = (unsigned long long)s_r[0] + s_r[1] + s_r[2] + s_r[3];
+  }
   if (st->error | st->overflow) return;
   const uint32_t stride = dest->cap / rec_regions(st->items);
   const uint32_t c = l < kRecRegions ? rcnt[l * kRecCountStride] : 0u;
@@ -680,8 +692,9 @@ __global__ void k_snap_count(const Status* st, uint32_t* host_dst) {
 
 // ---------------------------------------------------------------- launchers --
 
-hipError_t launch_rec_total(hipStream_t s, const RecDest* dest, const unsigned int* rcnt, Status* st) {
-  hipLaunchKernelGGL(k_rec_total, dim3(1), dim3(64), 0, s, dest, rcnt, st);
+hipError_t launch_rec_total(hipStream_t s, const uint32_t* bsum, const BatchCtl* ctl, const RecDest* dest,
+                            const unsigned int* rcnt, Status* st) {
+  hipLaunchKernelGGL(k_rec_total, dim3(1), dim3(256), 0, s, bsum, ctl, dest, rcnt, st);
   return hipGetLastError();
 }
 
@@ -697,17 +710,9 @@ hipError_t launch_seg_count(hipStream_t s, int grid, const int4* rayinfo, const 
   return hipGetLastError();
 }
 
-hipError_t launch_brick_offsets(hipStream_t s, BrickView bv, uint64_t* bsum, uint64_t* boff,
-                                BrickItem* items, uint32_t seg_cap, uint32_t item_cap,
+hipError_t launch_brick_offsets(hipStream_t s, BrickView bv, BrickItem* items, uint32_t seg_cap, uint32_t item_cap,
                                 uint32_t* split_slot, uint32_t split_cap, uint32_t item_segs, Status* st) {
-  const uint32_t nb = bv.slots() / 256;
-  hipLaunchKernelGGL(k_brick_sums, dim3(nb), dim3(256), 0, s, bv, bsum, item_segs);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_scan_u64, dim3(1), dim3(256), 0, s, bsum, boff, nb, &st->items, 32, &st->segs);
-  e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_brick_offsets, dim3(nb), dim3(256), 0, s, bv, boff, items, seg_cap, item_cap,
+  hipLaunchKernelGGL(k_brick_offsets, dim3(bv.slots() / kOffsetSlots), dim3(256), 0, s, bv, items, seg_cap, item_cap,
                      split_slot, split_cap, item_segs, st);
   return hipGetLastError();
 }
@@ -731,7 +736,7 @@ hipError_t launch_brick_walk(hipStream_t s, int grid, const BrickItem* items, co
 }
 
 hipError_t launch_scan_u64(hipStream_t s, const uint64_t* in, uint64_t* out, uint32_t n, unsigned int* total) {
-  hipLaunchKernelGGL(k_scan_u64, dim3(1), dim3(256), 0, s, in, out, n, total, 0, (unsigned int*)nullptr);
+  hipLaunchKernelGGL(k_scan_u64, dim3(1), dim3(256), 0, s, in, out, n, total);
   return hipGetLastError();
 }
 

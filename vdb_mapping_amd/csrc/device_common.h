@@ -156,12 +156,13 @@ struct GroupView {
 // no key to compare or insert, a count is one atomic without a result, and the
 // bricks are listed in space order. Farther rays hash the brick's key.
 constexpr uint32_t kDenseBricks = 1u << 20;
+constexpr uint32_t kOffsetSlots = 1024;  // slots per workgroup of k_brick_offsets; slots() is a multiple of it
 struct BrickView {
   unsigned long long* keys;  // hash: kEmpty = free
   uint32_t* cnt;             // segments in the brick
   uint32_t* cur;             // next free segment position (fill stage)
   uint32_t cap_mask;         // hash slots - 1
-  uint32_t cells;            // dense slots, a multiple of 256 (0: hash)
+  uint32_t cells;            // dense slots, a multiple of kOffsetSlots (0: hash)
   int half;                  // bricks to each side
   const ScanInfo* scan;      // the scan (its origin voxel)
   __host__ __device__ __forceinline__ uint32_t slots() const { return cells ? cells : cap_mask + 1; }

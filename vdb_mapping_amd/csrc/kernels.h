@@ -51,7 +51,8 @@ hipError_t launch_merge_records(hipStream_t s, UpdView rec, const RecIndex& ri, 
                                 uint32_t* list, unsigned int* listed);
 hipError_t launch_clear_listed(hipStream_t s, UpdView u, const uint32_t* list, uint32_t count);
 hipError_t launch_set_u32(hipStream_t s, unsigned int* p, uint32_t v);
-hipError_t launch_rec_total(hipStream_t s, const RecDest* dest, const unsigned int* rcnt, Status* st);
+hipError_t launch_rec_total(hipStream_t s, const uint32_t* bsum, const BatchCtl* ctl, const RecDest* dest,
+                            const unsigned int* rcnt, Status* st);
 hipError_t launch_snap_count(hipStream_t s, const Status* st, uint32_t* host_dst);
 // Deferred brick-path scans applied as one group pass (integrate_kernels.hip).
 constexpr int kDeferMax = 8;                       // scans per group pass
@@ -92,10 +93,8 @@ constexpr int kSegTab = 1024;
 hipError_t launch_seg_count(hipStream_t s, int grid, const int4* rayinfo, const ScanInfo* scans,
                             const BatchCtl* ctl, const double* tbl, BrickView bv, unsigned long long* wkey,
                             unsigned long long* wsc, Status* st);
-hipError_t launch_brick_offsets(hipStream_t s, BrickView bv, uint64_t* bsum, uint64_t* boff,
-                                BrickItem* items, uint32_t seg_cap, uint32_t item_cap,
-                                uint32_t* split_slot, uint32_t split_cap, uint32_t item_segs,
-                                Status* st);
+hipError_t launch_brick_offsets(hipStream_t s, BrickView bv, BrickItem* items, uint32_t seg_cap, uint32_t item_cap,
+                                uint32_t* split_slot, uint32_t split_cap, uint32_t item_segs, Status* st);
 hipError_t launch_seg_fill(hipStream_t s, int grid, const int4* rayinfo, const ScanInfo* scans,
                            const BatchCtl* ctl, const double* tbl, BrickView bv,
                            const unsigned long long* wkey, const unsigned long long* wsc, uint4* segs,

@@ -176,8 +176,6 @@ struct vdbgpu_map {
   // bitmaps of split bricks, update-leaf records
   unsigned long long* bkeys = nullptr;
   uint32_t* bcnt = nullptr;  // [0, bcap): segment counts, [bcap, 2 bcap): fill cursors
-  uint64_t* bbsum = nullptr;
-  uint64_t* bboff = nullptr;
   uint32_t bcap = 0;
   uint4* segs = nullptr;
   uint32_t seg_cap = 0;
@@ -931,7 +929,8 @@ int stage_scans(vdbgpu_map* m, hipStream_t stream, const float* xyz, int64_t str
   Timer t(m, kPrep, stream);
   CK(launch_prep(stream, (int)nb, pts, stride, vec4, m->d_scans, m->d_ctl, m->res, m->inv, m->tbl_n,
                  m->rayinfo, m->pre, m->bsum, &m->d_st[0]));
-  CK(launch_scan_blocks(stream, m->bsum, m->boff, m->d_ctl, &m->d_st[0]));
+  // (the brick path needs the sums' totals only, at its end: k_rec_total)
+  if (!dest) CK(launch_scan_blocks(stream, m->bsum, m->boff, m->d_ctl, &m->d_st[0]));
   return VDBGPU_OK;
 }
 
@@ -1153,13 +1152,9 @@ int ensure_bricks(vdbgpu_map* m, uint32_t bcap, uint32_t seg_cap, uint32_t split
   if (bcap > m->bcap) {
     dfree(m, &m->bkeys, m->bcap);
     dfree(m, &m->bcnt, (size_t)m->bcap * 2);
-    dfree(m, &m->bbsum, m->bcap / 256);
-    dfree(m, &m->bboff, m->bcap / 256);
     m->bcap = bcap;
     CK(dalloc(m, &m->bkeys, bcap));
     CK(dalloc(m, &m->bcnt, (size_t)bcap * 2));
-    CK(dalloc(m, &m->bbsum, bcap / 256));
-    CK(dalloc(m, &m->bboff, bcap / 256));
   }
   if (seg_cap > m->seg_cap) {
     dfree(m, &m->segs, m->seg_cap);
@@ -1322,7 +1317,7 @@ struct BrickCast {
 };
 
 // Bricks to each side of the sensor's that rays of range R can reach, and the
-// cells of that cube padded to workgroups of 256; 0 cells where it is too large
+// cells of that cube padded to kOffsetSlots; 0 cells where it is too large
 // (then the bricks are hashed).
 int dense_half(const vdbgpu_map* m, double R, uint32_t* cells) {
   *cells = 0;
@@ -1330,7 +1325,7 @@ int dense_half(const vdbgpu_map* m, double R, uint32_t* cells) {
   if (!(ext < (double)kMaxTableN)) return 0;
   const uint64_t half = ((uint64_t)ext >> 5) + 1, d = 2 * half + 1;
   if (d * d * d > kDenseBricks) return 0;
-  *cells = (uint32_t)((d * d * d + 255) / 256 * 256);
+  *cells = (uint32_t)((d * d * d + kOffsetSlots - 1) / kOffsetSlots * kOffsetSlots);
   return (int)half;
 }
 
@@ -1370,7 +1365,7 @@ int cast_chain(vdbgpu_map* m, int nb, uint32_t item_segs, int half, uint32_t cel
   {
     Timer t(m, kTraverse, cs);
     CK(launch_seg_count(cs, nb, m->rayinfo, m->d_scans, m->d_ctl, m->tbl, bv, m->wkey, m->wsc, &m->d_st[0]));
-    CK(launch_brick_offsets(cs, bv, m->bbsum, m->bboff, m->items, m->seg_cap, m->item_cap,
+    CK(launch_brick_offsets(cs, bv, m->items, m->seg_cap, m->item_cap,
                             m->split_slot, m->split_cap, item_segs, &m->d_st[0]));
     CK(launch_seg_fill(cs, nb, m->rayinfo, m->d_scans, m->d_ctl, m->tbl, bv, m->wkey, m->wsc, m->segs,
                        m->seg_cap, &m->d_st[0]));
@@ -1385,7 +1380,7 @@ int cast_chain(vdbgpu_map* m, int nb, uint32_t item_segs, int half, uint32_t cel
   {
     Timer t(m, kCompact, cs);
     CK(launch_split_emit(cs, m->num_cu, m->split_slot, m->shared_bits, bv, m->d_dest, m->d_rcnt, &m->d_st[0]));
-    CK(launch_rec_total(cs, m->d_dest, m->d_rcnt, &m->d_st[0]));
+    CK(launch_rec_total(cs, m->bsum, m->d_ctl, m->d_dest, m->d_rcnt, &m->d_st[0]));
   }
   return VDBGPU_OK;
 }
@@ -1407,7 +1402,7 @@ int launch_cast_graph(vdbgpu_map* m, int nb, uint32_t item_segs, int half, uint3
   auto u = [](const void* p) { return (uint64_t)(uintptr_t)p; };
   const std::vector<uint64_t> key = {
       (uint64_t)grid, (uint64_t)m->num_cu, item_segs, (uint64_t)half, cells, u(m->rayinfo), u(m->d_scans), u(m->d_ctl), u(m->tbl), u(m->bkeys),
-      u(m->bcnt), m->bcap, u(m->wkey), u(m->wsc), m->wtab_cap, u(m->segs), m->seg_cap, u(m->bbsum), u(m->bboff),
+      u(m->bcnt), m->bcap, u(m->wkey), u(m->wsc), m->wtab_cap, u(m->segs), m->seg_cap, u(m->bsum),
       u(m->items), m->item_cap, u(m->split_slot), m->split_cap, u(m->shared_bits), u(m->d_dest),
       u(m->d_rcnt), u(m->d_st)};
   vdbgpu_map::CastGraph* hit = nullptr;
@@ -2098,8 +2093,6 @@ uint64_t walk_scratch(vdbgpu_map* m, bool release) {
   one(m->eidx, m->eidx_cap);
   one(m->bkeys, m->bcap);
   one(m->bcnt, (size_t)m->bcap * 2);
-  one(m->bbsum, m->bcap / 256);
-  one(m->bboff, m->bcap / 256);
   one(m->segs, m->seg_cap);
   one(m->items, m->item_cap);
   one(m->split_slot, m->split_cap);
@@ -2316,8 +2309,6 @@ void vdbgpu_destroy(vdbgpu_map* m) {
   dfree(m, &m->eidx, m->eidx_cap);
   dfree(m, &m->bkeys, m->bcap);
   dfree(m, &m->bcnt, (size_t)m->bcap * 2);
-  dfree(m, &m->bbsum, m->bcap / 256);
-  dfree(m, &m->bboff, m->bcap / 256);
   dfree(m, &m->segs, m->seg_cap);
   dfree(m, &m->items, m->item_cap);
   dfree(m, &m->split_slot, m->split_cap);

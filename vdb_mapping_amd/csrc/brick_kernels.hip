@@ -194,6 +194,11 @@ __device__ void emit_leaves(const unsigned long long* bits, int ox, int oy, int 
   }
 }
 
+// The ray of this lane in the cut: every 2^spread-th lane has one (cut_spread).
+__device__ __forceinline__ uint32_t cut_ray(int spread) {
+  return (threadIdx.x & ((1u << spread) - 1)) ? kNone : (blockIdx.x * blockDim.x + threadIdx.x) >> spread;
+}
+
 }  // namespace
 
 __global__ __launch_bounds__(256) void k_seg_count(const int4* __restrict__ rayinfo,
@@ -201,7 +206,7 @@ __global__ __launch_bounds__(256) void k_seg_count(const int4* __restrict__ rayi
                                                    const BatchCtl* __restrict__ ctl,
                                                    const double* __restrict__ tbl, BrickView bv,
                                                    unsigned long long* __restrict__ wkey,
-                                                   unsigned long long* __restrict__ wsc, Status* st) {
+                                                   unsigned long long* __restrict__ wsc, Status* st, int spread) {
   __shared__ unsigned long long lkey[kLdsBricks];
   __shared__ uint32_t lcnt[kLdsBricks];
   __shared__ unsigned int s_stop;
@@ -211,7 +216,7 @@ __global__ __launch_bounds__(256) void k_seg_count(const int4* __restrict__ rayi
     lcnt[e] = 0;
   }
   __syncthreads();
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t i = cut_ray(spread);
   RayGeom g;
   if (i < ctl->n_rays && ray_geom(rayinfo, scans, i, g)) {
     SegEnum en;
@@ -345,7 +350,7 @@ __global__ __launch_bounds__(256) void k_seg_fill(const int4* __restrict__ rayin
                                                   const unsigned long long* __restrict__ wkey,
                                                   const unsigned long long* __restrict__ wsc,
                                                   uint4* __restrict__ segs, uint32_t seg_cap,
-                                                  Status* st) {
+                                                  Status* st, int spread) {
   __shared__ unsigned long long lkey[kLdsBricks];
   __shared__ uint32_t lcnt[kLdsBricks];
   __shared__ uint32_t lbase[kLdsBricks];
@@ -371,7 +376,7 @@ __global__ __launch_bounds__(256) void k_seg_fill(const int4* __restrict__ rayin
     }
   }
   __syncthreads();
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t i = cut_ray(spread);
   RayGeom g;
   const bool valid = i < ctl->n_rays && ray_geom(rayinfo, scans, i, g);
   // 2: write the records
@@ -705,8 +710,8 @@ hipError_t launch_snap_count(hipStream_t s, const Status* st, uint32_t* host_dst
 
 hipError_t launch_seg_count(hipStream_t s, int grid, const int4* rayinfo, const ScanInfo* scans,
                             const BatchCtl* ctl, const double* tbl, BrickView bv, unsigned long long* wkey,
-                            unsigned long long* wsc, Status* st) {
-  hipLaunchKernelGGL(k_seg_count, dim3(grid), dim3(256), 0, s, rayinfo, scans, ctl, tbl, bv, wkey, wsc, st);
+                            unsigned long long* wsc, Status* st, int spread) {
+  hipLaunchKernelGGL(k_seg_count, dim3(grid), dim3(256), 0, s, rayinfo, scans, ctl, tbl, bv, wkey, wsc, st, spread);
   return hipGetLastError();
 }
 
@@ -720,9 +725,9 @@ hipError_t launch_brick_offsets(hipStream_t s, BrickView bv, BrickItem* items, u
 hipError_t launch_seg_fill(hipStream_t s, int grid, const int4* rayinfo, const ScanInfo* scans,
                            const BatchCtl* ctl, const double* tbl, BrickView bv,
                            const unsigned long long* wkey, const unsigned long long* wsc, uint4* segs,
-                           uint32_t seg_cap, Status* st) {
+                           uint32_t seg_cap, Status* st, int spread) {
   hipLaunchKernelGGL(k_seg_fill, dim3(grid), dim3(256), 0, s, rayinfo, scans, ctl, tbl, bv, wkey, wsc, segs,
-                     seg_cap, st);
+                     seg_cap, st, spread);
   return hipGetLastError();
 }
 

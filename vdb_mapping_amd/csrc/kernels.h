@@ -86,19 +86,29 @@ hipError_t launch_gather_leaves(hipStream_t s, int grid, const uint32_t* list, u
                                 MapView mp, unsigned long long* keys_out, float* vals_out,
                                 unsigned long long* act_out);
 
+// log2 of the lanes per ray: a wave takes as long as its rays' paths laid over
+// one another, so while there are fewer rays than the chip has lanes resident
+// (four waves per SIMD), each gets a fraction of a wave, up to one of its own.
+// (num_cu / 4: while there are fewer than a wave per SIMD.)
+inline int ray_spread(int64_t n, int num_cu) {
+  int k = 0;
+  while (k < 6 && (n << (k + 1)) <= (int64_t)num_cu * 1024) ++k;
+  return k;
+}
+
 // Entries of a workgroup's brick table in k_seg_count / k_seg_fill (LDS); the
 // count stores each workgroup's table (keys; brick slot << 32 | segments) at
 // workgroup * kSegTab of wkey / wsc, and the fill rereads it.
 constexpr int kSegTab = 1024;
 hipError_t launch_seg_count(hipStream_t s, int grid, const int4* rayinfo, const ScanInfo* scans,
                             const BatchCtl* ctl, const double* tbl, BrickView bv, unsigned long long* wkey,
-                            unsigned long long* wsc, Status* st);
+                            unsigned long long* wsc, Status* st, int spread);
 hipError_t launch_brick_offsets(hipStream_t s, BrickView bv, BrickItem* items, uint32_t seg_cap, uint32_t item_cap,
                                 uint32_t* split_slot, uint32_t split_cap, uint32_t item_segs, Status* st);
 hipError_t launch_seg_fill(hipStream_t s, int grid, const int4* rayinfo, const ScanInfo* scans,
                            const BatchCtl* ctl, const double* tbl, BrickView bv,
                            const unsigned long long* wkey, const unsigned long long* wsc, uint4* segs,
-                           uint32_t seg_cap, Status* st);
+                           uint32_t seg_cap, Status* st, int spread);
 hipError_t launch_brick_walk(hipStream_t s, int grid, const BrickItem* items, const uint4* segs,
                              const int4* rayinfo, const ScanInfo* scans, const double* tbl,
                              BrickView bv, unsigned long long* shared_bits, const RecDest* dest,

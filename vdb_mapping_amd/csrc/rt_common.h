@@ -235,15 +235,6 @@ __device__ __forceinline__ void rt_clip(const RtView& rt, const RtRay& r, double
   }
 }
 
-// log2 of the lanes per ray: a wave takes as long as its rays' paths laid over
-// one another, so while there are fewer rays than the chip has lanes resident
-// (four waves per SIMD), each gets a fraction of a wave, up to one of its own.
-inline int ray_spread(int64_t n, int num_cu) {
-  int k = 0;
-  while (k < 6 && (n << (k + 1)) <= (int64_t)num_cu * 1024) ++k;
-  return k;
-}
-
 // VolumeHDDA over the snapshot (4096 -> 128 -> 8): the runs of existing leaves
 // along a ray as time spans, one per call. All lanes of a wave look for their
 // next span together and then walk them together; walking a span where it was

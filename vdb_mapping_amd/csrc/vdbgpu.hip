@@ -4,9 +4,11 @@
 // One vdbgpu_map owns: a HIP stream (default priority), a mutex, the device
 // leaf store + leaf hash, one update set per input source, per-scan scratch,
 // the DDA crossing table and a pinned status block. The per-scan path is
-//   accumulate: [H2D points] -> k_prep -> k_scan_blocks -> k_traverse -> k_compact
-//               -> one status read (the only host sync of a scan)
-//   integrate : k_map_insert -> k_apply per source, in source-id order (no sync)
+//   accumulate: [H2D points] -> the brick cast -> k_merge_records, or, for sparse
+//               clouds, k_prep -> k_scan_blocks -> k_traverse -> k_compact;
+//               one status read (the only host sync of a scan)
+//   integrate : k_map_insert -> k_apply, in source-id order (several sources: one
+//               group pass), no sync
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -86,7 +88,7 @@ struct vdbgpu_map {
   int device = 0;
   int num_cu = 256;
   hipStream_t stream = nullptr;  // map stream: every map read / update, the hash path
-  hipStream_t cast = nullptr;    // brick path casting (prep .. record list) of plain inserts
+  hipStream_t cast = nullptr;    // brick path casting (prep .. records)
   double res = 0, inv = 0;
 
   // config (VDBMapping.hpp:1456-1469, OccupancyVDBMapping.hpp:59-89)
@@ -200,6 +202,9 @@ struct vdbgpu_map {
   RecIndex rindex[kRecSets] = {};             // record set: where its scan's records lie
   uint32_t dcap[kRecSets] = {};
   uint32_t dense_hint = 0;     // record-set size for a first use (largest scan seen, +25%)
+  int64_t guess_rays = 0;      // rays and records of the scan with the most rays so far
+  uint32_t guess_recs = 0;
+  int64_t batch_rays = 0;      // most rays of a scan of the batch being inserted
   hipEvent_t rec_free[kRecSets] = {};  // recorded on the map stream after the last read
   // leaf count after the map insert of each record set's scan (pinned, copied
   // on the map stream before ins_done), for a tight leaf-count bound
@@ -1344,16 +1349,20 @@ int cut_blocks(const vdbgpu_map* m, int64_t n) { return (int)(((n << cut_spread(
 // scan: from its visit bound; the per-block segment tables: for its blocks).
 int brick_tables(vdbgpu_map* m, int64_t n, double R) {
   int r;
+  uint32_t cells = 0;
+  (void)dense_half(m, R, &cells);
   if (m->bcap == 0) {  // first brick-path scan: tables sized from the scan's visit bound
     const double ext = std::min<double>(std::ceil(R * m->inv) + 2.0, (double)kMaxTableN);
     const uint64_t vb = (uint64_t)n * (1 + 3 * (uint64_t)ext);
     const uint64_t segs0 = std::min<uint64_t>(vb, 16ull * (uint64_t)n);
-    if ((r = ensure_bricks(m, (uint32_t)std::max<uint64_t>(4096, next_pow2((uint64_t)n / 2)),
-                           (uint32_t)std::max<uint64_t>(1u << 16, std::min<uint64_t>(segs0, 0xC0000000ull)), 256)))
+    // (a quarter of the work items that the segments fill: the crowded bricks
+    // around the sensor hold several each)
+    const uint64_t items0 = segs0 / (n <= (int64_t)kSmallScanRays ? kSmallItemSegs : kItemSegs);
+    if ((r = ensure_bricks(m, (uint32_t)std::max<uint64_t>(4096, next_pow2(cells ? cells : (uint64_t)n / 2)),
+                           (uint32_t)std::max<uint64_t>(1u << 16, std::min<uint64_t>(segs0, 0xC0000000ull)),
+                           (uint32_t)std::clamp<uint64_t>(next_pow2(items0 / 4 + 1), 256, 4096))))
       return r;
   }
-  uint32_t cells = 0;
-  (void)dense_half(m, R, &cells);
   if (cells > m->bcap && (r = ensure_bricks(m, (uint32_t)next_pow2(cells), m->seg_cap, m->split_cap))) return r;
   const int nb = cut_blocks(m, n);
   if ((uint64_t)nb * kSegTab > m->wtab_cap) {  // (hipFree waits for the kernels using them)
@@ -1469,9 +1478,20 @@ int brick_enqueue(vdbgpu_map* m, BrickCast& c, int attempt) {
     m->cst_next ^= 1;
     CK(hipStreamWaitEvent(cs, m->rec_free[c.X], 0));
     if (m->dense_hint == 0 && m->dcap[c.X] == 0) {
-      // the map's first scan: a guess of its records, for this set alone
-      if ((r = grow_set(m, c.X, (uint32_t)std::max<int64_t>(4096, std::min<int64_t>(c.n / 4, 1 << 20))))) return r;
+      // the map's first scan: a guess of its records, for this set alone (a
+      // third of what a lidar sees outdoors, several times a room's; too small a
+      // set only costs another cast)
+      const double leaves = std::sqrt((double)c.n) * std::min(c.sc.R * m->inv, (double)kMaxTableN);
+      if ((r = grow_set(m, c.X, (uint32_t)std::max(4096.0, std::min(leaves, 1048576.0))))) return r;
       m->dense_hint = 0;
+    } else if (const int64_t most = std::max(c.n, m->batch_rays); m->guess_recs && most > m->guess_rays) {
+      // more rays than any scan so far (or a batch's largest): update leaves
+      // grow with about the root of the rays of one scene; too small a set only
+      // costs another cast. At most 2^21 records (280 MB) on a guess.
+      const double g = 1.25 * m->guess_recs * std::sqrt((double)most / (double)m->guess_rays);
+      m->dense_hint = std::max(m->dense_hint, (uint32_t)std::min(g, 2097152.0));
+      m->guess_rays = most;
+      m->guess_recs = m->dense_hint - m->dense_hint / 5;
     }
     if (m->dcap[c.X] < m->dense_hint) {  // a first use of set X: size it like the others
       CK(hipStreamSynchronize(cs));      // (the map stream is done with it)
@@ -1540,9 +1560,12 @@ int brick_check(vdbgpu_map* m, BrickCast& c) {
       // the records are at most 64 per item and split brick: room for them now
       // saves a growing map's scan another cast
       const uint64_t most = (uint64_t)(st.items + st.splits) * 64;
-      if (!(st.overflow & kOvfBricks) && most > m->dcap[X] && most <= 64ull * (uint64_t)c.n &&
-          (r = grow_set(m, X, (uint32_t)std::min<uint64_t>(most, 0xC0000000ull))))
-        return r;
+      // (for this set alone: the other sets are sized from the records it gets)
+      if (!(st.overflow & kOvfBricks) && most > m->dcap[X] && most <= 64ull * (uint64_t)c.n) {
+        const uint32_t hint = m->dense_hint;
+        if ((r = grow_set(m, X, (uint32_t)std::min<uint64_t>(most, 0xC0000000ull)))) return r;
+        m->dense_hint = hint;
+      }
       // split-brick bitmaps may hold partial ORs of the stopped run: cleared,
       // and any cast enqueued since runs again
       CK(launch_fill_u64(m->cast, m->shared_bits, (uint64_t)m->split_cap * 1024, 0));
@@ -1558,7 +1581,15 @@ int brick_check(vdbgpu_map* m, BrickCast& c) {
   }
   const Status& st = m->h_cst[2 * c.slot];
   const uint32_t recs = st.records;
-  m->dense_hint = std::max(m->dense_hint, std::min<uint32_t>(c.cap, recs + recs / 4 + 64));
+  // (the fullest region counts for all of them: a set that one scan's regions
+  // outgrow makes every set of the ring grow in turn)
+  const uint64_t regions = st.items >= kRecRegionItems ? kRecRegions : 1;
+  const uint64_t room = std::max<uint64_t>(recs, regions * st.rec_most);
+  m->dense_hint = std::max(m->dense_hint, (uint32_t)std::min<uint64_t>(c.cap, room + room / 4 + 64 * regions));
+  if (c.n >= m->guess_rays) {
+    m->guess_rays = c.n;
+    m->guess_recs = (uint32_t)room;
+  }
   m->stats.scans += 1;
   m->stats.rays += st.rays;
   m->stats.visits += st.total;
@@ -1624,9 +1655,9 @@ int run_brick_accumulate(vdbgpu_map* m, Source& src, const float* xyz, int64_t n
   if ((double)need > load * src.cap) {
     const uint64_t cap = next_pow2((uint64_t)((double)need / load) + 1);
     if (cap > (1u << 30)) return fail(m, VDBGPU_DEVICE_ERROR, "update set cannot grow");
-    if (src.pending == 0) {
+    if (src.pending == 0) {  // room for another cloud like this one
       free_update(m, src);
-      if ((r = alloc_update(m, src, (uint32_t)std::max<uint64_t>(kMinUpdateCap, cap)))) return r;
+      if ((r = alloc_update(m, src, (uint32_t)std::max<uint64_t>(kMinUpdateCap, std::min<uint64_t>(cap * 2, 1u << 30))))) return r;
     } else {
       if ((r = grow_update(m, src, (uint32_t)cap))) return r;
       CK(hipMemsetAsync(&m->d_st[2], 0, sizeof(Status), m->stream));
@@ -1823,7 +1854,7 @@ int refresh_snapshot(vdbgpu_map* m) {
 
 // integrateUpdate of several sources: up to kDeferMax update sets, in id
 // order, applied as one group pass that reads and writes each map leaf once
-// (three lidars' sets share most of their leaves: 3.3 -> 1.7 ms with the
+// (three lidars' sets share most of their leaves: 3.3 -> 2.1 ms with the
 // set-up and the clearing). One update per source and voxel in id order, as
 // one pass per source makes them.
 int integrate_groups(vdbgpu_map* m, const std::vector<Source*>& ready, bool ch, bool cm) {
@@ -2549,8 +2580,25 @@ int32_t vdbgpu_insert_batch(vdbgpu_map* m, const char* id, int32_t nscans, const
         const char* on = std::getenv("VDBGPU_GRAPH");
         m->graph_casts = on && on[0] == '1';
       }
-      ~GraphCasts() { m->graph_casts = false; }
+      ~GraphCasts() {
+        m->graph_casts = false;
+        m->batch_rays = 0;
+      }
     } graph_casts(m);
+    // tables for the largest scan at once: growing them between the scans frees
+    // memory, which waits for the device (16 scans of 10,000 to 300,000 points
+    // into a new map: 18.8 ms, 11.4 ms with the tables and record sets sized first)
+    double most_R = 0;
+    for (int i = 0; i < nscans; ++i)
+      if (scan_range(i) > 0 && counts[i] > 0 && counts[i] <= (int64_t)kMaxRays) {
+        m->batch_rays = std::max<int64_t>(m->batch_rays, counts[i]);
+        most_R = std::max(most_R, scan_range(i));
+      }
+    if (m->batch_rays) {
+      int r = ensure_rays(m, (uint32_t)m->batch_rays);
+      if (!r) r = brick_tables(m, m->batch_rays, most_R);
+      if (r) return r;
+    }
     BrickCast prev;
     bool have_prev = false;
     auto finish_prev = [&]() -> int {

@@ -588,7 +588,7 @@ __global__ __launch_bounds__(256) void k_compact(UpdView u, uint32_t cap,
   __shared__ uint32_t s_wave[4], s_base;
   if (st->error != 0 || st->overflow != 0) return;  // same for every thread
   // eight slots per thread and append: at one slot a table of 4 M slots made
-  // 16 k appends to one counter, which was all of its 190 us
+  // 16 k appends to one counter, which was nearly all of its 190 us
   constexpr int kSlots = 8;
   const uint32_t tile = blockDim.x * kSlots;
   for (uint32_t base = blockIdx.x * tile; base < cap; base += gridDim.x * tile) {

@@ -1053,7 +1053,7 @@ int run_pipeline(vdbgpu_map* m, Source& src, const float* xyz, int64_t stride, b
 }
 
 // raycastPointCloud in fast mode (VDBMapping.hpp:520-527, castRayIntoGridFast
-// :577-602) into the source's update set: k_fast_cast marks the map-active
+// :577-602) into the source's update set: k_fast_walk marks the map-active
 // voxels along each ray's runs of existing leaves (topology snapshot of the
 // last fast-mode integrate) plus the endpoint hits; nothing is cast while the
 // map is empty. An update-set overflow grows the set and re-runs (marks are

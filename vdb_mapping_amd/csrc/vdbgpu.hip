@@ -1770,10 +1770,8 @@ void create_flags(const vdbgpu_map* m, bool* ch, bool* cm) {
 // updateVolumeRayIntersectors (VDBMapping.hpp:1436-1449): in fast mode, a
 // non-empty map gets a fresh topology snapshot after every integrate.
 int build_snapshot(vdbgpu_map* m) {
-  if (!m->rt_info) {
-    CK(dalloc(m, &m->rt_info, 1));
-    CK(hipHostMalloc((void**)&m->h_rt_info, sizeof(RtInfo), hipHostMallocDefault));
-  }
+  if (!m->rt_info) CK(dalloc(m, &m->rt_info, 1));
+  if (!m->h_rt_info) CK(hipHostMalloc((void**)&m->h_rt_info, sizeof(RtInfo), hipHostMallocDefault));
   auto tables_fit = [&] {
     return 2 * m->leaf_count_ub + 2 <= m->rt_n128_cap &&
            2 * m->leaf_count_ub + 2 * vdbgpu_map::kNoopCap <= m->rt_n4096_cap;
@@ -1784,7 +1782,7 @@ int build_snapshot(vdbgpu_map* m) {
   if (!tables_fit() && (r = read_status(m))) return r;
   if (!tables_fit()) {
     const uint64_t ub = m->leaf_count_ub;
-    m->has_isect = false;  // until this build is through
+    m->has_isect = false;
     m->rt_full = true;
     dfree(m, &m->rt.n128, m->rt_n128_cap);
     dfree(m, &m->rt.nidx, m->rt_n128_cap);
@@ -1802,7 +1800,10 @@ int build_snapshot(vdbgpu_map* m) {
   m->rt.n128_mask = m->rt_n128_cap - 1;
   m->rt.n4096_mask = m->rt_n4096_cap - 1;
   const bool full = m->rt_full || m->ntiles > 0;
-  m->rt_full = true;  // until this build is through
+  // until this build is through: from the next launch on the node hash may name
+  // nodes that the bitmaps have no room for yet
+  m->rt_full = true;
+  m->has_isect = false;
   const uint32_t first = full ? 0 : m->rt_leaves;
   if (full) {
     CK(launch_fill_u64(m->stream, m->rt.n128, m->rt_n128_cap, kEmpty));

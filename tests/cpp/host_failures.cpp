@@ -37,6 +37,7 @@ std::map<std::string, int> g_launches;
 std::map<const void*, size_t> g_blocks;  // live allocations
 long g_fail_in = 0;                      // the n-th allocation from here fails (0: none)
 bool g_failed = false;
+size_t g_pinned = 0;  // bytes ever allocated as pinned memory
 
 // The plain name of a kernel's symbol, _ZN6vdbgpu<length>k_name...
 std::string plain(const char* mangled) {
@@ -103,7 +104,10 @@ int hipLaunchKernel(const void* host, Dim3, Dim3, void** args, size_t, void*) {
 }
 int hipMalloc(void** p, size_t bytes) { return allocate(p, bytes); }
 int hipFree(void* p) { return release(p); }
-int hipHostMalloc(void** p, size_t bytes, unsigned) { return allocate(p, bytes); }
+int hipHostMalloc(void** p, size_t bytes, unsigned) {
+  g_pinned += bytes;
+  return allocate(p, bytes);
+}
 int hipHostFree(void* p) { return release(p); }
 int hipHostGetDevicePointer(void** d, void* h, unsigned) {
   *d = h;
@@ -248,10 +252,54 @@ void snapshot() {
   }
 }
 
+// Map sections: pinned staging comes a few chunks a read and stays bounded; a
+// refused chunk is done without, a refused device buffer fails the read alone.
+void section() {
+  unsigned int leaves = 1100;
+  g_kernels["k_compact"] = [](void** a) { *arg<unsigned int*>(a, 3) = 1; };
+  g_kernels["k_scan_u64"] = [&](void** a) { *arg<unsigned int*>(a, 3) = leaves; };
+  const int32_t box[6] = {0, 0, 0, 255, 255, 255};  // 32,768 cells
+  std::vector<int32_t> o(3 * 32768);
+  std::vector<float> v((size_t)512 * 32768);
+  std::vector<uint64_t> w(8 * 32768);
+  auto read = [&](vdbgpu_map* m) {
+    return vdbgpu_export_section(m, box, 1, o.data(), v.data(), w.data(), 32768);
+  };
+  vdbgpu_map* m = new_map(false);
+  CHECK(edit(m) == VDBGPU_OK);
+  const size_t start = g_pinned;
+  for (int k = 0; k < 40; ++k) {
+    const size_t before = g_pinned;
+    leaves = k < 20 ? 1100 : 30000;
+    CHECK(read(m) == leaves);
+    CHECK(g_pinned - before <= (size_t)leaves * 2124 / 3 + (1 << 20));
+  }
+  CHECK(g_pinned - start <= 16u << 20);
+  CHECK(vdbgpu_release_scratch(m) == VDBGPU_OK && read(m) == leaves);
+  close_map(m);
+  bool through = false;
+  for (long k = 1; !through; ++k) {
+    m = new_map(false);
+    CHECK(edit(m) == VDBGPU_OK);
+    leaves = 200;
+    CHECK(read(m) == 200);
+    leaves = 3000;
+    g_fail_in = k;
+    g_failed = false;
+    const int64_t n = read(m);
+    through = !g_failed;
+    g_fail_in = 0;
+    CHECK(n == 3000 || (g_failed && n == -1));
+    CHECK(read(m) == 3000 && read(m) == 3000);
+    close_map(m);
+    CHECK(k > 1 || !through);
+  }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
-  const std::map<std::string, void (*)()> scenarios = {{"snapshot", snapshot}};
+  const std::map<std::string, void (*)()> scenarios = {{"snapshot", snapshot}, {"section", section}};
   const auto s = argc > 1 ? scenarios.find(argv[1]) : scenarios.end();
   if (s == scenarios.end()) return 3;
   s->second();

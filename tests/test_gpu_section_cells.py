@@ -1,6 +1,6 @@
 """Map sections by the cells of their box against the oracle: boxes cut through leaves on every side, one voxel, one
 leaf, around the 16 cells of a workgroup, at the ends of the coordinate range, larger than the map, more cells than
-the path takes, staging that grows between calls, and caps one too small."""
+the path takes, staging that grows between calls (pinned chunks, the rest in device memory), and caps one too small."""
 import numpy as np
 import pytest
 
@@ -64,3 +64,14 @@ def test_tiles_are_not_section_leaves():
     both(g, o, "create_map_from_points", p, True, True)
     for full in (True, False):
         same_section(g, o, [-30] * 3 + [30] * 3, full)
+
+
+@pytest.mark.parametrize("sizes", [[255, 256, 257], [300, 300, 512, 513, 511], [4096, 4097, 4095, 1], [6000] * 20 + [100]])
+def test_staging_chunks(sizes):
+    """Sections around the 256 leaves of a pinned chunk and the 16 chunks of a map, read while the chunks still grow."""
+    g, o = pair(1.0, 8.0, **PROBS)
+    p = np.zeros((6000, 3), np.float32) + 0.5
+    p[:, 0] += 8 * np.arange(6000)  # a row of leaves: a box of n cells holds n of them
+    both(g, o, "add_points_to_grid", p)
+    for k, n in enumerate(sizes):
+        assert same_section(g, o, [0, 0, 0, 8 * n - 1, 7, 7], k % 3 != 1) == n

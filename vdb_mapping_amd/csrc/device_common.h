@@ -225,6 +225,18 @@ struct SectionBox {
   int box[6];
 };
 constexpr uint32_t kSectionCells = 16;  // cells per workgroup
+// Where the leaves of a section go, in cell order: the first `pinned` of them
+// into host-visible chunks of kSectionChunk leaves, the others up to `cap` into
+// `rest`. A chunk of k leaves holds their values, then their masks, then their
+// origins (2,048, 64 and 12 bytes each); so does rest, for cap - pinned leaves.
+constexpr uint32_t kSectionChunk = 256;
+constexpr uint32_t kSectionChunks = 16;
+constexpr size_t kSectionLeaf = 2048 + 64 + 12;
+struct SectionDest {
+  char* chunk[kSectionChunks];
+  char* rest;
+  uint32_t pinned, cap;
+};
 
 constexpr uint32_t kRtNodeWords = 128;  // words of RtView::bits per node
 // What a snapshot build hands back: bbox (min, max) of leaves with an active

@@ -345,13 +345,12 @@ __global__ __launch_bounds__(256) void k_section_cells(MapView mp, SectionBox sb
   if (threadIdx.x == 0) bsum[blockIdx.x] = s_n[0] + s_n[1] + s_n[2] + s_n[3];
 }
 
-// The picked cells' leaves at their ranks (host-visible memory: each wave
+// The picked cells' leaves at their ranks (host-visible memory mostly: each wave
 // writes its leaf's 2 KiB as one run). Full: every inside voxel from the
 // leaf's first creating one on keeps its value; sparse: active ones are 1.
 __global__ __launch_bounds__(256) void k_section_rows(MapView mp, SectionBox sb, uint32_t cells, uint32_t full,
-                                                      const uint32_t* __restrict__ cell,
-                                                      const uint64_t* __restrict__ boff, uint32_t cap, int* origins,
-                                                      float* values, unsigned long long* masks) {
+                                                      uint32_t values, const uint32_t* __restrict__ cell,
+                                                      const uint64_t* __restrict__ boff, SectionDest dest) {
   const int lane = lane_id(), w = threadIdx.x >> 6;
   const uint32_t c0 = blockIdx.x * kSectionCells;
   const uint32_t mine = lane < (int)kSectionCells && c0 + lane < cells ? cell[c0 + lane] : kNone;
@@ -361,7 +360,15 @@ __global__ __launch_bounds__(256) void k_section_rows(MapView mp, SectionBox sb,
     const int k = w * (int)(kSectionCells / 4) + (int)q;
     if (!((picked >> k) & 1)) continue;  // the whole wave
     const uint64_t at = boff[blockIdx.x] + (uint64_t)__popcll(picked & ((1ull << k) - 1));
-    if (at >= cap) return;
+    if (at >= dest.cap) return;
+    const bool pinned = at < dest.pinned;
+    char* base = dest.rest;
+    uint32_t leaves = dest.cap - dest.pinned, i = (uint32_t)at - dest.pinned;
+    if (pinned) {
+      base = dest.chunk[at / kSectionChunk];
+      leaves = kSectionChunk;
+      i = (uint32_t)at % kSectionChunk;
+    }
     const uint32_t idx = __shfl(mine, k, 64);
     int o[3];
     cell_origin(sb, c0 + (uint32_t)k, o);
@@ -387,15 +394,17 @@ __global__ __launch_bounds__(256) void k_section_rows(MapView mp, SectionBox sb,
     if (!(keep & 64u)) r.b.z = 0.f;
     if (!(keep & 128u)) r.b.w = 0.f;
     if (values) {
-      float4* out = reinterpret_cast<float4*>(values) + at * 128 + 2 * lane;
+      float4* out = reinterpret_cast<float4*>(base) + (size_t)i * 128 + 2 * lane;
       out[0] = r.a;
       out[1] = r.b;
     }
     uint64_t m = (uint64_t)(r.in & r.act) << ((lane & 7) * 8);
 #pragma unroll
     for (int s = 1; s < 8; s <<= 1) m |= __shfl_xor(m, s, 64);
-    if (masks && (lane & 7) == 0) masks[at * 8 + (lane >> 3)] = m;
-    if (origins && lane < 3) origins[at * 3 + lane] = lane == 0 ? o[0] : (lane == 1 ? o[1] : o[2]);
+    char* heads = base + (size_t)leaves * 2048;
+    if ((lane & 7) == 0) reinterpret_cast<unsigned long long*>(heads)[(size_t)i * 8 + (lane >> 3)] = m;
+    if (lane < 3)
+      reinterpret_cast<int*>(heads + (size_t)leaves * 64)[(size_t)i * 3 + lane] = lane == 0 ? o[0] : (lane == 1 ? o[1] : o[2]);
   }
 }
 
@@ -893,12 +902,11 @@ hipError_t launch_section_cells(hipStream_t s, MapView mp, const SectionBox& sb,
   return launch_scan_u64(s, bsum, boff, nb, total);
 }
 
-hipError_t launch_section_rows(hipStream_t s, MapView mp, const SectionBox& sb, uint32_t cells, bool full,
-                               const uint32_t* cell, const uint64_t* boff, uint32_t cap, int* origins, float* values,
-                               unsigned long long* masks) {
+hipError_t launch_section_rows(hipStream_t s, MapView mp, const SectionBox& sb, uint32_t cells, bool full, bool values,
+                               const uint32_t* cell, const uint64_t* boff, const SectionDest& dest) {
   const uint32_t nb = (cells + kSectionCells - 1) / kSectionCells;
-  hipLaunchKernelGGL(k_section_rows, dim3(nb), dim3(256), 0, s, mp, sb, cells, full ? 1u : 0u, cell, boff, cap,
-                     origins, values, masks);
+  hipLaunchKernelGGL(k_section_rows, dim3(nb), dim3(256), 0, s, mp, sb, cells, full ? 1u : 0u, values ? 1u : 0u, cell,
+                     boff, dest);
   return hipGetLastError();
 }
 

@@ -126,9 +126,8 @@ hipError_t launch_snapshot_bits(hipStream_t s, MapView mp, uint32_t first, uint3
 // (edit_kernels.hip); then the leaves, in cell order, up to cap of them.
 hipError_t launch_section_cells(hipStream_t s, MapView mp, const SectionBox& sb, uint32_t cells, bool full,
                                 uint32_t* cell, uint64_t* bsum, uint64_t* boff, unsigned int* total, TileView tv);
-hipError_t launch_section_rows(hipStream_t s, MapView mp, const SectionBox& sb, uint32_t cells, bool full,
-                               const uint32_t* cell, const uint64_t* boff, uint32_t cap, int* origins, float* values,
-                               unsigned long long* masks);
+hipError_t launch_section_rows(hipStream_t s, MapView mp, const SectionBox& sb, uint32_t cells, bool full, bool values,
+                               const uint32_t* cell, const uint64_t* boff, const SectionDest& dest);
 // Active points in value-on order (edit_kernels.hip): the leaves that hold some (st->entries of them, st->total
 // points), then the points.
 hipError_t launch_point_leaves(hipStream_t s, MapView mp, uint64_t leaf_bound, const Status* stmap, TileView tv,

@@ -139,7 +139,7 @@ struct vdbgpu_map {
   RtView rt{};
   uint32_t rt_n128_cap = 0, rt_n4096_cap = 0, rt_node_cap = 0;
   RtInfo* rt_info = nullptr;    // device
-  RtInfo* h_rt_info = nullptr;  // pinned
+  RtInfo* h_rt_info = nullptr;  // in h_block
   // pool leaves the snapshot covers; the next build adds the ones after them,
   // or starts over (rt_full: the grid was emptied, tiles came or went)
   uint32_t rt_leaves = 0, rt_nodes = 0;
@@ -253,14 +253,18 @@ struct vdbgpu_map {
   uint64_t pt_cap = 0;
   float* pt_xyz = nullptr;
   uint64_t pt_xyz_cap = 0;
-  // map sections by cells: cell table and its block sums, and the pinned
-  // staging buffer that the section's leaves are written to
+  // map sections by cells: cell table and its block sums, and the buffers that
+  // the section's leaves are written to, pinned chunks of kSectionChunk leaves
+  // (the first one in h_block) and for the leaves after them a device one of sec_cap
   uint32_t* sec_cell = nullptr;
   uint64_t* sec_sums = nullptr;  // sums, then their scan
   uint32_t sec_cells = 0;
-  char* h_sec = nullptr;
-  uint32_t sec_cap = 0;  // leaves the staging buffer holds
-  bool sec_again = false;  // a section was read before
+  char* h_sec[kSectionChunks] = {};
+  char* hd_sec[kSectionChunks] = {};  // their device addresses
+  uint32_t sec_chunks = 0;
+  uint32_t sec_pinned = kSectionChunk;  // leaves of the chunks that are used
+  char* d_sec = nullptr;
+  uint32_t sec_cap = 0;
 
   // direct edits (addPointsToGrid / removePointsFromGrid) and artificial areas
   Source edit;                 // marked voxels of one edit call (cleared after it)
@@ -272,6 +276,9 @@ struct vdbgpu_map {
   bool art_leaves = false;     // every artificial leaf exists in the map
   std::vector<double> art_verts;  // walls added since the last restore: vertices (x, y, z)
   std::vector<int> art_walls;     // and {a, b, k0, k1} per wall
+
+  // pinned memory of the handle in one block (HostBlock, then the section staging)
+  char* h_block = nullptr;
 
   // status: [0] scan, [1] map (leaf_count), [2] auxiliary, [3] cumulative counters
   Status* d_st = nullptr;
@@ -1771,7 +1778,6 @@ void create_flags(const vdbgpu_map* m, bool* ch, bool* cm) {
 // non-empty map gets a fresh topology snapshot after every integrate.
 int build_snapshot(vdbgpu_map* m) {
   if (!m->rt_info) CK(dalloc(m, &m->rt_info, 1));
-  if (!m->h_rt_info) CK(hipHostMalloc((void**)&m->h_rt_info, sizeof(RtInfo), hipHostMallocDefault));
   auto tables_fit = [&] {
     return 2 * m->leaf_count_ub + 2 <= m->rt_n128_cap &&
            2 * m->leaf_count_ub + 2 * vdbgpu_map::kNoopCap <= m->rt_n4096_cap;
@@ -2166,6 +2172,7 @@ uint64_t walk_scratch(vdbgpu_map* m, bool release) {
   one(m->pt_xyz, m->pt_xyz_cap);
   one(m->sec_cell, m->sec_cells);
   one(m->sec_sums, (size_t)m->sec_cells / kSectionCells * 2);
+  one(m->d_sec, (size_t)m->sec_cap * kSectionLeaf);
   one(m->q_in, (size_t)m->q_cap * 7);
   one(m->q_succ, (size_t)m->q_cap);
   one(m->q_end, (size_t)m->q_cap * 3);
@@ -2179,8 +2186,8 @@ uint64_t walk_scratch(vdbgpu_map* m, bool release) {
   for (auto& kv : m->sources) upd(kv.second);
   upd(m->edit);
   if (release) {
-    if (m->h_sec) (void)hipHostFree(m->h_sec);
-    m->h_sec = nullptr;
+    for (; m->sec_chunks > 1; --m->sec_chunks) (void)hipHostFree(m->h_sec[m->sec_chunks - 1]);
+    m->sec_pinned = kSectionChunk;
     m->sec_cells = m->sec_cap = 0;
     m->f_groups = m->f_rays = 0;
     m->pt_cap = m->pt_xyz_cap = 0;
@@ -2268,9 +2275,38 @@ static bool create_rec_events(vdbgpu_map* m) {
     if (hipEventCreateWithFlags(&m->rec_free[i], hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&m->ins_done[i], hipEventDisableTiming) != hipSuccess)
       return false;
-  return hipHostMalloc((void**)&m->h_lc, vdbgpu_map::kRecSets * sizeof(uint32_t), hipHostMallocDefault) ==
-             hipSuccess &&
-         hipHostGetDevicePointer((void**)&m->d_lc, m->h_lc, 0) == hipSuccess;
+  return true;
+}
+
+// The handle's pinned memory, allocated once: a call to hipHostMalloc takes
+// 50-100 us whatever its size (below 2 MB), and the host's first access to each
+// of its pages another 1.6 us, so nothing is touched here that is not used.
+static bool create_host_block(vdbgpu_map* m) {
+  struct HostBlock {
+    Status st[4], cst[4];
+    ScanInfo scans[kMaxBatchScans];
+    BatchCtl ctl;
+    RtInfo rt;
+    uint32_t lc[vdbgpu_map::kRecSets];
+  };
+  constexpr size_t head = (sizeof(HostBlock) + 255) & ~(size_t)255;
+  char* d = nullptr;
+  if (hipHostMalloc((void**)&m->h_block, head + kSectionChunk * kSectionLeaf, hipHostMallocDefault) != hipSuccess ||
+      hipHostGetDevicePointer((void**)&d, m->h_block, 0) != hipSuccess)
+    return false;
+  HostBlock* b = reinterpret_cast<HostBlock*>(m->h_block);
+  memset(b, 0, sizeof *b);
+  m->h_st = b->st;
+  m->h_cst = b->cst;
+  m->h_scans = b->scans;
+  m->h_ctl = &b->ctl;
+  m->h_rt_info = &b->rt;
+  m->h_lc = b->lc;
+  m->d_lc = reinterpret_cast<uint32_t*>(d + ((char*)b->lc - m->h_block));
+  m->h_sec[0] = m->h_block + head;
+  m->hd_sec[0] = d + head;
+  m->sec_chunks = 1;
+  return true;
 }
 
 int32_t vdbgpu_create(double resolution, vdbgpu_map** out) {
@@ -2291,10 +2327,8 @@ int32_t vdbgpu_create(double resolution, vdbgpu_map** out) {
     m->num_cu = cu;
   if (hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking) != hipSuccess ||
       hipStreamCreateWithFlags(&m->cast, hipStreamNonBlocking) != hipSuccess ||
-      !create_rec_events(m) ||
+      !create_rec_events(m) || !create_host_block(m) ||
       hipMalloc((void**)&m->d_st, 4 * sizeof(Status)) != hipSuccess ||
-      hipHostMalloc((void**)&m->h_st, 4 * sizeof(Status), hipHostMallocDefault) != hipSuccess ||
-      hipHostMalloc((void**)&m->h_cst, 4 * sizeof(Status), hipHostMallocDefault) != hipSuccess ||
       hipMalloc((void**)&m->d_dest, sizeof(RecDest)) != hipSuccess ||
       hipMalloc((void**)&m->d_rcnt, kRecRegions * kRecCountStride * sizeof(unsigned int)) != hipSuccess ||
       hipEventCreateWithFlags(&m->cst_done[0], hipEventDisableTiming) != hipSuccess ||
@@ -2303,12 +2337,8 @@ int32_t vdbgpu_create(double resolution, vdbgpu_map** out) {
     vdbgpu_destroy(m);
     return VDBGPU_DEVICE_ERROR;
   }
-  memset(m->h_st, 0, 4 * sizeof(Status));
-  memset(m->h_cst, 0, 4 * sizeof(Status));
   if (hipMalloc((void**)&m->d_scans, kMaxBatchScans * sizeof(ScanInfo)) != hipSuccess ||
       hipMalloc((void**)&m->d_ctl, sizeof(BatchCtl)) != hipSuccess ||
-      hipHostMalloc((void**)&m->h_scans, kMaxBatchScans * sizeof(ScanInfo), hipHostMallocDefault) != hipSuccess ||
-      hipHostMalloc((void**)&m->h_ctl, sizeof(BatchCtl), hipHostMallocDefault) != hipSuccess ||
       hipMalloc((void**)&m->noop4096, vdbgpu_map::kNoopCap * 8) != hipSuccess ||
       launch_fill_u64(m->stream, m->noop4096, vdbgpu_map::kNoopCap, kEmpty) != hipSuccess) {
     vdbgpu_destroy(m);
@@ -2363,7 +2393,6 @@ void vdbgpu_destroy(vdbgpu_map* m) {
     if (m->rec_free[i]) (void)hipEventDestroy(m->rec_free[i]);
     if (m->ins_done[i]) (void)hipEventDestroy(m->ins_done[i]);
   }
-  if (m->h_lc) (void)hipHostFree(m->h_lc);
   dfree(m, &m->gslot, m->gslot_cap);
   dfree(m, &m->rgrp, m->rgrp_cap);
   dfree(m, &m->gl, m->grp_cap);
@@ -2377,7 +2406,6 @@ void vdbgpu_destroy(vdbgpu_map* m) {
   dfree(m, &m->rt.bits, (size_t)m->rt_node_cap * kRtNodeWords);
   dfree(m, &m->rt.n4096, m->rt_n4096_cap);
   dfree(m, &m->rt_info, 1);
-  if (m->h_rt_info) (void)hipHostFree(m->h_rt_info);
   dfree(m, &m->q_in, (size_t)m->q_cap * 7);
   dfree(m, &m->q_succ, (size_t)m->q_cap);
   dfree(m, &m->q_end, (size_t)m->q_cap * 3);
@@ -2391,23 +2419,21 @@ void vdbgpu_destroy(vdbgpu_map* m) {
   dfree(m, &m->pt_xyz, m->pt_xyz_cap);
   dfree(m, &m->sec_cell, m->sec_cells);
   dfree(m, &m->sec_sums, (size_t)m->sec_cells / kSectionCells * 2);
-  if (m->h_sec) (void)hipHostFree(m->h_sec);
+  dfree(m, &m->d_sec, (size_t)m->sec_cap * kSectionLeaf);
+  for (; m->sec_chunks > 1; --m->sec_chunks) (void)hipHostFree(m->h_sec[m->sec_chunks - 1]);
   if (m->noop4096) (void)hipFree(m->noop4096);
   if (m->d_scans) (void)hipFree(m->d_scans);
   if (m->d_ctl) (void)hipFree(m->d_ctl);
-  if (m->h_scans) (void)hipHostFree(m->h_scans);
-  if (m->h_ctl) (void)hipHostFree(m->h_ctl);
   dfree(m, &m->gkeys, m->gcap);
   dfree(m, &m->gscans, (size_t)m->gcap * 2);
   dfree(m, &m->gneed, m->gcap);
   dfree(m, &m->glist, m->gcap);
   dfree(m, &m->gidx, m->gcap);
   if (m->d_st) (void)hipFree(m->d_st);
-  if (m->h_st) (void)hipHostFree(m->h_st);
   drop_cast_graphs(m);
   if (m->d_dest) (void)hipFree(m->d_dest);
   if (m->d_rcnt) (void)hipFree(m->d_rcnt);
-  if (m->h_cst) (void)hipHostFree(m->h_cst);
+  if (m->h_block) (void)hipHostFree(m->h_block);
   for (hipEvent_t e : m->cst_done)
     if (e) (void)hipEventDestroy(e);
   for (auto& t : m->timed) {
@@ -3538,7 +3564,7 @@ int64_t vdbgpu_export_artificial(vdbgpu_map* m, int32_t* origins, uint64_t* mask
 namespace {
 
 // Boxes of more leaf cells than this scan the pool instead (and are sorted on
-// the host); the staging buffer stays below 280 MB.
+// the host).
 constexpr uint64_t kMaxSectionCells = 1u << 17;
 
 // The box's leaf cells, clipped to the leaf key range; their number in *cells.
@@ -3558,12 +3584,16 @@ SectionBox section_box(const int32_t bbox[6], uint64_t* cells) {
   return sb;
 }
 
-// Section of at most kMaxSectionCells cells. A map's first section is gathered
-// in device memory and copied. From the second on (a program that reads one
-// after every scan) the leaves are written straight into a pinned staging
-// buffer, guessed to hold them as it held the last section; when it does not,
-// it grows and they are written again. Pinning it costs about a millisecond,
-// which a single read would not win back.
+// Section of at most kMaxSectionCells cells. Its first leaves are written straight
+// into pinned chunks (no copy is queued: the section of a 2,000-point room map
+// takes 50 us, with copies 110), the ones after them into a device buffer that is kept, and copied
+// to the caller's memory from there. Both are written before the count is known;
+// a device buffer found too small costs one more launch.
+//
+// The host's first access to a page of pinned memory takes 1.6 us, so a map comes to
+// use its chunks by and by, an eighth of a section more with each read of one: pinning
+// all 1,100 leaves of a section with the second read made that read 1,604 us, where
+// gathering and sorting on the host had taken 870 (now 560, and 225 once all are pinned).
 int64_t export_section_cells(vdbgpu_map* m, const SectionBox& sb, uint32_t cells, bool full, int32_t* origins,
                              float* values, uint64_t* masks, int64_t cap) {
   const uint32_t want = (cells + 255) / 256 * 256;
@@ -3579,51 +3609,64 @@ int64_t export_section_cells(vdbgpu_map* m, const SectionBox& sb, uint32_t cells
   CKN(launch_section_cells(m->stream, map_view(m), sb, cells, full, m->sec_cell, m->sec_sums, boff,
                            &m->d_st[2].entries, tile_view(m)));
   const bool out = origins || values || masks;
-  auto rows = [&]() -> hipError_t {
-    char* p = nullptr;
-    const hipError_t e = hipHostGetDevicePointer((void**)&p, m->h_sec, 0);
-    if (e != hipSuccess) return e;
-    return launch_section_rows(m->stream, map_view(m), sb, cells, full, m->sec_cell, boff, m->sec_cap,
-                               (int*)(p + (size_t)m->sec_cap * 2112), values ? (float*)p : nullptr,
-                               (unsigned long long*)(p + (size_t)m->sec_cap * 2048));
+  const uint32_t pinned = m->sec_pinned;
+  auto rows = [&]() {
+    SectionDest d{};
+    std::copy(m->hd_sec, m->hd_sec + m->sec_chunks, d.chunk);
+    d.rest = m->d_sec;
+    d.pinned = pinned;
+    d.cap = pinned + m->sec_cap;
+    return launch_section_rows(m->stream, map_view(m), sb, cells, full, values != nullptr, m->sec_cell, boff, d);
   };
-  if (out && m->sec_cap) CKN(rows());
+  if (out) CKN(rows());
   if (read_status(m)) return -1;
   const uint32_t n = m->h_st[2].entries;
   if (!out) return n;
   if ((int64_t)n > cap) return -(int64_t)n;
-  if (n == 0) return 0;
-  if (!m->sec_again) {
-    m->sec_again = true;
-    char* d = nullptr;
-    CKN(dalloc(m, &d, (size_t)n * 2124));
-    int* d_o = (int*)(d + (size_t)n * 2112);
-    unsigned long long* d_a = (unsigned long long*)(d + (size_t)n * 2048);
-    const hipError_t e = [&]() -> hipError_t {
-      hipError_t e = launch_section_rows(m->stream, map_view(m), sb, cells, full, m->sec_cell, boff, n, d_o,
-                                         values ? (float*)d : nullptr, d_a);
-      if (!e && values) e = hipMemcpyAsync(values, d, (size_t)n * 2048, hipMemcpyDeviceToHost, m->stream);
-      if (!e && masks) e = hipMemcpyAsync(masks, d_a, (size_t)n * 64, hipMemcpyDeviceToHost, m->stream);
-      if (!e && origins) e = hipMemcpyAsync(origins, d_o, (size_t)n * 12, hipMemcpyDeviceToHost, m->stream);
-      return e ? e : hipStreamSynchronize(m->stream);
-    }();
-    dfree(m, &d, (size_t)n * 2124);
-    CKN(e);
-    return n;
-  }
-  if (n > m->sec_cap) {
-    if (m->h_sec) (void)hipHostFree(m->h_sec);
-    m->h_sec = nullptr;
+  const uint32_t rest = n > pinned ? n - pinned : 0;
+  if (rest > m->sec_cap) {
+    dfree(m, &m->d_sec, (size_t)m->sec_cap * kSectionLeaf);
     m->sec_cap = 0;
-    const uint32_t room = std::min(cells, std::max<uint32_t>(256, n + n / 4));
-    CKN(hipHostMalloc((void**)&m->h_sec, (size_t)room * 2124, hipHostMallocDefault));
+    const uint32_t room = std::min(cells, rest + rest / 4);
+    CKN(dalloc(m, &m->d_sec, (size_t)room * kSectionLeaf));
     m->sec_cap = room;
     CKN(rows());
+  }
+  if (rest) {
+    const char* a = m->d_sec + (size_t)m->sec_cap * 2048;
+    if (values)
+      CKN(hipMemcpyAsync(values + (size_t)pinned * 512, m->d_sec, (size_t)rest * 2048, hipMemcpyDeviceToHost, m->stream));
+    if (masks) CKN(hipMemcpyAsync(masks + (size_t)pinned * 8, a, (size_t)rest * 64, hipMemcpyDeviceToHost, m->stream));
+    if (origins)
+      CKN(hipMemcpyAsync(origins + (size_t)pinned * 3, a + (size_t)m->sec_cap * 64, (size_t)rest * 12,
+                         hipMemcpyDeviceToHost, m->stream));
     CKN(hipStreamSynchronize(m->stream));
   }
-  if (values) std::memcpy(values, m->h_sec, (size_t)n * 2048);
-  if (masks) std::memcpy(masks, m->h_sec + (size_t)m->sec_cap * 2048, (size_t)n * 64);
-  if (origins) std::memcpy(origins, m->h_sec + (size_t)m->sec_cap * 2112, (size_t)n * 12);
+  const uint32_t head = std::min(n, pinned);
+  for (uint32_t c = 0, at = 0; at < head; ++c, at += kSectionChunk) {
+    const uint32_t k = std::min(head - at, kSectionChunk);
+    const char* h = m->h_sec[c];
+    if (values) std::memcpy(values + (size_t)at * 512, h, (size_t)k * 2048);
+    if (masks) std::memcpy(masks + (size_t)at * 8, h + (size_t)kSectionChunk * 2048, (size_t)k * 64);
+    if (origins) std::memcpy(origins + (size_t)at * 3, h + (size_t)kSectionChunk * 2112, (size_t)k * 12);
+  }
+  if (rest) {  // more of the next section through pinned memory
+    const uint32_t more = std::min(std::min(pinned + n / 8 + 32, n), kSectionChunks * kSectionChunk);
+    while (m->sec_chunks * kSectionChunk < more) {
+      char*& h = m->h_sec[m->sec_chunks];
+      if (hipHostMalloc((void**)&h, kSectionChunk * kSectionLeaf, hipHostMallocDefault) != hipSuccess) {
+        (void)refused();
+        break;
+      }
+      if (hipHostGetDevicePointer((void**)&m->hd_sec[m->sec_chunks], h, 0) != hipSuccess) {
+        (void)refused();
+        (void)hipHostFree(h);
+        break;
+      }
+      ++m->sec_chunks;
+    }
+    m->sec_pinned = std::max(pinned, std::min(more, m->sec_chunks * kSectionChunk));
+  }
   return n;
 }
 

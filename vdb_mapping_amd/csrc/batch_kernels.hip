@@ -43,7 +43,7 @@ __device__ __forceinline__ uint32_t find_slot(const unsigned long long* __restri
     const unsigned long long k = keys[h];
     if (k == key) return h;
     if (k == kEmpty) return kNone;
-    h = (h + 1) & mask;
+    h = (h + kUpdStep) & mask;
   }
   return kNone;
 }

@@ -1022,7 +1022,7 @@ __global__ __launch_bounds__(256) void k_merge_records(UpdView rec, RecIndex ri,
         slot = h;
         break;
       }
-      h = (h + 1) & u.cap_mask;
+      h = (h + kUpdStep) & u.cap_mask;
     }
   }
   s_slot[threadIdx.x] = slot;

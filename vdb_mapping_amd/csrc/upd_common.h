@@ -40,7 +40,7 @@ __device__ __forceinline__ uint32_t upd_slot(const UpdView& u, uint64_t key, uns
       const unsigned long long prev = atomicCAS(&u.keys[h], kEmpty, (unsigned long long)key);
       if (prev == kEmpty || prev == key) return h;
     }
-    h = (h + 1) & u.cap_mask;
+    h = (h + kUpdStep) & u.cap_mask;
   }
   atomicOr(ovf, kOvfHard);
   return kNone;

@@ -90,3 +90,14 @@ def test_rejected_cloud_leaves_the_set():
     far = np.array([[9e5, 0, 0]], np.float32)
     assert g.accumulate("test", far, [0, 0, 0]) == V.OUT_OF_RANGE
     same_update(g, o, "test")
+
+
+def test_record_sets_stay_two():
+    """A map that only accumulates takes two record sets, not the ring of deferred scans."""
+    g, _ = pair(0.1, 8.0, **PROBS)
+    bytes_at = []
+    for k in range(6):
+        assert g.accumulate("test", cloud(20000, k), [0, 0, 0]) == V.OK
+        bytes_at.append(g.stats()["scratch_bytes"])
+    leaves = len(g.export_update("test")[0])
+    assert bytes_at[1] - bytes_at[0] <= 2 * 140 * leaves and bytes_at[5] - bytes_at[1] <= 2 * 140 * leaves

@@ -427,8 +427,9 @@ uint64_t ledger_since(const vdbgpu_map* m, uint64_t q) {
 // while the map stream may still be busy: the leaf count `cast_lc` that the
 // cast stream read after waiting for an event at ledger position cast_q, or
 // the newest map-insert snapshot already complete (no wait), each plus the
-// leaves enqueued after it; the smaller bound is used. Both kinds of
-// positions only grow, so ledger entries before both are dropped.
+// leaves enqueued after it; the smaller bound is used. Ledger entries before
+// both positions are dropped: what the cast stream has once waited for every
+// later snapshot of that stream holds too, whatever set its scan uses.
 uint64_t leaf_bound(vdbgpu_map* m, uint32_t cast_lc, uint64_t cast_q) {
   uint64_t best = (uint64_t)cast_lc + ledger_since(m, cast_q);
   uint64_t q = cast_q;
@@ -1324,6 +1325,7 @@ struct BrickCast {
   ScanInfo sc{};
   int X = 0;     // record set
   int slot = 0;  // host status slot: m->h_cst[2 slot] (scan), [2 slot + 1] (map snapshot)
+  bool alone = false;  // an accumulated cloud: its records are merged before the next cast
   uint32_t cap = 0;    // capacity of set X when it was cast
   uint64_t epoch = 0;  // m->cast_epoch then
 };
@@ -1479,35 +1481,36 @@ int brick_enqueue(vdbgpu_map* m, BrickCast& c, int attempt) {
   const int nb = cut_blocks(m, c.n), spread = cut_spread(m, c.n);
   if (attempt == 0) {
     // record set X: free once the map stream has applied the scan that last used it
-    c.X = m->rec_cur;
+    // (an accumulated cloud's set is free again once it is merged: two take turns)
+    c.X = c.alone ? m->rec_cur & 1 : m->rec_cur;
     m->rec_cur = (c.X + 1) % m->rec_sets;
     c.slot = m->cst_next;
     m->cst_next ^= 1;
     CK(hipStreamWaitEvent(cs, m->rec_free[c.X], 0));
-    if (m->dense_hint == 0 && m->dcap[c.X] == 0) {
-      // the map's first scan: a guess of its records, for this set alone (a
-      // third of what a lidar sees outdoors, several times a room's; too small a
-      // set only costs another cast)
-      const double leaves = std::sqrt((double)c.n) * std::min(c.sc.R * m->inv, (double)kMaxTableN);
-      if ((r = grow_set(m, c.X, (uint32_t)std::max(4096.0, std::min(leaves, 1048576.0))))) return r;
-      m->dense_hint = 0;
-    } else if (const int64_t most = std::max(c.n, m->batch_rays); m->guess_recs && most > m->guess_rays) {
+    uint32_t want = m->dense_hint;
+    const int64_t most = std::max(c.n, m->batch_rays);
+    if (want == 0) {
+      // the map's first scan: its records are guessed, on the large side (a set too
+      // small costs another cast: 65,536 outdoor rays of 500 voxels 1.4 ms for the
+      // first scan with a quarter of this, 0.9 ms), at most 2^21 of them (290 MB)
+      const double g = 4.0 * std::sqrt((double)c.n) * std::min(c.sc.R * m->inv, (double)kMaxTableN);
+      want = (uint32_t)std::max(4096.0, std::min(g, 2097152.0));
+    } else if (m->guess_recs && most > m->guess_rays) {
       // more rays than any scan so far (or a batch's largest): update leaves
-      // grow with about the root of the rays of one scene; too small a set only
-      // costs another cast. At most 2^21 records (280 MB) on a guess.
+      // grow with about the root of the rays of one scene
       const double g = 1.25 * m->guess_recs * std::sqrt((double)most / (double)m->guess_rays);
-      m->dense_hint = std::max(m->dense_hint, (uint32_t)std::min(g, 2097152.0));
-      m->guess_rays = most;
-      m->guess_recs = m->dense_hint - m->dense_hint / 5;
+      want = std::max(want, (uint32_t)std::min(g, 2097152.0));
     }
-    if (m->dcap[c.X] < m->dense_hint) {  // a first use of set X: size it like the others
-      CK(hipStreamSynchronize(cs));      // (the map stream is done with it)
-      if ((r = grow_set(m, c.X, m->dense_hint))) return r;
-      // the ring's sets never used yet are sized now as well, so the next
-      // scans of the ring do not each stop the cast stream for an allocation
-      for (int y = 0; y < m->rec_sets; ++y)
-        if (m->dcap[y] == 0 && (r = grow_set(m, y, m->dense_hint))) return r;
+    const uint32_t hint = m->dense_hint;
+    if (m->dcap[c.X] < want) {
+      if (m->dcap[c.X]) CK(hipStreamSynchronize(cs));  // (the map stream is done with it)
+      if ((r = grow_set(m, c.X, want))) return r;
+      m->dense_hint = hint;  // a guess is for this set alone
     }
+    // the ring's sets never used yet get the size measured so far, so the next
+    // scans of the ring do not each stop for an allocation
+    for (int y = 0; hint && want == hint && !c.alone && y < m->rec_sets; ++y)
+      if (m->dcap[y] == 0 && (r = grow_set(m, y, hint))) return r;
   }
   c.cap = m->dcap[c.X];  // (a later first use may size an empty set X before this is checked)
   uint32_t cells = 0;
@@ -1651,6 +1654,7 @@ int run_brick_accumulate(vdbgpu_map* m, Source& src, const float* xyz, int64_t n
   int r;
   if ((r = commit_staged(m)) || (r = brick_tables(m, n, src.max_range))) return r;
   BrickCast c = brick_cast(src, xyz, n, stride, origin, on_device);
+  c.alone = true;
   if ((r = brick_enqueue(m, c, 0)) || (r = brick_check(m, c))) return r;
   if (!m->staged) return VDBGPU_OK;  // nothing marked
   m->staged = false;

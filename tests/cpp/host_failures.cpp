@@ -38,6 +38,7 @@ std::map<const void*, size_t> g_blocks;  // live allocations
 long g_fail_in = 0;                      // the n-th allocation from here fails (0: none)
 bool g_failed = false;
 size_t g_pinned = 0;  // bytes ever allocated as pinned memory
+size_t g_read = 0;    // bytes ever copied from the device
 
 // The plain name of a kernel's symbol, _ZN6vdbgpu<length>k_name...
 std::string plain(const char* mangled) {
@@ -113,14 +114,12 @@ int hipHostGetDevicePointer(void** d, void* h, unsigned) {
   *d = h;
   return 0;
 }
-int hipMemcpy(void* d, const void* s, size_t n, int) {
+int hipMemcpy(void* d, const void* s, size_t n, int kind) {
+  if (kind == 2) g_read += n;  // hipMemcpyDeviceToHost
   std::memcpy(d, s, n);
   return 0;
 }
-int hipMemcpyAsync(void* d, const void* s, size_t n, int, void*) {
-  std::memcpy(d, s, n);
-  return 0;
-}
+int hipMemcpyAsync(void* d, const void* s, size_t n, int kind, void*) { return hipMemcpy(d, s, n, kind); }
 int hipMemsetAsync(void* d, int v, size_t n, void*) {
   std::memset(d, v, n);
   return 0;
@@ -296,10 +295,31 @@ void section() {
   }
 }
 
+// An update set's export reads its entries, whatever room the set has.
+void update_export() {
+  constexpr int kLeaves = 100;
+  g_kernels["k_compact"] = [](void** a) { *arg<unsigned int*>(a, 3) = kLeaves; };
+  vdbgpu_map* m = new_map(false);
+  vdbgpu_tuning t{256, 32, 16, 0.5, 1, 8};
+  CHECK(vdbgpu_set_tuning(m, &t) == VDBGPU_OK);
+  const std::vector<float> p(3 * 2000, 0.5f);
+  const double origin[3] = {0, 0, 0};
+  CHECK(vdbgpu_accumulate(m, "s", p.data(), 2000, 12, origin, 0) == VDBGPU_OK);
+  std::vector<int32_t> o(3 * kLeaves);
+  std::vector<uint64_t> v(8 * kLeaves), h(8 * kLeaves);
+  const size_t before = g_read;
+  CHECK(vdbgpu_export_update(m, "s", o.data(), v.data(), h.data(), kLeaves) == kLeaves);
+  CHECK(g_read - before <= kLeaves * 136 + 4096);
+  g_fail_in = 1;
+  CHECK(vdbgpu_export_update(m, "s", o.data(), v.data(), h.data(), kLeaves) == -1);
+  CHECK(vdbgpu_export_update(m, "s", o.data(), v.data(), h.data(), kLeaves - 1) == -kLeaves);
+  close_map(m);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
-  const std::map<std::string, void (*)()> scenarios = {{"snapshot", snapshot}, {"section", section}};
+  const std::map<std::string, void (*)()> scenarios = {{"snapshot", snapshot}, {"section", section}, {"update_export", update_export}};
   const auto s = argc > 1 ? scenarios.find(argv[1]) : scenarios.end();
   if (s == scenarios.end()) return 3;
   s->second();

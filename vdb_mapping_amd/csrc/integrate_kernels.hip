@@ -1055,6 +1055,33 @@ __global__ __launch_bounds__(256) void k_clear_listed(UpdView u, const uint32_t*
   }
 }
 
+// Every entry of an update set emptied: only the keys of a free slot are read
+// (its masks are zero), so it costs the slots 8 bytes each, not 136.
+__global__ __launch_bounds__(256) void k_clear_set(UpdView u, uint32_t cap) {
+  ulonglong2* m = reinterpret_cast<ulonglong2*>(u.masks);
+  const uint32_t G = gridDim.x * blockDim.x;
+  for (uint32_t slot = blockIdx.x * blockDim.x + threadIdx.x; slot < cap; slot += G) {
+    if (u.keys[slot] == kEmpty) continue;
+#pragma unroll
+    for (int l = 0; l < 8; ++l) m[(size_t)slot * 8 + l] = ulonglong2{0, 0};
+    u.keys[slot] = kEmpty;
+  }
+}
+
+// The listed slots of an update set side by side: keys, and masks 16 bytes per lane.
+__global__ __launch_bounds__(256) void k_copy_listed(UpdView u, const uint32_t* __restrict__ list, uint32_t count,
+                                                     unsigned long long* __restrict__ keys,
+                                                     unsigned long long* __restrict__ masks) {
+  const uint64_t G = (uint64_t)gridDim.x * blockDim.x;
+  const ulonglong2* __restrict__ src = reinterpret_cast<const ulonglong2*>(u.masks);
+  ulonglong2* dst = reinterpret_cast<ulonglong2*>(masks);
+  for (uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; t < (uint64_t)count * 8; t += G) {
+    const uint32_t slot = list[t >> 3];
+    dst[t] = src[(size_t)slot * 8 + (t & 7)];
+    if ((t & 7) == 0) keys[t >> 3] = u.keys[slot];
+  }
+}
+
 __global__ void k_set_u32(unsigned int* p, uint32_t v) {
   if (threadIdx.x == 0) *p = v;
 }
@@ -1277,6 +1304,20 @@ hipError_t launch_clear_listed(hipStream_t s, UpdView u, const uint32_t* list, u
   if (!count) return hipSuccess;
   const int grid = (int)std::min<uint64_t>(8192, ((uint64_t)count * 8 + 255) / 256);
   hipLaunchKernelGGL(k_clear_listed, dim3(grid), dim3(256), 0, s, u, list, count);
+  return hipGetLastError();
+}
+
+hipError_t launch_clear_set(hipStream_t s, UpdView u, uint32_t cap) {
+  if (!cap) return hipSuccess;
+  hipLaunchKernelGGL(k_clear_set, dim3(std::min(4096u, (cap + 255) / 256)), dim3(256), 0, s, u, cap);
+  return hipGetLastError();
+}
+
+hipError_t launch_copy_listed(hipStream_t s, UpdView u, const uint32_t* list, uint32_t count, unsigned long long* keys,
+                              unsigned long long* masks) {
+  if (!count) return hipSuccess;
+  const int grid = (int)std::min<uint64_t>(8192, ((uint64_t)count * 8 + 255) / 256);
+  hipLaunchKernelGGL(k_copy_listed, dim3(grid), dim3(256), 0, s, u, list, count, keys, masks);
   return hipGetLastError();
 }
 

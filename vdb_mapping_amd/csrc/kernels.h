@@ -50,6 +50,9 @@ hipError_t launch_map_insert(hipStream_t s, UpdView u, const uint32_t* list, con
 hipError_t launch_merge_records(hipStream_t s, UpdView rec, const RecIndex& ri, uint32_t count, UpdView u,
                                 uint32_t* list, unsigned int* listed);
 hipError_t launch_clear_listed(hipStream_t s, UpdView u, const uint32_t* list, uint32_t count);
+hipError_t launch_clear_set(hipStream_t s, UpdView u, uint32_t cap);
+hipError_t launch_copy_listed(hipStream_t s, UpdView u, const uint32_t* list, uint32_t count, unsigned long long* keys,
+                              unsigned long long* masks);
 hipError_t launch_set_u32(hipStream_t s, unsigned int* p, uint32_t v);
 hipError_t launch_rec_total(hipStream_t s, const uint32_t* bsum, const BatchCtl* ctl, const RecDest* dest,
                             const unsigned int* rcnt, Status* st);

@@ -2721,10 +2721,7 @@ int32_t vdbgpu_reset(vdbgpu_map* m) {
   if ((r = clear_grid(m))) return r;
   for (auto& kv : m->sources) {
     Source& s = kv.second;
-    if (s.cap) {
-      CK(launch_fill_u64(m->stream, s.keys, s.cap, kEmpty));
-      CK(hipMemsetAsync(s.masks, 0, (size_t)s.cap * 16 * sizeof(unsigned long long), m->stream));
-    }
+    if (s.cap) CK(launch_clear_set(m->stream, upd_view(s), s.cap));
     s.pending = 0;
     s.counting = false;
   }
@@ -2868,20 +2865,25 @@ int64_t vdbgpu_export_update(vdbgpu_map* m, const char* id, int32_t* origins, ui
   if (!origins && !visited && !hit) return s.pending;
   if ((int64_t)s.pending > cap) return -(int64_t)s.pending;
   if (s.cap == 0 || s.pending == 0) return 0;
-  if (hipStreamSynchronize(m->stream)) return -1;
-  std::vector<unsigned long long> keys(s.cap), masks((size_t)s.cap * 16);
-  if (hipMemcpy(keys.data(), s.keys, (size_t)s.cap * 8, hipMemcpyDeviceToHost) ||
-      hipMemcpy(masks.data(), s.masks, (size_t)s.cap * 128, hipMemcpyDeviceToHost))
-    return -1;
-  std::vector<std::pair<std::array<int, 3>, uint32_t>> order;
-  for (uint32_t i = 0; i < s.cap; ++i) {
-    if (keys[i] == kEmpty) continue;
-    std::array<int, 3> o;
-    key_origin(keys[i], o.data());
-    order.push_back({o, i});
+  // the listed entries alone: the set has room for two to four times as many
+  const uint32_t n = s.pending;
+  std::vector<unsigned long long> keys(n), masks((size_t)n * 16);
+  unsigned long long* d = nullptr;
+  CKN(dalloc(m, &d, (size_t)n * 17));
+  const hipError_t e = [&]() -> hipError_t {
+    hipError_t e = launch_copy_listed(m->stream, upd_view(s), s.list, n, d + (size_t)n * 16, d);
+    if (!e) e = hipMemcpyAsync(keys.data(), d + (size_t)n * 16, (size_t)n * 8, hipMemcpyDeviceToHost, m->stream);
+    if (!e) e = hipMemcpyAsync(masks.data(), d, (size_t)n * 128, hipMemcpyDeviceToHost, m->stream);
+    return e ? e : hipStreamSynchronize(m->stream);
+  }();
+  dfree(m, &d, (size_t)n * 17);
+  CKN(e);
+  std::vector<std::pair<std::array<int, 3>, uint32_t>> order(n);
+  for (uint32_t i = 0; i < n; ++i) {
+    key_origin(keys[i], order[i].first.data());
+    order[i].second = i;
   }
   std::sort(order.begin(), order.end());
-  if ((int64_t)order.size() > cap) return -(int64_t)order.size();
   for (size_t j = 0; j < order.size(); ++j) {
     const uint32_t i = order[j].second;
     if (origins) std::memcpy(origins + 3 * j, order[j].first.data(), 12);

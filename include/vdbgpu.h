@@ -81,7 +81,7 @@ typedef struct vdbgpu_tuning {
   int32_t steps_per_lane; /* DDA visits per lane work item (chunk length) */
   int32_t waves_per_cu;   /* resident waves per CU requested for the traversal grid */
   double load_factor;     /* update-set hash target load (0.3..0.9) */
-  int32_t traversal;      /* inserts and accumulates: 0 = brick walk (default; accumulates of sparse clouds, or
+  int32_t traversal;      /* inserts and accumulates: 0 = brick walk (default; accumulates of small or sparse clouds, or
                            * with another block, steps_per_lane or waves_per_cu than the defaults, use the
                            * hash traversal that those shape), 1 = update-set hash traversal */
   int32_t defer;          /* brick-walk inserts: the map update of up to this many consecutive scans (1..8,

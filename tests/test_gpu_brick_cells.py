@@ -1,5 +1,6 @@
 """The brick tables of a scan (cells of the cube around the sensor up to a range of 1,597 voxels, hashed keys beyond)
-and the size of its work items (256 segments up to 65,536 rays, 1,024 beyond) against the oracle, bit for bit."""
+and the size of its work items (256 segments up to 65,536 rays, 1,024 beyond) against the oracle, bit for bit. The
+accumulated clouds beside them take the brick path at 200 voxels only (test_gpu_accumulate.py has the larger ones)."""
 import numpy as np
 import pytest
 

@@ -37,11 +37,6 @@ constexpr uint32_t kMinUpdateCap = 1u << 12;
 constexpr uint32_t kMaxRays = 1u << 30;
 constexpr uint32_t kMaxPointLeaves = 1u << 19;  // leaves with active voxels that are ordered on the device
 constexpr int64_t kBrickAccumulateRays = 1 << 22;
-// Rays per squared voxel of range from which an accumulated cloud takes the
-// brick path. Three clouds and their integrate, brick against hash traversal:
-// range 1,000 voxels, 2,000 rays 2.2 : 1.2 ms, 12,000 2.9 : 2.7, 65,536 3.5 : 5.2;
-// range 300 voxels, 2,000 rays 0.53 : 0.62.
-constexpr double kBrickAccumulateDensity = 0.012;
 constexpr vdbgpu_tuning kTuning{256, 32, 16, 0.5, 0, kDeferMax};  // as a map is created
 constexpr int kTraverseMaxBlock = 256;  // __launch_bounds__ of k_traverse
 
@@ -1131,6 +1126,30 @@ int run_fast(vdbgpu_map* m, Source& src, const float* xyz, int64_t n, int64_t st
   return VDBGPU_OK;
 }
 
+// Does an accumulated cloud of n rays of `vox` voxels of range take the brick path? Bricks pay
+// when several rays share one, and the rays through a brick at the range thin out with its
+// square: from (vox / 1,000)^2 on as many clouds of 16,000 rays. Up to 1,000 voxels 16,000 rays
+// are enough; below 300 the traversal's chains are short, and what the brick path
+// launches more costs more than the rays do. A few rays of 175 to 400 voxels are the exception:
+// the traversal waits for the chains of too few workgroups. Time of three
+// clouds and their integrate, hash traversal over brick path (outdoor scans, room
+// scans beside them; above 1 the brick path is faster):
+//   voxels   1,000 rays   4,000        12,000       16,000       24,000       65,536
+//      150          0.93         0.88         0.87         0.85         0.90         0.88
+//      200   1.27   1.04  0.94   0.91  0.95   0.88  1.00   0.93  1.04   0.94  1.24   1.18
+//      300   1.32   1.15  1.11   1.04  1.05   0.93  1.07   0.95  1.19   1.05  1.33   1.24
+//      400   1.12   1.17  1.01   1.07  1.03   0.96  1.05   1.06  1.15   1.15  1.43   1.58
+//      500   1.04   1.12  0.95   1.00  0.93   1.00  1.00   1.07  1.25   1.46  1.44   1.72
+//      750   0.98   1.05  0.81   0.88  0.92   1.01  1.19   1.33  1.25   1.49  1.40   1.70
+//    1,000   0.77         0.72         0.85         1.01         1.16         1.37
+//    1,500   0.63         0.56         0.67         0.71         0.82 (32,000 0.94, 48,000 1.11)
+//    2,000   0.52         0.48         0.52         0.62         0.69 (48,000 0.94, 65,536 1.04)
+bool brick_pays(int64_t n, double vox) {
+  const double far = vox / 1000.0, near = 300.0 / vox;
+  return (double)n >= 16000.0 * std::max(1.0, std::max(far * far, near * near)) ||
+         (vox >= 175.0 && vox <= 400.0 && (double)n <= 14.0 * vox);
+}
+
 int do_accumulate(vdbgpu_map* m, Source& src, const float* xyz, int64_t n, int64_t stride,
                   const double origin[3], bool on_device) {
   if (!m->config_set) return fail(m, VDBGPU_NOT_CONFIGURED, "Map not properly configured. Did you call setConfig method?");
@@ -1141,14 +1160,12 @@ int do_accumulate(vdbgpu_map* m, Source& src, const float* xyz, int64_t n, int64
   // The brick path lists a cloud's update leaves and merges them into the
   // source's set. The hash traversal stays where the caller asked for it or for
   // its launch shape, for clouds whose segments (16 bytes each, some 30 per ray)
-  // would take gigabytes, and for sparse ones: bricks pay when several rays
-  // share one, and the rays through a brick at the range thin out with its
-  // square (kBrickAccumulateDensity).
+  // would take gigabytes, and where it is the faster one (brick_pays).
   const vdbgpu_tuning& tn = m->tuning;
   const bool shaped = tn.block != kTuning.block || tn.steps_per_lane != kTuning.steps_per_lane ||
                       tn.waves_per_cu != kTuning.waves_per_cu;
   if (tn.traversal == 0 && !shaped && n <= kBrickAccumulateRays && src.max_range > 0 &&
-      (double)n >= kBrickAccumulateDensity * (src.max_range * m->inv) * (src.max_range * m->inv))
+      brick_pays(n, src.max_range * m->inv))
     return run_brick_accumulate(m, src, xyz, n, stride, origin, on_device);
   ScanInfo sc{};
   sc.o[0] = origin[0];

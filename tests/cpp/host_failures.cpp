@@ -316,10 +316,47 @@ void update_export() {
   close_map(m);
 }
 
+// The point export: tables for the leaves there are, and the host's own way when the
+// device has no room for tables or points.
+void points() {
+  struct StatusHead {  // Status
+    unsigned long long total, voxels, rays;
+    unsigned int error, overflow, entries, leaf_count;
+  };
+  g_kernels["k_compact"] = [](void** a) { *arg<unsigned int*>(a, 3) = 1; };
+  g_kernels["k_map_insert"] = [](void** a) { arg<StatusHead*>(a, 10)->leaf_count = 1; };
+  g_kernels["k_point_leaves"] = [](void** a) {
+    arg<StatusHead*>(a, 6)->entries = 1;
+    arg<StatusHead*>(a, 6)->total = 1;
+  };
+  std::vector<float> xyz(3);
+  bool through = false;
+  for (long k = 1; !through; ++k) {
+    vdbgpu_map* m = new_map(false);
+    // many edits of one leaf: the host's bound of the leaf count is far above it
+    for (int i = 0; i < 50; ++i) CHECK(edit(m) == VDBGPU_OK);
+    vdbgpu_stats before{}, after{};
+    CHECK(vdbgpu_get_stats(m, &before) == VDBGPU_OK);
+    for (int i = 0; i < 50; ++i) CHECK(edit(m) == VDBGPU_OK);
+    g_fail_in = k;
+    g_failed = false;
+    const int64_t n = vdbgpu_export_active_points(m, xyz.data(), 1);
+    through = !g_failed;
+    g_fail_in = 0;
+    // (kernels write nothing here, so the host finds the leaf without an active voxel)
+    CHECK(n == (g_failed ? 0 : 1));
+    CHECK(vdbgpu_export_active_points(m, xyz.data(), 1) == 1);
+    CHECK(vdbgpu_get_stats(m, &after) == VDBGPU_OK);
+    CHECK(after.scratch_bytes - before.scratch_bytes <= 24 + 12);
+    close_map(m);
+    CHECK(k > 1 || !through);
+  }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
-  const std::map<std::string, void (*)()> scenarios = {{"snapshot", snapshot}, {"section", section}, {"update_export", update_export}};
+  const std::map<std::string, void (*)()> scenarios = {{"snapshot", snapshot}, {"section", section}, {"update_export", update_export}, {"points", points}};
   const auto s = argc > 1 ? scenarios.find(argv[1]) : scenarios.end();
   if (s == scenarios.end()) return 3;
   s->second();

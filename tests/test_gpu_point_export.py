@@ -65,3 +65,16 @@ def test_capacity(short):
     got = V.lib().vdbgpu_export_active_points(g.h, out.ctypes.data_as(ctypes.c_void_p), len(want) - short)
     assert got == (-len(want) if short else len(want))
     assert np.all(out[-1] == -7.0) and (short or np.array_equal(out[:-1], want))
+
+
+def test_more_leaves_than_are_ordered_on_the_device():
+    """Above 2^19 leaves the host sorts: the same points in the same order."""
+    n = (1 << 19) + 300
+    g, o = pair(1.0, 10.0, **PROBS)
+    i = np.random.default_rng(1).permutation(n)
+    p = (np.stack([i % 83 - 40, i // 83 % 81 - 40, i // (83 * 81) - 35], 1) * 8 + 3.5).astype(np.float32)
+    both(g, o, "add_points_to_grid", p)
+    assert g.leaf_count() == n
+    assert same_points(g, o) == n
+    both(g, o, "remove_points_from_grid", p[:400])  # back below the line
+    assert same_points(g, o) == n - 400

@@ -20,7 +20,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("scenario", ["snapshot", "section", "update_export"])
+@pytest.mark.parametrize("scenario", ["snapshot", "section", "update_export", "points"])
 def test_refused_memory(program, scenario):
     r = subprocess.run([program, scenario], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0 and "%s ok" % scenario in r.stdout, r.stdout + r.stderr

@@ -35,7 +35,10 @@ namespace {
 constexpr uint32_t kMaxTableN = 8192;       // longest per-axis ray extent in voxels
 constexpr uint32_t kMinUpdateCap = 1u << 12;
 constexpr uint32_t kMaxRays = 1u << 30;
-constexpr uint32_t kMaxPointLeaves = 1u << 19;  // leaves with active voxels that are ordered on the device
+// Leaves with active voxels that are ordered on the device, by n^2 compares (16,384 leaves 0.5 ms
+// and 4.8 on the host, 131,072 4.1 and 37, 524,288 39 and 173: from about four times as many on
+// the host's sort would be the faster one).
+constexpr uint32_t kMaxPointLeaves = 1u << 19;
 constexpr int64_t kBrickAccumulateRays = 1 << 22;
 constexpr vdbgpu_tuning kTuning{256, 32, 16, 0.5, 0, kDeferMax};  // as a map is created
 constexpr int kTraverseMaxBlock = 256;  // __launch_bounds__ of k_traverse
@@ -3221,6 +3224,27 @@ int clear_grid(vdbgpu_map* m) {
   return VDBGPU_OK;
 }
 
+// Tables of the point export for n leaves; false (and none) when the device has
+// no room for them.
+bool grow_points(vdbgpu_map* m, uint64_t n) {
+  dfree(m, &m->pt_key, m->pt_cap);
+  dfree(m, &m->pt_cnt, m->pt_cap);
+  dfree(m, &m->pt_idx, m->pt_cap);
+  dfree(m, &m->pt_off, m->pt_cap);
+  m->pt_cap = 0;
+  if (dalloc(m, &m->pt_key, n) == hipSuccess && dalloc(m, &m->pt_cnt, n) == hipSuccess &&
+      dalloc(m, &m->pt_idx, n) == hipSuccess && dalloc(m, &m->pt_off, n) == hipSuccess) {
+    m->pt_cap = n;
+    return true;
+  }
+  (void)refused();
+  dfree(m, &m->pt_key, n);
+  dfree(m, &m->pt_cnt, n);
+  dfree(m, &m->pt_idx, n);
+  dfree(m, &m->pt_off, n);
+  return false;
+}
+
 }  // namespace
 
 extern "C" {
@@ -3336,42 +3360,36 @@ int64_t vdbgpu_export_active_points(vdbgpu_map* m, float* xyz, int64_t cap) {
   if (!m) return -1;
   Guard g(m);
   if (g.rc) return -1;
+  if (m->leaf_count_ub > m->pt_cap && read_status(m)) return -1;  // the exact count, before tables are sized by it
   const uint64_t bound = m->leaf_count_ub;
   if (bound == 0) return 0;
-  if (bound > m->pt_cap) {
-    dfree(m, &m->pt_key, m->pt_cap);
-    dfree(m, &m->pt_cnt, m->pt_cap);
-    dfree(m, &m->pt_idx, m->pt_cap);
-    dfree(m, &m->pt_off, m->pt_cap);
-    m->pt_cap = 0;
-    CKN(dalloc(m, &m->pt_key, bound));
-    CKN(dalloc(m, &m->pt_cnt, bound));
-    CKN(dalloc(m, &m->pt_idx, bound));
-    CKN(dalloc(m, &m->pt_off, bound));
-    m->pt_cap = bound;
+  const bool tables = bound <= m->pt_cap || grow_points(m, bound);
+  uint32_t listed = 0;
+  int64_t points = 0;
+  if (tables) {
+    CKN(launch_zero_words(m->stream, (unsigned long long*)&m->d_st[2], sizeof(Status) / 8));
+    CKN(launch_point_leaves(m->stream, map_view(m), bound, &m->d_st[1], tile_view(m), m->pt_key, m->pt_cnt, m->pt_idx,
+                            &m->d_st[2]));
+    if (read_status(m)) return -1;
+    listed = m->h_st[2].entries;
+    points = (int64_t)m->h_st[2].total;
+    if (!xyz) return points;
+    if (points > cap) return -points;
+    if (points == 0) return 0;
   }
-  CKN(launch_zero_words(m->stream, (unsigned long long*)&m->d_st[2], sizeof(Status) / 8));
-  CKN(launch_point_leaves(m->stream, map_view(m), bound, &m->d_st[1], tile_view(m), m->pt_key, m->pt_cnt, m->pt_idx,
-                          &m->d_st[2]));
-  if (read_status(m)) return -1;
-  const uint32_t listed = m->h_st[2].entries;
-  const int64_t points = (int64_t)m->h_st[2].total;
-  if (!xyz) return points;
-  if (points > cap) return -points;
-  if (points == 0) return 0;
-  if (listed <= kMaxPointLeaves) {
-    if ((uint64_t)points * 3 > m->pt_xyz_cap) {
-      dfree(m, &m->pt_xyz, m->pt_xyz_cap);
-      m->pt_xyz_cap = 0;
-      CKN(dalloc(m, &m->pt_xyz, (uint64_t)points * 3));
-      m->pt_xyz_cap = (uint64_t)points * 3;
-    }
+  if (tables && listed <= kMaxPointLeaves && (uint64_t)points * 3 > m->pt_xyz_cap) {
+    dfree(m, &m->pt_xyz, m->pt_xyz_cap);
+    m->pt_xyz_cap = dalloc(m, &m->pt_xyz, (uint64_t)points * 3) == hipSuccess ? (uint64_t)points * 3 : 0;
+    if (!m->pt_xyz_cap) (void)refused();
+  }
+  if (tables && listed <= kMaxPointLeaves && (uint64_t)points * 3 <= m->pt_xyz_cap) {
     CKN(launch_points(m->stream, map_view(m), tile_view(m), m->pt_key, m->pt_cnt, m->pt_idx, listed, m->pt_off,
                       m->res, m->pt_xyz));
     CKN(hipMemcpyAsync(xyz, m->pt_xyz, (size_t)points * 12, hipMemcpyDeviceToHost, m->stream));
     CKN(hipStreamSynchronize(m->stream));
     return points;
   }
+  // on the host: more leaves than are ordered on the device, or no memory for it there
   const uint32_t n = m->h_st[1].leaf_count;
   std::vector<unsigned long long> keys(n), act((size_t)n * 8);
   if (n && (hipMemcpy(keys.data(), m->leaf_keys, n * sizeof(unsigned long long), hipMemcpyDeviceToHost) ||

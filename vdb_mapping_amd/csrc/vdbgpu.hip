@@ -2214,6 +2214,7 @@ uint64_t walk_scratch(vdbgpu_map* m, bool release) {
     m->sec_pinned = kSectionChunk;
     m->sec_cells = m->sec_cap = 0;
     m->f_groups = m->f_rays = 0;
+    m->f_cap = kFastSpans;
     m->pt_cap = m->pt_xyz_cap = 0;
     m->points_bytes = 0;
     m->ray_cap = 0;

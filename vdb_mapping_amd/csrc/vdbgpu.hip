@@ -1510,10 +1510,12 @@ int brick_enqueue(vdbgpu_map* m, BrickCast& c, int attempt) {
     uint32_t want = m->dense_hint;
     const int64_t most = std::max(c.n, m->batch_rays);
     if (want == 0) {
-      // the map's first scan: its records are guessed, on the large side (a set too
-      // small costs another cast: 65,536 outdoor rays of 500 voxels 1.4 ms for the
-      // first scan with a quarter of this, 0.9 ms), at most 2^21 of them (290 MB)
-      const double g = 4.0 * std::sqrt((double)c.n) * std::min(c.sc.R * m->inv, (double)kMaxTableN);
+      // the map's first scan: its records are guessed, on the large side, since a set
+      // too small costs another cast (65,536 outdoor rays of 500 voxels 1.4 ms, not
+      // 0.7). Room and outdoor scans of 500 to 262,144 rays have up to 2.43 times
+      // sqrt(rays) * range records up to 500 voxels; farther ones overflow the
+      // segments of a first scan anyway and are sized by that cast's work items.
+      const double g = 2.5 * std::sqrt((double)c.n) * std::min(c.sc.R * m->inv, (double)kMaxTableN);
       want = (uint32_t)std::max(4096.0, std::min(g, 2097152.0));
     } else if (m->guess_recs && most > m->guess_rays) {
       // more rays than any scan so far (or a batch's largest): update leaves

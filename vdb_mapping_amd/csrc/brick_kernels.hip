@@ -11,8 +11,8 @@
 // positions per work item, listed and copied densely afterwards, needed no
 // counters but four launches and a copy: 105 us of an outdoor scan's cast.)
 // No global atomics touch voxel bits except for the few
-// bricks so crowded (more than kItemSegs segments, around the sensor) that
-// several workgroups share them.
+// bricks so crowded (more segments than a work item takes, around the sensor)
+// that several workgroups share them.
 //
 //   k_seg_count     one lane per ray: enumerate its bricks, count segments
 //                   per brick (aggregated per workgroup in an LDS table,
@@ -283,7 +283,7 @@ __global__ __launch_bounds__(256) void k_scan_u64(const uint64_t* __restrict__ b
 // (four to a lane). A workgroup takes its run of segments and of items with one
 // atomic on the pair of totals; which run a brick gets does not matter, so no
 // scan over the workgroups is needed (it took two more launches, 9 us of a
-// 2,000-point scan's 160 us of GPU time). A range of 1,000 voxels has 268
+// 2,000-point scan's 160 us of GPU time). A range of 1,000 voxels has 269
 // workgroups, and only those with a segment touch the counter.
 __global__ __launch_bounds__(256) void k_brick_offsets(BrickView bv, BrickItem* __restrict__ items,
                                                        uint32_t seg_cap, uint32_t item_cap,

@@ -56,8 +56,10 @@ constexpr uint32_t kOvfSpans = 64u;   // fast-mode span lists
 // too few bricks to fill the chip, and its crowded ones (all rays start in one)
 // are the walk's critical path, so they are cut finer (the walk of a room scan of
 // 32,768 rays 69 -> 36 us, of 65,536 outdoor rays 255 -> 238 us). Larger scans
-// keep 1,024: the outdoor stream of 262,144-ray scans ran 5% slower at 256, with
-// more split bricks to merge.
+// keep 1,024: with 256 there are more split bricks to merge (a lone outdoor scan of
+// 131,072 rays over 500 voxels 443 -> 475 us, of 262,144 542 -> 625; a room scan of
+// 100,000 rays over 150 voxels 200 -> 209, of 262,144 300 -> 339; at 80,000 rays
+// both are within 2%).
 constexpr uint32_t kItemSegs = 1024;
 constexpr uint32_t kSmallItemSegs = 256;
 constexpr uint32_t kSmallScanRays = 65536;
@@ -71,7 +73,12 @@ constexpr int kEditActivate = 3;  // setActiveState(on)
 // A scan's update-leaf records lie in up to kRecRegions equal regions of its
 // record set, each filled from its start (see emit_leaves).
 constexpr uint32_t kRecRegions = 16;
-constexpr uint32_t kRecRegionItems = 4096;  // work items from which all regions are used
+// Work items from which all regions are used: where many workgroups append at once one
+// counter holds them up (a lone outdoor scan of 4,000 rays over 1,000 voxels 545 us with
+// 16 regions, 670 with one; of 16,384 rays 870 and 1,010; of 262,144 rays 1,700 and 1,745).
+// Scans of fewer items differ by 7% at most either way, and equal regions fill unevenly, so
+// that their set has to be larger.
+constexpr uint32_t kRecRegionItems = 4096;
 constexpr uint32_t kRecCountStride = 32;    // words between the regions' counters (a line each)
 
 struct Status {
@@ -152,7 +159,7 @@ struct GroupView {
 
 // Bricks (32^3 voxels) of one scan: slot -> segment count and fill cursor. A
 // slot is a cell of the cube of 2 half + 1 bricks around the sensor's brick
-// where that has at most kDenseBricks cells (ranges up to 1,600 voxels), x-major:
+// where that has at most kDenseBricks cells (ranges up to 1,597 voxels), x-major:
 // no key to compare or insert, a count is one atomic without a result, and the
 // bricks are listed in space order. Farther rays hash the brick's key.
 constexpr uint32_t kDenseBricks = 1u << 20;

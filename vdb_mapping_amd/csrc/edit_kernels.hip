@@ -404,7 +404,8 @@ __global__ __launch_bounds__(256) void k_section_rows(MapView mp, SectionBox sb,
     char* heads = base + (size_t)leaves * 2048;
     if ((lane & 7) == 0) reinterpret_cast<unsigned long long*>(heads)[(size_t)i * 8 + (lane >> 3)] = m;
     if (lane < 3)
-      reinterpret_cast<int*>(heads + (size_t)leaves * 64)[(size_t)i * 3 + lane] = lane == 0 ? o[0] : (lane == 1 ? o[1] : o[2]);
+      reinterpret_cast<int*>(heads + (size_t)leaves * 64)[(size_t)i * 3 + lane] =
+          lane == 0 ? o[0] : (lane == 1 ? o[1] : o[2]);
   }
 }
 

@@ -1279,8 +1279,8 @@ hipError_t launch_group_add(hipStream_t s, const uint32_t* eidx, const uint32_t*
                             unsigned int* ngroups) {
   if (!count) return hipSuccess;
   const int block = list_block(count);
-  hipLaunchKernelGGL(k_group_add, dim3((count + block - 1) / block), dim3(block), 0, s, eidx, list, ri, count, t, gslot, rgrp,
-                     rgrp_stride, glist, grec, ngroups);
+  hipLaunchKernelGGL(k_group_add, dim3((count + block - 1) / block), dim3(block), 0, s, eidx, list, ri, count, t, gslot,
+                     rgrp, rgrp_stride, glist, grec, ngroups);
   return hipGetLastError();
 }
 

@@ -4,8 +4,8 @@
 // One vdbgpu_map owns: a HIP stream (default priority), a mutex, the device
 // leaf store + leaf hash, one update set per input source, per-scan scratch,
 // the DDA crossing table and a pinned status block. The per-scan path is
-//   accumulate: [H2D points] -> the brick cast -> k_merge_records, or, for sparse
-//               clouds, k_prep -> k_scan_blocks -> k_traverse -> k_compact;
+//   accumulate: [H2D points] -> the brick cast -> k_merge_records, or, where
+//               that is the slower one (brick_pays), k_prep -> k_scan_blocks -> k_traverse -> k_compact;
 //               one status read (the only host sync of a scan)
 //   integrate : k_map_insert -> k_apply, in source-id order (several sources: one
 //               group pass), no sync
@@ -199,7 +199,7 @@ struct vdbgpu_map {
   uint32_t* reidx[kRecSets] = {};             // record set: map leaf index of each record
   RecIndex rindex[kRecSets] = {};             // record set: where its scan's records lie
   uint32_t dcap[kRecSets] = {};
-  uint32_t dense_hint = 0;     // record-set size for a first use (largest scan seen, +25%)
+  uint32_t dense_hint = 0;     // record-set size for a first use (largest set, largest scan +25%)
   int64_t guess_rays = 0;      // rays and records of the scan with the most rays so far
   uint32_t guess_recs = 0;
   int64_t batch_rays = 0;      // most rays of a scan of the batch being inserted
@@ -927,8 +927,8 @@ int stage_scans(vdbgpu_map* m, hipStream_t stream, const float* xyz, int64_t str
     CK(launch_stage_scan(stream, scans[0], ctl, m->d_scans, m->d_ctl, &m->d_st[0],
                          clear_bricks && !dense_cells ? m->bkeys : nullptr,
                          clear_bricks ? reinterpret_cast<unsigned long long*>(m->bcnt) : nullptr,
-                         clear_bricks ? (dense_cells ? dense_cells / 2 : m->bcap) : 0, dest ? *dest : RecDest{}, dest ? m->d_dest : nullptr,
-                         m->d_rcnt));
+                         clear_bricks ? (dense_cells ? dense_cells / 2 : m->bcap) : 0, dest ? *dest : RecDest{},
+                         dest ? m->d_dest : nullptr, m->d_rcnt));
   } else {
     std::copy(scans.begin(), scans.end(), m->h_scans);
     *m->h_ctl = ctl;
@@ -948,8 +948,9 @@ int stage_scans(vdbgpu_map* m, hipStream_t stream, const float* xyz, int64_t str
 // Status code of the kernel error bits of a scan (0 = none).
 int scan_error(vdbgpu_map* m, const Status& st, bool batched) {
   if (st.error & kErrRange)
-    return fail(m, VDBGPU_OUT_OF_RANGE, batched ? "a voxel index is outside [-2^21, 2^21) (batch) or not finite; batch rejected"
-                                                : "a voxel index is outside [-2^23, 2^23) or not finite; scan rejected");
+    return fail(m, VDBGPU_OUT_OF_RANGE,
+                batched ? "a voxel index is outside [-2^21, 2^21) (batch) or not finite; batch rejected"
+                        : "a voxel index is outside [-2^23, 2^23) or not finite; scan rejected");
   if (st.error & kErrTable) return fail(m, VDBGPU_UNSUPPORTED, "a ray spans more than 8192 voxels along one axis");
   if (st.error & kErrEntry) return fail(m, VDBGPU_DEVICE_ERROR, "mid-ray DDA entry did not converge");
   if (st.error & kErrBrick) return fail(m, VDBGPU_DEVICE_ERROR, "brick walk inconsistency (a segment left its brick)");
@@ -1311,8 +1312,8 @@ int flush_pending(vdbgpu_map* m) {
     Timer t(m, kCompact);
     for (int p = 0; p < P; ++p) {  // in scan order: a scan's records join the groups earlier ones opened
       const int X = m->pend_set[p];
-      CK(launch_group_add(m->stream, m->reidx[X], nullptr, m->rindex[X], m->pend_recs[p], (uint32_t)p, m->gslot, m->rgrp, rs,
-                          m->gl, m->grec, m->ngroups));
+      CK(launch_group_add(m->stream, m->reidx[X], nullptr, m->rindex[X], m->pend_recs[p], (uint32_t)p, m->gslot, m->rgrp,
+                          rs, m->gl, m->grec, m->ngroups));
       gs.masks[p] = m->dmasks[X];
     }
   }
@@ -1450,7 +1451,8 @@ int launch_cast_graph(vdbgpu_map* m, int nb, int spread, uint32_t item_segs, int
   const int grid = (int)next_pow2((uint64_t)nb);
   auto u = [](const void* p) { return (uint64_t)(uintptr_t)p; };
   const std::vector<uint64_t> key = {
-      (uint64_t)grid, (uint64_t)m->num_cu, (uint64_t)spread, item_segs, (uint64_t)half, cells, u(m->rayinfo), u(m->d_scans), u(m->d_ctl), u(m->tbl), u(m->bkeys),
+      (uint64_t)grid, (uint64_t)m->num_cu, (uint64_t)spread, item_segs, (uint64_t)half, cells, u(m->rayinfo), u(m->d_scans),
+      u(m->d_ctl), u(m->tbl), u(m->bkeys),
       u(m->bcnt), m->bcap, u(m->wkey), u(m->wsc), m->wtab_cap, u(m->segs), m->seg_cap, u(m->bsum),
       u(m->items), m->item_cap, u(m->split_slot), m->split_cap, u(m->shared_bits), u(m->d_dest),
       u(m->d_rcnt), u(m->d_st)};
@@ -1584,7 +1586,8 @@ int brick_check(vdbgpu_map* m, BrickCast& c) {
     if ((st.overflow & kOvfBricks) && cells)
       return fail(m, VDBGPU_DEVICE_ERROR, "a ray left the bricks of its range (internal bound violated)");
     if (st.overflow & ~kOvfRecords) {
-      const uint32_t bcap = (st.overflow & kOvfBricks) ? (uint32_t)std::min<uint64_t>(1u << 30, (uint64_t)m->bcap * 4) : m->bcap;
+      const uint32_t bcap =
+          (st.overflow & kOvfBricks) ? (uint32_t)std::min<uint64_t>(1u << 30, (uint64_t)m->bcap * 4) : m->bcap;
       const uint32_t seg_cap = st.segs > m->seg_cap ? grow_cap(st.segs, m->seg_cap) : m->seg_cap;
       const uint32_t split_cap = st.splits > m->split_cap ? grow_cap(st.splits, m->split_cap) : m->split_cap;
       if ((st.overflow & kOvfBricks) && bcap == m->bcap) return fail(m, VDBGPU_DEVICE_ERROR, "brick table cannot grow");
@@ -1690,7 +1693,8 @@ int run_brick_accumulate(vdbgpu_map* m, Source& src, const float* xyz, int64_t n
     if (cap > (1u << 30)) return fail(m, VDBGPU_DEVICE_ERROR, "update set cannot grow");
     if (src.pending == 0) {  // room for another cloud like this one
       free_update(m, src);
-      if ((r = alloc_update(m, src, (uint32_t)std::max<uint64_t>(kMinUpdateCap, std::min<uint64_t>(cap * 2, 1u << 30))))) return r;
+      const uint64_t grown = std::max<uint64_t>(kMinUpdateCap, std::min<uint64_t>(cap * 2, 1u << 30));
+      if ((r = alloc_update(m, src, (uint32_t)grown))) return r;
     } else {
       if ((r = grow_update(m, src, (uint32_t)cap))) return r;
       CK(hipMemsetAsync(&m->d_st[2], 0, sizeof(Status), m->stream));
@@ -1916,8 +1920,8 @@ int integrate_groups(vdbgpu_map* m, const std::vector<Source*>& ready, bool ch, 
         const uint32_t p = (uint32_t)(i - i0);
         CK(launch_map_insert(m->stream, upd_view(s), s.list, RecIndex{}, s.pending, map_view(m), m->eidx + off, ch, cm,
                              m->noop4096, vdbgpu_map::kNoopCap - 1, &m->d_st[1]));
-        CK(launch_group_add(m->stream, m->eidx + off, s.list, RecIndex{}, s.pending, p, m->gslot, m->rgrp, rs, m->gl, m->grec,
-                            m->ngroups));
+        CK(launch_group_add(m->stream, m->eidx + off, s.list, RecIndex{}, s.pending, p, m->gslot, m->rgrp, rs, m->gl,
+                            m->grec, m->ngroups));
         gs.masks[p] = s.masks;
         off += s.pending;
       }
@@ -2545,7 +2549,8 @@ int32_t vdbgpu_accumulate(vdbgpu_map* m, const char* id, const float* xyz, int64
   Guard g(m);
   if (g.rc) return g.rc;
   auto it = m->sources.find(id);
-  if (it == m->sources.end()) return fail(m, VDBGPU_UNKNOWN_SOURCE, std::string("Tried to accumulate update for ") + id + ". Source not available");
+  if (it == m->sources.end())
+    return fail(m, VDBGPU_UNKNOWN_SOURCE, std::string("Tried to accumulate update for ") + id + ". Source not available");
   if (!(it->second.max_range > 0)) return VDBGPU_OK;
   return do_accumulate(m, it->second, xyz, n, stride, origin, on_device != 0);
 }
@@ -2586,7 +2591,8 @@ int32_t vdbgpu_insert_batch(vdbgpu_map* m, const char* id, int32_t nscans, const
     int status = VDBGPU_OK;
     if (nscans > 0) {
       if (it == m->sources.end())
-        status = fail(m, VDBGPU_UNKNOWN_SOURCE, std::string("Tried to accumulate update for ") + id + ". Source not available");
+        status = fail(m, VDBGPU_UNKNOWN_SOURCE,
+                      std::string("Tried to accumulate update for ") + id + ". Source not available");
       else if (!m->config_set)
         status = fail(m, VDBGPU_NOT_CONFIGURED, "Map not properly configured. Did you call setConfig method?");
     }
@@ -3181,7 +3187,8 @@ int mark_points(vdbgpu_map* m, const float* xyz, int64_t n, int64_t stride, uint
   CK(dalloc(m, &pts, (bytes + 3) / 4));
   CK(hipMemcpyAsync(pts, xyz, bytes, hipMemcpyHostToDevice, m->stream));
   // at most n leaves; large edits start smaller and grow on overflow
-  const uint32_t cap0 = (uint32_t)std::max<uint64_t>(kMinUpdateCap, next_pow2(std::min<uint64_t>(2 * (uint64_t)n, 1u << 22)));
+  const uint32_t cap0 =
+      (uint32_t)std::max<uint64_t>(kMinUpdateCap, next_pow2(std::min<uint64_t>(2 * (uint64_t)n, 1u << 22)));
   const int r = mark_set(m, m->edit, cap0, [&]() -> int {
     CK(launch_mark_points(m->stream, pts, stride, (uint32_t)n, m->inv, upd_view(m->edit), &m->d_st[2]));
     return VDBGPU_OK;

@@ -25,3 +25,22 @@ def test_one_cast(scene, n, res, R):
     if n < 8192:
         assert o.insert("test", p, pose[:3]) == 0
         same_map(g, o)
+
+
+def test_sets_that_hold_a_scan_stay():
+    """The first scan's set is guessed larger than the ring's others. A scan that any of them holds makes none grow,
+    also when it lies in the larger one; a scan that none holds does."""
+    g, o = pair(0.1, 15.0, **W.PROBS)
+    assert g.set_tuning(defer=1) == V.OK
+    d = np.random.default_rng(3).normal(size=(20000, 3))
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    at = []
+    for r in (10.0, 10.5, 14.5):  # a ball of about 9,200 leaves, 10,500, 26,000; sets are sized for a quarter more
+        p = (d * r).astype(np.float32)
+        for k in range(8):  # four sets in the ring
+            assert g.insert("test", p, [0, 0, 0], check=True) == V.OK
+            assert o.insert("test", p, [0, 0, 0]) == 0
+        g.synchronize()
+        at.append(g.stats()["scratch_bytes"])
+    assert at[1] == at[0] and at[2] > at[1]
+    same_map(g, o)

@@ -427,7 +427,7 @@ __global__ __launch_bounds__(256) void k_seg_fill(const int4* __restrict__ rayin
 // 64-bit word in registers and OR-ing it when the walk left it (in three
 // layouts, each segment in the one whose words it left least) saved LDS
 // operations but cost the loop some fifteen more instructions (a 262,144-ray
-// outdoor scan alone: 496 us, now 390).
+// outdoor scan alone: 496 us, now 400).
 // The word index is clamped to the bitmap. The path is monotone along every
 // axis, so it stayed inside the brick exactly when the end lies where m - 1
 // steps of the right signs lead (a field that left [0, 31] has carried into

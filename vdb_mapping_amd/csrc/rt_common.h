@@ -56,8 +56,8 @@ struct RtDda {
   // The state is the one that many step() calls leave: an axis's times are its
   // own running sum whatever the other axes do, and the events before the
   // exit are those with an earlier time, or the same one and a larger axis.
-  // Some ten sums and compares per axis stand for up to 3 kBig / kDim steps of
-  // forty instructions each.
+  // Some ten sums and compares per axis stand for up to 3 kBig / kDim whole
+  // steps.
   template <int kBig>
   __device__ __forceinline__ bool skip(const RtRay& r, int& n) {
     double T[3];
